@@ -356,3 +356,108 @@ def run(s):
     return pk.attend(s["q"], pool.k, pool.v, kind, pool.tables, s["rows"], s["starts"], s["firsts"], columns, page,
                      counts=s["counts"], offsets=s["starts"], tokens=s["q"].shape[0], partitions=s["parts"],
                      parents=s.get("parents"), out=s["out"], workspace=s["workspace"], **pool.scales)
+
+
+# -- the same in 64 bits -----------------------------------------------------------------------------------------------------
+def _exact_rows(case, q, pool, firsts, scale, parents=None, fresh=None):
+    """(out, log-sum-exps) of every row's window over its pages: q [rows][new][heads][dim], float64 on the GPU."""
+    n_rows, new, hq, d = q.shape
+    page, hkv = case["page"], case["hkv"]
+    g = hq // hkv
+    out, lse = torch.empty(n_rows, new, hq, d, dtype=torch.float64, device="cuda"), torch.empty(n_rows, new, hq, dtype=torch.float64, device="cuda")
+
+    def real(x, scales, which, at, head):
+        y = x.reshape(-1, hkv, d)[at, head].double()
+        if scales is not None:
+            y = y * scales.reshape(-1, hkv)[at, head].double()[:, None]
+        if torch.is_tensor(pool.multipliers):
+            y = y * pool.multipliers[which, head].double()
+        return y
+
+    for r in range(n_rows):
+        first = firsts[r]
+        n = torch.arange(first + new, device="cuda")
+        at = pool.tables[r].long()[n // page] * page + n % page
+        seen = torch.ones(new, first + new, dtype=torch.bool, device="cuda").tril(first)
+        if parents is not None:      # of the window's own positions only a node's ancestors and itself
+            for c in range(new):
+                up, mine = c, []
+                while up >= 0:
+                    mine.append(up)
+                    up = parents[r][up]
+                seen[c, first:] = False
+                seen[c, [first + m for m in mine]] = True
+        for h in range(hkv):
+            k, v = real(pool.k, pool.ks, 0, at, h), real(pool.v, pool.vs, 1, at, h)
+            if fresh is not None:      # the chunk's own rows, unquantised
+                k[first:], v[first:] = fresh[0][r, :, h].double(), fresh[1][r, :, h].double()
+            x = q[r, :, h * g:(h + 1) * g].double().reshape(new * g, d) @ k.T.contiguous()
+            x = (x * scale).reshape(new, g, -1).masked_fill(~seen[:, None, :], -math.inf)
+            lse[r, :, h * g:(h + 1) * g] = x.logsumexp(-1)
+            out[r, :, h * g:(h + 1) * g] = (x.softmax(-1).reshape(new * g, -1) @ v).reshape(new, g, d)
+    return out, lse
+
+
+def _coded(x, kind, pool, which):
+    """A step's new rows as its pages hold them: (stored, row scales or None)."""
+    x = x.float()
+    if kind in ("bf16", "fp16"):
+        return x.to(STORE[kind]), None
+    if kind == "fp8":
+        return (x / pool.multipliers[which][None, :, None]).clamp(-448, 448).to(STORE[kind]), None
+    top = 448.0 if kind == "fp8:row" else 127.0
+    s = (x.abs().amax(dim=-1) / top).clamp(min=1e-30)
+    y = (x / s[..., None]).clamp(-top, top)
+    return (y.round() if kind == "int8" else y).to(STORE[kind]), s
+
+
+def _rotated(x, table, positions):
+    """Keys turned by their positions' angles, pairs (j, j + dim / 2), rounded to their own type."""
+    half = x.shape[-1] // 2
+    row = table[positions][:, None, :]
+    cos, sin, a, b = row[..., :half], row[..., half:], x[..., :half].float(), x[..., half:].float()
+    return torch.cat([a * cos - b * sin, b * cos + a * sin], -1).to(x.dtype)
+
+
+def exact(case, seed):
+    """What run() returns, in 64 bits by plain torch; pages, slots and picks have no such value."""
+    path, kind, rows = case["path"], case["kind"], case["rows"]
+    if path in ("append", "index"):
+        return None
+    s = prepare(case, seed)
+    firsts = s["firsts"].tolist()
+    if path == "latent":
+        new, page, h = case["columns"], case["page"], case["hq"]
+        out = torch.empty(rows, new, h, RANK, dtype=torch.float64, device="cuda")
+        q = s["q"].reshape(rows, new, h, RANK + ROPE)
+        for r, first in enumerate(firsts):
+            n = torch.arange(first + new, device="cuda")
+            at = s["tables"][r].long()[n // page] * page + n % page
+            kv = s["cache"].reshape(-1, RANK + ROPE)[at].double()
+            if kind == "fp8":
+                scales = s["scales"].reshape(-1, 2)[at].double()
+                kv[:, :RANK] *= scales[:, :1]
+                kv[:, RANK:] *= scales[:, 1:]
+            for c in range(new):
+                x = q[r, c].double() @ kv[:first + c + 1].T.contiguous() * (RANK + ROPE) ** -0.5
+                out[r, c] = x.softmax(-1) @ kv[:first + c + 1, :RANK].contiguous()
+        return out.reshape(rows * new, h, RANK)
+    d, hq, page = case["d"], case["hq"], case["page"]
+    if path == "step":
+        outs = []
+        for i, pool in enumerate(s["pools"]):
+            keys = s["keys"][i] if s["rope"] is None else _rotated(s["keys"][i], s["rope"], s["firsts"])
+            at = pool.tables.long()[torch.arange(rows, device="cuda"), s["firsts"] // page] * page + s["firsts"] % page
+            for x, scales, new, which in ((pool.k, pool.ks, keys, 0), (pool.v, pool.vs, s["values"][i], 1)):
+                codes, own = _coded(new, kind, pool, which)
+                x.reshape(-1, case["hkv"], d)[at] = codes
+                if own is not None:
+                    scales.reshape(-1, case["hkv"])[at] = own
+            outs.append(_exact_rows(case, s["q"][i][:, None], pool, firsts, d ** -0.5)[0][:, 0])
+        return {"out": outs, "slots": None, "pages": [None] * (2 * len(outs))}
+    tokens, new = s["q"].shape[0], s["q"].shape[0] // rows
+    parents = s["parents"].reshape(rows, new).tolist() if "parents" in s else None
+    fresh = [x.reshape(rows, new, case["hkv"], d) for x in s["fresh"]] if "fresh" in s else None
+    out, lse = _exact_rows(case, s["q"].reshape(rows, new, hq, d), s["pool"], firsts, d ** -0.5, parents, fresh)
+    out, lse = out.reshape(tokens, hq, d), lse.reshape(tokens, hq)
+    return (out, lse) if path == "long" else out
