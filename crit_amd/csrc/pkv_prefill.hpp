@@ -22,7 +22,8 @@ struct PrefillArgs {
     float* lse;
     const float* sinks;
     int64_t q_st, q_sh, o_st, o_sh, tab_stride;
-    int tab_width, chunks, max_count, hq, hkv, g, page, page_l, sliding, out_dtype, tiles;
+    int tab_width, chunks, max_count, hq, hkv, g, page, page_l, sliding, out_dtype;
+    int shares, share_tiles;      // XCDs a (chunk, KV head) pair is dealt to, tiles of it each takes at most
     uint32_t page_magic;     // n / page == (mulhi(page_magic, n) + n) >> page_l for 0 <= n < 2^31
     float sscale, k_mult, v_mult;
     // A chunk whose own positions from `first` on are read from fresh 16-bit rows takes two launches that hand a row's
