@@ -350,9 +350,13 @@ static int launch_attend_checked(const crit_pkv_attend_params* p, hipStream_t st
     // columns 383 -> 288 us, 5 columns 519 -> 424, 8 columns 676 -> 480; one row of 32,768: 55 -> 45, 72 -> 56 and 91 ->
     // 62. Not taken where it measured slower: four tiles of 8-bit pages (8 columns 376 -> 334 us but 5 columns 279 ->
     // 302, one row 55 -> 92: the converted rows' steps are too long a chain for one wavefront a SIMD).
+    // Three tiles where as many workgroups hold the window as with four (3, 5, 6 and 9 tiles): a step is bound by its
+    // matrix and softmax work, which the tiles that no row fills cost as well, and three leave nothing in scratch. The
+    // same 64 rows, three tiles against four: 5 columns 427 -> 365 us (a draft tree 635 -> 518), 6 columns 443 -> 380;
+    // 20 rows of 56 / 8 heads, 3 columns 142 -> 116. Three in a second workgroup's registers spill 336 bytes a lane.
     a.query_tiles = 1;
     if (a.fast128 && !p->blocks && !p->fused && wide128 && p->kind == 0 && a.tiles >= 2) {
-        a.query_tiles = a.tiles >= 3 ? 4 : 2;
+        a.query_tiles = a.tiles == 2 ? 2 : ((a.tiles + 2) / 3 == (a.tiles + 3) / 4 ? 3 : 4);
         a.tiles = (a.tiles + a.query_tiles - 1) / a.query_tiles;
     }
     // 8-bit pages: two tiles a workgroup, two workgroups a compute unit still (FP8 in 242-252 registers; the row-scaled

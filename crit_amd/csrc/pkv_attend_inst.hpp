@@ -119,7 +119,7 @@ static int launch_mfma(const AttendArgs& a, bool fused, dim3 grid, hipStream_t s
     if (units <= resident) u.ticket = nullptr;
     const bool masked = a.parents != nullptr || a.parents64 != nullptr || a.sliding > 0;
     const int which = (a.narrow ? 64 : 0) + (a.dk == 256 ? 8 : (a.heads_per_wave == 2 ? 4 : 0)) + (fused ? 2 : 0) + (masked ? 1 : 0) +
-                      (a.query_tiles == 4 ? 12 : (a.query_tiles == 2 ? 24 : 0));
+                      (a.query_tiles == 4 ? 12 : (a.query_tiles == 3 ? 36 : (a.query_tiles == 2 ? 24 : 0)));
     switch (which) {
 #define PKV_MFMA(W, HWV, FU, MA, DH) \
     case W: hipLaunchKernelGGL((attend_mfma_kernel<KIND, F16, HWV, FU, MA, DH>), pgrid, dim3(256), 0, stream, u); break;
@@ -133,15 +133,16 @@ static int launch_mfma(const AttendArgs& a, bool fused, dim3 grid, hipStream_t s
         PKV_MFMA_NARROW(0, 1, false, false) PKV_MFMA_NARROW(1, 1, false, true) PKV_MFMA_NARROW(2, 1, true, false) PKV_MFMA_NARROW(3, 1, true, true)
         PKV_MFMA_NARROW(4, 2, false, false) PKV_MFMA_NARROW(5, 2, false, true) PKV_MFMA_NARROW(6, 2, true, false) PKV_MFMA_NARROW(7, 2, true, true)
 #undef PKV_MFMA_NARROW
-        // four query tiles a workgroup: split launches of 128-wide heads over 16-bit pages
-#define PKV_MFMA_QT(W, HWV, MA) \
+        // four query tiles a workgroup, or three: split launches of 128-wide heads over 16-bit pages
+#define PKV_MFMA_QT(W, HWV, MA, QTV) \
     case W:                                                                                                                  \
         if constexpr (KIND == 0) {                                                                                           \
-            hipLaunchKernelGGL((attend_mfma_kernel<KIND, F16, HWV, false, MA, 1, 4>), pgrid, dim3(256), 0, stream, u);       \
+            hipLaunchKernelGGL((attend_mfma_kernel<KIND, F16, HWV, false, MA, 1, QTV>), pgrid, dim3(256), 0, stream, u);     \
             break;                                                                                                           \
         }                                                                                                                    \
         return CRIT_PKV_E_GEOMETRY;
-        PKV_MFMA_QT(12, 1, false) PKV_MFMA_QT(13, 1, true) PKV_MFMA_QT(16, 2, false) PKV_MFMA_QT(17, 2, true)
+        PKV_MFMA_QT(12, 1, false, 4) PKV_MFMA_QT(13, 1, true, 4) PKV_MFMA_QT(16, 2, false, 4) PKV_MFMA_QT(17, 2, true, 4)
+        PKV_MFMA_QT(36, 1, false, 3) PKV_MFMA_QT(37, 1, true, 3) PKV_MFMA_QT(40, 2, false, 3) PKV_MFMA_QT(41, 2, true, 3)
 #undef PKV_MFMA_QT
         // two query tiles a workgroup, two workgroups a compute unit still
 #define PKV_MFMA_QT2(W, HWV, MA) \

@@ -1,0 +1,30 @@
+"""Verify windows read three query tiles a workgroup: every column against float64 attention over the stored values and,
+bit for bit, against its fused launch."""
+import pytest
+import torch
+
+from tests.support import Cache, rand_q
+
+pytestmark = pytest.mark.gpu
+dev = "cuda"
+# 16-bit probabilities and results: 2^-8 of the largest weight and of the result, four times that
+ATOL, RTOL = 8e-3, 2e-2
+
+
+@pytest.mark.parametrize("kind", ["bf16", "fp16"])
+@pytest.mark.parametrize("hkv,g,columns", [(2, 4, 5), (2, 4, 6), (2, 7, 3), (2, 7, 6), (2, 8, 9), (3, 4, 9), (3, 4, 12), (3, 7, 11)])
+def test_windows_of_three_tiles_a_workgroup(kind, hkv, g, columns):
+    # 3, 5, 6 and 9 tiles (of 8 rows with two KV heads a wavefront, of 16 with one), the last ones full and not
+    cache = Cache(kind, hkv, 128, 128, 16, [1100, 25, 530])
+    firsts, counts = [1100 - columns, 25 - columns, 511], [columns, max(1, columns - 2), min(columns, 4)]
+    starts = [0, columns, 2 * columns]
+    q = rand_q(3 * columns, hkv * g, 128, 31)
+    i32 = torch.tensor(counts, dtype=torch.int32, device=dev)
+    out = cache.attend(q, [0, 1, 2], starts, firsts, columns, counts=i32)
+    fused = cache.attend(q, [0, 1, 2], starts, firsts, columns, counts=i32, fused=True)
+    for s, (start, first, n) in enumerate(zip(starts, firsts, counts)):
+        assert torch.equal(out[start:start + n], fused[start:start + n]), s
+        want, _ = cache.want(q[start:start + n], s, first, n)
+        torch.testing.assert_close(out[start:start + n].double().cpu(), want, atol=ATOL, rtol=RTOL, msg=str(s))
+        one = cache.attend(q[start + n - 1:start + n], [s], [0], [first + n - 1], 1)
+        assert torch.equal(one[0], out[start + n - 1]), s
