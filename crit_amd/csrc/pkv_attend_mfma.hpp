@@ -566,21 +566,33 @@ __global__ __launch_bounds__(256, (DH == 2 || QT > 2) ? 1 : kMfmaWaves) void att
                     for (int i = 0; i < 4; ++i) ks4[i] = KIND >= 2 ? tl.ks[i] : 1.0f, vs4[i] = KIND >= 2 ? tl.vs[i] : 1.0f;
                     refill_k();      // (the keys' registers are free: the loads of NT steps ahead go out)
                     u32x2 pb[QT];
+                    // A draft tree's step wholly before the window's first position: every column of the row sees all of
+                    // it, so nothing is asked a position (a shift by 64 bits and three comparisons each, on the vector
+                    // pipe that 8-bit pages keep busy: one row of 50,000, 56 / 8 heads, 8 columns, INT8 179 -> 138 us; 64
+                    // rows ~U[1024, 8192], 32 / 8 heads, 5 columns INT8 370 -> 303 us, BF16 518 -> 397; the same bits).
+                    const bool before = MASKED && win <= 0 && base + SPW <= min(cur.first, cur.n_keys);
 #pragma unroll
                     for (int q = 0; q < QT; ++q) {
                         // the lane's scores: its column at positions base + r_pos + i of head r_head; another head's column sees nothing
                         const int room = lim[q] - (base + r_pos);      // visible while i <= room
                         float x[4];
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            x[i] = (s0[q][i] + s1[q][i]) * (KIND >= 2 ? sscale * ks4[i] : sscale);
-                            bool vis = mine && i <= room;
-                            if constexpr (MASKED) {
-                                const int n = base + r_pos + i;
-                                if (tree) vis = vis && (n < cur.first || ((anc[q] >> ((n - cur.first) & 63)) & 1ull) != 0);
-                                if (win > 0) vis = vis && n > cur.first + col[q] - win;
+                        for (int i = 0; i < 4; ++i) x[i] = (s0[q][i] + s1[q][i]) * (KIND >= 2 ? sscale * ks4[i] : sscale);
+                        if (MASKED && before) {
+                            const bool vis = mine && lim[q] >= 0;
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) x[i] = vis ? x[i] : -INFINITY;
+                        } else {
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                bool vis = mine && i <= room;
+                                if constexpr (MASKED) {
+                                    const int n = base + r_pos + i;
+                                    if (tree) vis = vis && (n < cur.first || ((anc[q] >> ((n - cur.first) & 63)) & 1ull) != 0);
+                                    if (win > 0) vis = vis && n > cur.first + col[q] - win;
+                                }
+                                x[i] = vis ? x[i] : -INFINITY;
                             }
-                            x[i] = vis ? x[i] : -INFINITY;
                         }
                         const float top = max_across_quarters(__builtin_fmaxf(__builtin_fmaxf(x[0], x[1]), __builtin_fmaxf(x[2], x[3])));
                         const float m_new = __builtin_fmaxf(m[q], top);

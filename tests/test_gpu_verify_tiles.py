@@ -1,5 +1,5 @@
-"""Verify windows read three query tiles a workgroup: every column against float64 attention over the stored values and,
-bit for bit, against its fused launch."""
+"""Verify windows read three query tiles a workgroup, and draft trees whose steps lie before, across and behind the window's
+first position: every column against float64 attention over the stored values and, bit for bit, against its fused launch."""
 import pytest
 import torch
 
@@ -28,3 +28,18 @@ def test_windows_of_three_tiles_a_workgroup(kind, hkv, g, columns):
         torch.testing.assert_close(out[start:start + n].double().cpu(), want, atol=ATOL, rtol=RTOL, msg=str(s))
         one = cache.attend(q[start + n - 1:start + n], [s], [0], [first + n - 1], 1)
         assert torch.equal(one[0], out[start + n - 1]), s
+
+
+@pytest.mark.parametrize("kind", ["bf16", "fp8", "fp8:row", "int8"])
+@pytest.mark.parametrize("hkv,g,d,columns", [(2, 4, 128, 5), (2, 7, 128, 8), (3, 4, 128, 5), (2, 6, 256, 5), (4, 4, 64, 6)])
+@pytest.mark.parametrize("first", [0, 1, 7, 8, 15, 16, 17, 520, 527])
+def test_trees_at_every_place_of_the_windows_first_position_in_a_step(kind, hkv, g, d, columns, first):
+    cache = Cache(kind, hkv, d, d, 16, [first + columns])
+    parents = torch.tensor([-1, 0, 0, 1, 1, 2, 5, 3][:columns], dtype=torch.int32, device=dev)
+    q = rand_q(columns, hkv * g, d, 32)
+    out = cache.attend(q, [0], [0], [first], columns, parents=parents)
+    assert torch.equal(out, cache.attend(q, [0], [0], [first], columns, parents=parents, fused=True))
+    chain = cache.attend(q, [0], [0], [first], columns, parents=torch.arange(-1, columns - 1, dtype=torch.int32, device=dev))
+    assert torch.equal(chain, cache.attend(q, [0], [0], [first], columns))
+    want, _ = cache.want(q.to(torch.bfloat16), 0, first, columns, parents=parents.tolist())
+    torch.testing.assert_close(out.double().cpu(), want, atol=ATOL, rtol=RTOL)
