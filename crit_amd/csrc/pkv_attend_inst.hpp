@@ -104,6 +104,61 @@ static int launch_one(const AttendArgs& a, int lpr, bool page16, dim3 grid, hipS
     return hip_code(hipGetLastError());
 }
 
+// The bandwidth path's kernel for one kind of mask, by the KV heads a wavefront serves, the heads' width and the query
+// tiles a workgroup holds.
+template <int KIND, bool F16, int MASK>
+static int launch_mfma_masked(const AttendArgs& u, bool fused, dim3 grid, hipStream_t stream) {
+#define PKV_MFMA(...) hipLaunchKernelGGL((attend_mfma_kernel<KIND, F16, __VA_ARGS__>), grid, dim3(256), 0, stream, u)
+    const bool pair = u.heads_per_wave == 2;
+    if (fused) {
+        if (u.query_tiles != 1) return CRIT_PKV_E_GEOMETRY;
+        if (u.narrow) {      // 64-wide heads in pairs
+            if (pair) PKV_MFMA(2, true, MASK, 1, 1, true);
+            else PKV_MFMA(1, true, MASK, 1, 1, true);
+        } else if (u.dk == 256) {
+            PKV_MFMA(1, true, MASK, 2);
+        } else if (pair) {
+            PKV_MFMA(2, true, MASK);
+        } else {
+            PKV_MFMA(1, true, MASK);
+        }
+        return hip_code(hipGetLastError());
+    }
+    if (u.narrow) {
+        if (u.query_tiles != 1) return CRIT_PKV_E_GEOMETRY;
+        if (pair) PKV_MFMA(2, false, MASK, 1, 1, true);
+        else PKV_MFMA(1, false, MASK, 1, 1, true);
+        return hip_code(hipGetLastError());
+    }
+    switch (u.query_tiles) {
+        case 1:
+            if (u.dk == 256) PKV_MFMA(1, false, MASK, 2);
+            else if (pair) PKV_MFMA(2, false, MASK);
+            else PKV_MFMA(1, false, MASK);
+            return hip_code(hipGetLastError());
+        case 2:      // two workgroups a compute unit still (256-wide heads: one)
+            if (u.dk == 256) PKV_MFMA(1, false, MASK, 2, 2);
+            else if (pair) PKV_MFMA(2, false, MASK, 1, 2);
+            else PKV_MFMA(1, false, MASK, 1, 2);
+            return hip_code(hipGetLastError());
+        case 3: case 4:      // split launches of 128-wide heads over 16-bit pages
+            if constexpr (KIND == 0) {
+                if (u.dk == 256) return CRIT_PKV_E_GEOMETRY;
+                if (u.query_tiles == 3) {
+                    if (pair) PKV_MFMA(2, false, MASK, 1, 3);
+                    else PKV_MFMA(1, false, MASK, 1, 3);
+                } else {
+                    if (pair) PKV_MFMA(2, false, MASK, 1, 4);
+                    else PKV_MFMA(1, false, MASK, 1, 4);
+                }
+                return hip_code(hipGetLastError());
+            }
+            break;
+    }
+    return CRIT_PKV_E_GEOMETRY;
+#undef PKV_MFMA
+}
+
 // 128- and 256-wide heads over pages of a multiple of 16 positions: the bandwidth path, resident workgroups pulling units.
 template <int KIND, bool F16>
 static int launch_mfma(const AttendArgs& a, bool fused, dim3 grid, hipStream_t stream) {
@@ -117,48 +172,12 @@ static int launch_mfma(const AttendArgs& a, bool fused, dim3 grid, hipStream_t s
     // A unit a workgroup at most: nothing to draw, and no counter touched (a draw's round trip and the count of the
     // finished workgroups are a few microseconds at the end of a launch that is one unit long).
     if (units <= resident) u.ticket = nullptr;
-    const bool masked = a.parents != nullptr || a.parents64 != nullptr || a.sliding > 0;
-    const int which = (a.narrow ? 64 : 0) + (a.dk == 256 ? 8 : (a.heads_per_wave == 2 ? 4 : 0)) + (fused ? 2 : 0) + (masked ? 1 : 0) +
-                      (a.query_tiles == 4 ? 12 : (a.query_tiles == 3 ? 36 : (a.query_tiles == 2 ? 24 : 0)));
-    switch (which) {
-#define PKV_MFMA(W, HWV, FU, MA, DH) \
-    case W: hipLaunchKernelGGL((attend_mfma_kernel<KIND, F16, HWV, FU, MA, DH>), pgrid, dim3(256), 0, stream, u); break;
-        PKV_MFMA(0, 1, false, false, 1) PKV_MFMA(1, 1, false, true, 1) PKV_MFMA(2, 1, true, false, 1) PKV_MFMA(3, 1, true, true, 1)
-        PKV_MFMA(4, 2, false, false, 1) PKV_MFMA(5, 2, false, true, 1) PKV_MFMA(6, 2, true, false, 1) PKV_MFMA(7, 2, true, true, 1)
-        PKV_MFMA(8, 1, false, false, 2) PKV_MFMA(9, 1, false, true, 2) PKV_MFMA(10, 1, true, false, 2) PKV_MFMA(11, 1, true, true, 2)
-#undef PKV_MFMA
-        // 64-wide heads in pairs
-#define PKV_MFMA_NARROW(W, HWV, FU, MA) \
-    case 64 + W: hipLaunchKernelGGL((attend_mfma_kernel<KIND, F16, HWV, FU, MA, 1, 1, true>), pgrid, dim3(256), 0, stream, u); break;
-        PKV_MFMA_NARROW(0, 1, false, false) PKV_MFMA_NARROW(1, 1, false, true) PKV_MFMA_NARROW(2, 1, true, false) PKV_MFMA_NARROW(3, 1, true, true)
-        PKV_MFMA_NARROW(4, 2, false, false) PKV_MFMA_NARROW(5, 2, false, true) PKV_MFMA_NARROW(6, 2, true, false) PKV_MFMA_NARROW(7, 2, true, true)
-#undef PKV_MFMA_NARROW
-        // four query tiles a workgroup, or three: split launches of 128-wide heads over 16-bit pages
-#define PKV_MFMA_QT(W, HWV, MA, QTV) \
-    case W:                                                                                                                  \
-        if constexpr (KIND == 0) {                                                                                           \
-            hipLaunchKernelGGL((attend_mfma_kernel<KIND, F16, HWV, false, MA, 1, QTV>), pgrid, dim3(256), 0, stream, u);     \
-            break;                                                                                                           \
-        }                                                                                                                    \
-        return CRIT_PKV_E_GEOMETRY;
-        PKV_MFMA_QT(12, 1, false, 4) PKV_MFMA_QT(13, 1, true, 4) PKV_MFMA_QT(16, 2, false, 4) PKV_MFMA_QT(17, 2, true, 4)
-        PKV_MFMA_QT(36, 1, false, 3) PKV_MFMA_QT(37, 1, true, 3) PKV_MFMA_QT(40, 2, false, 3) PKV_MFMA_QT(41, 2, true, 3)
-#undef PKV_MFMA_QT
-        // two query tiles a workgroup, two workgroups a compute unit still
-#define PKV_MFMA_QT2(W, HWV, MA) \
-    case W:                                                                                                                  \
-        if constexpr (KIND <= 3) {                                                                                           \
-            hipLaunchKernelGGL((attend_mfma_kernel<KIND, F16, HWV, false, MA, 1, 2>), pgrid, dim3(256), 0, stream, u);       \
-            break;                                                                                                           \
-        }                                                                                                                    \
-        return CRIT_PKV_E_GEOMETRY;
-        PKV_MFMA_QT2(24, 1, false) PKV_MFMA_QT2(25, 1, true) PKV_MFMA_QT2(28, 2, false) PKV_MFMA_QT2(29, 2, true)
-#undef PKV_MFMA_QT2
-        case 32: hipLaunchKernelGGL((attend_mfma_kernel<KIND, F16, 1, false, false, 2, 2>), pgrid, dim3(256), 0, stream, u); break;
-        case 33: hipLaunchKernelGGL((attend_mfma_kernel<KIND, F16, 1, false, true, 2, 2>), pgrid, dim3(256), 0, stream, u); break;
-        default: return CRIT_PKV_E_GEOMETRY;
+    const int mask = a.sliding > 0 ? kMaskSliding : (a.parents != nullptr || a.parents64 != nullptr ? kMaskTree : kMaskNone);
+    switch (mask) {
+        case kMaskNone: return launch_mfma_masked<KIND, F16, kMaskNone>(u, fused, pgrid, stream);
+        case kMaskTree: return launch_mfma_masked<KIND, F16, kMaskTree>(u, fused, pgrid, stream);
+        default: return launch_mfma_masked<KIND, F16, kMaskSliding>(u, fused, pgrid, stream);
     }
-    return hip_code(hipGetLastError());
 }
 
 template <int KIND, bool F16>

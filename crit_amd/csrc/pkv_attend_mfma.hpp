@@ -102,6 +102,7 @@ struct Tile {
     float ks[KIND >= 2 ? 4 : 1], vs[KIND >= 2 ? 4 : 1];      // row-scaled kinds: the scales of positions 4 u .. 4 u + 3
 };
 
+constexpr int kMaskNone = 0, kMaskTree = 1, kMaskSliding = 2;
 constexpr int kTileRows = 16;      // query rows (columns of S^T) a tile holds
 constexpr int kLdsRows = 512;      // batch rows whose descriptors a workgroup keeps in LDS (the others are read from memory)
 
@@ -122,7 +123,12 @@ constexpr int kMfmaTiles = 2;
 // happen while the next unit's rows are already on their way. A drawn unit without work (the list is a grid over rows
 // of different lengths) is passed over by the drawing thread at once. The last workgroup to finish zeroes the counters
 // for the next launch that uses them. Without counters the units are dealt in turn.
-// MASKED: draft trees and sliding windows. DH: 128-wide halves of a head (1: heads of 128; 2: heads of 256, whose rows
+// MASK: what hides positions of a column beside its own end: nothing, a draft tree, or a sliding window (with or
+// without a tree). Trees and windows are kernels of their own: a tree's short mask (in the step) is of no use to a
+// window, whose kernels it cost registers (20 bytes of scratch a lane in the fused 16-bit ones, 40 more in pairs of
+// tiles) and time: 64 rows ~U[1024, 8192], 32 / 8 heads, a window of 1,024, 3 columns: BF16 174 us in one kernel, 154
+// apart; INT8 194 and 184; and a tree's kernels keep fewer registers without a window: INT8, 5 columns 305 -> 283 us.
+// DH: 128-wide halves of a head (1: heads of 128; 2: heads of 256, whose rows
 // are 512 bytes of 16-bit pages by themselves, so a wavefront serves one KV head: HW 1): twice the key pieces, query
 // pieces, score products and output tiles, the same layouts otherwise; twice the registers too, so one workgroup a
 // compute unit, which keeps as many bytes in flight as two of the narrower ones (a step's rows are twice as long).
@@ -142,7 +148,7 @@ constexpr int kMfmaTiles = 2;
 // which its own head's 64 are kept. Twice the matrix work a byte, on a pipe this kernel leaves nine tenths idle, for
 // the 128-wide kernel's loads: 512 contiguous bytes a position and wavefront. What follows a KV head (row scales, an
 // FP8 pool's multipliers) is looked up by the column's own head.
-template <int KIND, bool F16, int HW, bool FUSED, bool MASKED, int DH = 1, int QT = 1, bool NARROW = false>
+template <int KIND, bool F16, int HW, bool FUSED, int MASK, int DH = 1, int QT = 1, bool NARROW = false>
 __global__ __launch_bounds__(256, (DH == 2 || QT > 2) ? 1 : kMfmaWaves) void attend_mfma_kernel(AttendArgs a) {
     static_assert(!NARROW || (DH == 1 && QT == 1), "64-wide heads: one 128-wide pair a tile row, one tile a workgroup");
     constexpr int NT = DH == 2 && QT == 2 ? 1 : kMfmaTiles;
@@ -174,8 +180,10 @@ __global__ __launch_bounds__(256, (DH == 2 || QT > 2) ? 1 : kMfmaWaves) void att
     const bool dense = a.n_rows <= kLdsRows;
     const unsigned per_row = (unsigned)(hgroups * a.tiles);
     const int slot_bytes = a.hkv * D * EB;
-    const bool tree = MASKED && (a.parents != nullptr || a.parents64 != nullptr);
-    const int win = MASKED ? a.sliding : 0;
+    const bool tree = MASK == kMaskTree || (MASK == kMaskSliding && (a.parents != nullptr || a.parents64 != nullptr));
+    // (A tree's launch has no window. The kernel of four tiles asks for one all the same: left out, the compiler schedules
+    // its steps so that 98 registers a lane go to scratch instead of 39, 64 rows of 8 columns 600 us instead of 520.)
+    const int win = MASK == kMaskSliding || (MASK == kMaskTree && QT > 3) ? a.sliding : 0;
 
     // -- every row's descriptors, once per workgroup
     auto row_from_memory = [&](int r, int (&d)[5]) __attribute__((always_inline)) {
@@ -568,25 +576,24 @@ __global__ __launch_bounds__(256, (DH == 2 || QT > 2) ? 1 : kMfmaWaves) void att
                     u32x2 pb[QT];
                     // A draft tree's step wholly before the window's first position: every column of the row sees all of
                     // it, so nothing is asked a position (a shift by 64 bits and three comparisons each, on the vector
-                    // pipe that 8-bit pages keep busy: one row of 50,000, 56 / 8 heads, 8 columns, INT8 179 -> 138 us; 64
-                    // rows ~U[1024, 8192], 32 / 8 heads, 5 columns INT8 370 -> 303 us, BF16 518 -> 397; the same bits).
-                    const bool before = MASKED && win <= 0 && base + SPW <= min(cur.first, cur.n_keys);
+                    // pipe that 8-bit pages keep busy: one row of 50,000, 56 / 8 heads, 8 columns, INT8 179 -> 124 us; 64
+                    // rows ~U[1024, 8192], 32 / 8 heads, 5 columns INT8 370 -> 283 us, BF16 518 -> 393; the same bits).
+                    const bool before = MASK == kMaskTree && win <= 0 && base + SPW <= min(cur.first, cur.n_keys);
 #pragma unroll
                     for (int q = 0; q < QT; ++q) {
                         // the lane's scores: its column at positions base + r_pos + i of head r_head; another head's column sees nothing
                         const int room = lim[q] - (base + r_pos);      // visible while i <= room
                         float x[4];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) x[i] = (s0[q][i] + s1[q][i]) * (KIND >= 2 ? sscale * ks4[i] : sscale);
-                        if (MASKED && before) {
+                        if (MASK == kMaskTree && before) {
                             const bool vis = mine && lim[q] >= 0;
 #pragma unroll
-                            for (int i = 0; i < 4; ++i) x[i] = vis ? x[i] : -INFINITY;
+                            for (int i = 0; i < 4; ++i) x[i] = vis ? (s0[q][i] + s1[q][i]) * (KIND >= 2 ? sscale * ks4[i] : sscale) : -INFINITY;
                         } else {
 #pragma unroll
                             for (int i = 0; i < 4; ++i) {
+                                x[i] = (s0[q][i] + s1[q][i]) * (KIND >= 2 ? sscale * ks4[i] : sscale);
                                 bool vis = mine && i <= room;
-                                if constexpr (MASKED) {
+                                if constexpr (MASK != kMaskNone) {
                                     const int n = base + r_pos + i;
                                     if (tree) vis = vis && (n < cur.first || ((anc[q] >> ((n - cur.first) & 63)) & 1ull) != 0);
                                     if (win > 0) vis = vis && n > cur.first + col[q] - win;

@@ -43,3 +43,28 @@ def test_trees_at_every_place_of_the_windows_first_position_in_a_step(kind, hkv,
     assert torch.equal(chain, cache.attend(q, [0], [0], [first], columns))
     want, _ = cache.want(q.to(torch.bfloat16), 0, first, columns, parents=parents.tolist())
     torch.testing.assert_close(out.double().cpu(), want, atol=ATOL, rtol=RTOL)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "fp16", "fp8", "fp8:row", "int8"])
+@pytest.mark.parametrize("sliding", [0, 33, 300])
+@pytest.mark.parametrize("hkv,g,d,columns", [(2, 4, 128, 4), (2, 4, 128, 5), (2, 4, 128, 8), (3, 4, 128, 9), (2, 7, 128, 6), (2, 8, 128, 9), (2, 6, 256, 5), (4, 4, 64, 6)])
+def test_trees_and_sliding_windows_over_several_ragged_rows(kind, sliding, hkv, g, d, columns):
+    # 1 to 9 tiles, rows of every column and of fewer (dead columns in a tile, tiles without a live row), a tree alone, a
+    # sliding window alone and both, split and fused: the same bits, a chain's tree those of the window without one
+    counts = [columns, 1, columns - 1, max(1, columns // 2)]
+    lengths = [1100, 25, 530, 40 + columns]
+    cache = Cache(kind, hkv, d, d, 16, lengths)
+    firsts, starts = [n - c for n, c in zip(lengths, counts)], [columns * i for i in range(4)]
+    q = rand_q(4 * columns, hkv * g, d, 33)
+    i32 = torch.tensor(counts, dtype=torch.int32, device=dev)
+    links = [-1, 0, 0, 1, 1, 2, 5, 3, 6][:columns]
+    parents = torch.tensor(links * 4, dtype=torch.int32, device=dev)
+    chains = torch.arange(-1, columns - 1, dtype=torch.int32, device=dev).repeat(4)
+    run = lambda **kw: cache.attend(q, [0, 1, 2, 3], starts, firsts, columns, counts=i32, sliding=sliding, **kw)
+    out, fused, chain, plain = run(parents=parents), run(parents=parents, fused=True), run(parents=chains), run()
+    for s, (start, first, n) in enumerate(zip(starts, firsts, counts)):
+        assert torch.equal(out[start:start + n], fused[start:start + n]), s
+        assert torch.equal(chain[start:start + n], plain[start:start + n]), s
+        for got, up in ((out, links[:n]), (plain, None)):
+            want, _ = cache.want(q[start:start + n], s, first, n, sliding=sliding, parents=up)
+            torch.testing.assert_close(got[start:start + n].double().cpu(), want, atol=ATOL, rtol=RTOL, msg=f"{s} {up}")
