@@ -49,16 +49,11 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 1 : 8 / WAVES) void prefill_
     __shared__ float ks_lds[2][BN], vs_lds[VBUFS][BN];
 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n32 = lane & 31, h = lane >> 5;
-    // Workgroups go to the 8 XCDs round robin by linear id, and each XCD has its own L2: all tiles of one (chunk, KV
-    // head) read the same keys, so they take ids of one residue mod 8 and share that XCD's L2. Where the (chunk, KV
-    // head) pairs are no multiple of 8, each is dealt to `a.shares` XCDs in turn (every a.shares-th tile to each), the
-    // fewest at which every XCD holds as many: else one chunk of a model with two KV heads runs on two XCDs alone
-    // (24 / 2 heads x 256, 777 tokens after 1,024: 200 us, and 96 us dealt over all eight). Later tiles see more
-    // keys: they start first.
-    const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
-    const int share = xcd + 8 * (q / a.share_tiles);
-    const int group = share / a.shares;
-    const int tile = (a.share_tiles - 1 - q % a.share_tiles) * a.shares + share % a.shares;
+    // All tiles of one (chunk, KV head) pair read the same keys: they share one XCD's L2, or those of the few XCDs that
+    // the launcher deals the pair to (pkv_split.hpp).
+    const DealtTile mine = dealt_tile(blockIdx.x, (uint32_t)a.share_tiles, a.share_l);
+    const int group = mine.pair, tile = mine.tile;
+    if (group >= a.hkv * a.chunks || tile >= a.tiles) return;
     const int kvh = group % a.hkv, z = chunk_by_rank(a, group / a.hkv, lane);
     int count = a.max_count;
     if (a.counts) count = min(a.counts[z], a.max_count);
@@ -701,11 +696,13 @@ static int launch_one(PrefillArgs a, int kind, bool f16, int head_dim, int kv_he
     // three loops per wavefront group the eight-wavefront one spills.)
     const bool wide = head_dim == 128 && a.mode != 2 && tiles * kv_heads * chunks >= compute_units();
     if (!wide) tiles = ((int64_t)max_count * a.g + BM - 1) / BM;
-    a.shares = groups % 8 == 0 ? 1 : (groups % 4 == 0 ? 2 : (groups % 2 == 0 ? 4 : 8));
-    const int64_t share_tiles = (tiles + a.shares - 1) / a.shares;
-    if (share_tiles * groups * a.shares > 0x7fffffff) return CRIT_PKV_E_GEOMETRY;
-    a.share_tiles = (int)share_tiles;
-    const dim3 grid((unsigned)(share_tiles * groups * a.shares));
+    // (256-wide heads and the eight-wavefront shape: one workgroup a compute unit, the others two)
+    const int64_t units = compute_units() / kXcds;
+    a.share_l = xcds_of_pair_log2(groups, tiles, units, wide || head_dim == 256 ? units : 2 * units);
+    const int64_t workgroups = dealt_workgroups(groups, tiles, a.share_l);
+    if (tiles > 0x7fffffff || workgroups > 0x7fffffff) return CRIT_PKV_E_GEOMETRY;
+    a.tiles = (int)tiles, a.share_tiles = (int)tiles_of_share(tiles, a.share_l);
+    const dim3 grid((unsigned)workgroups);
     switch (kind) {
         case 0:
             if (a.mode == 2) return f16 ? launch_d<0, true, true>(a, head_dim, wide, grid, stream) : launch_d<0, false, true>(a, head_dim, wide, grid, stream);
@@ -769,7 +766,7 @@ int launch_prefill(const crit_pkv_prefill_params* p, hipStream_t stream) {
     a.firsts = nullptr, a.state = nullptr, a.mode = 0;
     a.iqk = p->int8_qk != 0;
     a.k_slot_bytes = a.v_slot_bytes = (uint32_t)p->kv_heads * p->head_dim * (p->kind == 0 ? 2 : 1);
-    a.shares = a.share_tiles = 0;
+    a.tiles = a.share_l = a.share_tiles = 0;
     if (!fresh) return launch_one(a, p->kind, f16, p->head_dim, p->kv_heads, p->chunks, p->max_count, stream);
     // The positions below each chunk's first fresh one from the pages, then the rest from the fresh rows (16-bit, in
     // q's type, no scales), through the rows' states.

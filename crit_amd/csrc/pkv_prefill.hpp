@@ -2,6 +2,7 @@
 // order in which chunks are taken.
 #pragma once
 #include "pkv_common.hpp"
+#include "pkv_split.hpp"
 
 namespace pkv {
 
@@ -23,7 +24,7 @@ struct PrefillArgs {
     const float* sinks;
     int64_t q_st, q_sh, o_st, o_sh, tab_stride;
     int tab_width, chunks, max_count, hq, hkv, g, page, page_l, sliding, out_dtype;
-    int shares, share_tiles;      // XCDs a (chunk, KV head) pair is dealt to, tiles of it each takes at most
+    int tiles, share_l, share_tiles;      // query tiles of a (chunk, KV head) pair; log2 of the XCDs it is dealt to; tiles of it each takes at most
     uint32_t page_magic;     // n / page == (mulhi(page_magic, n) + n) >> page_l for 0 <= n < 2^31
     float sscale, k_mult, v_mult;
     // A chunk whose own positions from `first` on are read from fresh 16-bit rows takes two launches that hand a row's

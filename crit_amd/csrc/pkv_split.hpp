@@ -1,0 +1,61 @@
+// How the launches split their work: plain arithmetic over sizes, without device code, so that it can be checked apart
+// from the kernels (tests/test_split.py compiles it for the host).
+#pragma once
+#include <stdint.h>
+
+#ifdef __HIPCC__
+#define PKV_SPLIT_FN __host__ __device__ static inline
+#else
+#define PKV_SPLIT_FN static inline
+#endif
+
+namespace pkv {
+
+constexpr int kXcds = 8;      // dies with an L2 of their own; workgroups go to them round robin by linear id
+
+// -- prompt chunks: the tiles of a (chunk, KV head) pair over the XCDs ----------------------------------------------------
+// A pair's tiles read the same keys, so they belong on one XCD, unless the pairs are too few or too uneven to keep all of
+// them busy: a launch of `pairs` pairs of `tiles` tiles each, a pair dealt to 1 << l XCDs, leaves its busiest XCD
+// ceil(pairs << l / 8) * ceil(tiles >> l) tiles. Taken is the smallest l within a tenth of the least load: splitting
+// costs the L2s another copy of the keys. Pairs that are a multiple of 8 are even as they are. `units` compute units an
+// XCD, `held` workgroups it holds at once.
+//   - A tenth less load is the least that measured as less time; 8 XCDs a pair is for a lone pair (more pairs of which
+//     each XCD has an eighth start the later pairs' longest tiles last: 7 pairs of 64 tiles 86 -> 120 us; 5 pairs of 2,048
+//     tokens after 2,048: 206 us as they are, 190 on four XCDs, 197 on eight).
+//   - Where an XCD has more tiles than it holds, but none of its pairs alone, less than half a tile a compute unit is not
+//     worth the copies (17 pairs of 16 tiles of 256 rows: 39 us, 42 / 48 / 45 on 2 / 4 / 8 XCDs; 33: 57, 61 / 73 / 67; 65:
+//     83, 89 / 106 / 95). Half a tile is: 20 pairs of 32 tiles 144 -> 123 us, 18 pairs of 48 tiles (256 wide) 485 -> 392.
+//   - Few pairs: 2 of 192 tiles (256 wide, 2,048 tokens after 2,048) 762 -> 262 us on four XCDs, 4 of 64 tiles 209 -> 129
+//     on two, 1 of 128 tiles 182 -> 81 on eight. Pairs of one tile stay as they are whatever their count.
+PKV_SPLIT_FN int64_t busiest_xcd(int64_t pairs, int64_t tiles, int l) {
+    return ((pairs << l) + kXcds - 1) / kXcds * ((tiles + (1 << l) - 1) >> l);
+}
+PKV_SPLIT_FN int xcds_of_pair_log2(int64_t pairs, int64_t tiles, int64_t units, int64_t held) {
+    const int most = pairs == 1 ? 3 : 2;
+    const int64_t whole = busiest_xcd(pairs, tiles, 0);
+    int64_t least = whole;
+    for (int l = 1; l <= most; ++l) least = busiest_xcd(pairs, tiles, l) < least ? busiest_xcd(pairs, tiles, l) : least;
+    int l = 0;
+    while (10 * busiest_xcd(pairs, tiles, l) > 11 * least) ++l;
+    if (tiles <= held && whole > held && 2 * (whole - busiest_xcd(pairs, tiles, l)) < units) l = 0;
+    return l;
+}
+// Tiles of a pair one of its XCDs takes at most, and the workgroups of the launch.
+PKV_SPLIT_FN int64_t tiles_of_share(int64_t tiles, int l) { return (tiles + (1 << l) - 1) >> l; }
+PKV_SPLIT_FN int64_t dealt_workgroups(int64_t pairs, int64_t tiles, int l) {
+    return tiles_of_share(tiles, l) * (((pairs << l) + kXcds - 1) / kXcds * kXcds);
+}
+// The pair and the tile of a workgroup; a pair from `pairs` on or a tile from `tiles` on is nobody's. Shares (a pair's
+// part on one XCD) are numbered round by round, one a XCD; a pair's shares lie in one round, and which of its tiles the
+// first of them takes moves on by one every round: otherwise the few tiles of short chunks all meet on the same XCDs.
+// Later tiles see more keys: they start first.
+struct DealtTile {
+    int pair, tile;
+};
+PKV_SPLIT_FN DealtTile dealt_tile(uint32_t workgroup, uint32_t share_tiles, int l) {
+    const uint32_t xcd = workgroup % kXcds, q = workgroup / kXcds, round = q / share_tiles;
+    return DealtTile{(int)((xcd + kXcds * round) >> l),
+                     (int)(((share_tiles - 1 - (q - round * share_tiles)) << l) + ((xcd + round) & ((1u << l) - 1)))};
+}
+
+}   // namespace pkv

@@ -1,0 +1,86 @@
+"""The launches' splits (crit_amd/csrc/pkv_split.hpp, compiled here for the host): every piece of work is somebody's, once,
+and no XCD is left with much more of it than the others."""
+import ctypes
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+UNITS = 32      # compute units an XCD
+
+
+@pytest.fixture(scope="module")
+def split(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("no g++")
+    where = tmp_path_factory.mktemp("split")
+    (where / "split.cpp").write_text("""#include "pkv_split.hpp"
+extern "C" int xcds_log2(int64_t pairs, int64_t tiles, int64_t units, int64_t held) { return pkv::xcds_of_pair_log2(pairs, tiles, units, held); }
+extern "C" int64_t workgroups(int64_t pairs, int64_t tiles, int l) { return pkv::dealt_workgroups(pairs, tiles, l); }
+extern "C" void deal(int64_t pairs, int64_t tiles, int l, int* pair, int* tile) {
+    const int64_t n = pkv::dealt_workgroups(pairs, tiles, l);
+    for (int64_t w = 0; w < n; ++w) {
+        const pkv::DealtTile d = pkv::dealt_tile((uint32_t)w, (uint32_t)pkv::tiles_of_share(tiles, l), l);
+        pair[w] = d.pair, tile[w] = d.tile;
+    }
+}
+""")
+    out = str(where / "split.so")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-O1", "-shared", "-fPIC", "-I", os.path.join(ROOT, "crit_amd", "csrc"),
+                    str(where / "split.cpp"), "-o", out], check=True)
+    lib = ctypes.CDLL(out)
+    lib.xcds_log2.argtypes, lib.workgroups.argtypes = [ctypes.c_int64] * 4, [ctypes.c_int64, ctypes.c_int64, ctypes.c_int]
+    lib.workgroups.restype = ctypes.c_int64
+    lib.deal.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
+    return lib
+
+
+def dealt(split, pairs, tiles, l):
+    """[(xcd, pair, tile)] of the launch's workgroups that have one."""
+    n = split.workgroups(pairs, tiles, l)
+    pair, tile = (ctypes.c_int * n)(), (ctypes.c_int * n)()
+    split.deal(pairs, tiles, l, pair, tile)
+    return [(w % 8, pair[w], tile[w]) for w in range(n) if pair[w] < pairs and tile[w] < tiles]
+
+
+def test_every_tile_of_every_pair_is_dealt_once(split):
+    for pairs in list(range(1, 35)) + [63, 64, 65, 66, 70]:
+        for tiles in (1, 2, 3, 7, 8, 9, 16, 33, 73):
+            for l in range(4):
+                work = dealt(split, pairs, tiles, l)
+                assert sorted((p, t) for _, p, t in work) == [(p, t) for p in range(pairs) for t in range(tiles)], (pairs, tiles, l)
+
+
+@pytest.mark.parametrize("held", [UNITS, 2 * UNITS])
+def test_the_busiest_xcd_has_no_more_than_with_whole_pairs(split, held):
+    for pairs in range(1, 71):
+        for tiles in (1, 2, 3, 7, 8, 9, 10, 16, 32, 48, 64, 73, 128, 192):
+            l = split.xcds_log2(pairs, tiles, UNITS, held)
+            whole = -(-pairs // 8) * tiles
+            load = [0] * 8
+            for xcd, _, _ in dealt(split, pairs, tiles, l):
+                load[xcd] += 1
+            assert max(load) <= whole and (l == 0 or 10 * max(load) <= 11 * whole)
+            assert split.workgroups(pairs, tiles, l) <= -(-pairs // 8) * 8 * tiles      # no wider a launch than with whole pairs
+            assert l == 0 or (pairs % 8 != 0 and tiles > 1)
+    # a few pairs fill the card
+    assert [split.xcds_log2(n, 64, UNITS, held) for n in (1, 2, 4, 8)] == [3, 2, 1, 0]
+
+
+@pytest.mark.parametrize("pairs", [1, 2, 4, 9, 18, 20, 33, 63, 66])
+@pytest.mark.parametrize("live", [1, 2, 3])
+def test_short_chunks_of_a_long_launch_do_not_meet_on_one_xcd(split, pairs, live):
+    # the launch is sized for its longest chunk; the others' few tiles are spread over the XCDs however their pairs are dealt
+    for tiles in (16, 48):
+        for l in range(4):
+            load = [0] * 8
+            for xcd, _, tile in dealt(split, pairs, tiles, l):
+                load[xcd] += tile < live
+            assert max(load) <= -(-pairs // 8) * live, (tiles, l, load)
+
+
+@pytest.mark.parametrize("pairs,tiles,held", [(17, 16, 32), (21, 16, 32), (33, 16, 32), (65, 16, 32), (63, 1, 64), (66, 1, 64), (7, 64, 32), (64, 8, 32)])
+def test_many_even_pairs_and_short_chunks_stay_whole(split, pairs, tiles, held):
+    assert split.xcds_log2(pairs, tiles, UNITS, held) == 0
