@@ -4,6 +4,7 @@
 
 #include "pkv_attend_args.hpp"
 #include "pkv_launch.hpp"
+#include "pkv_split.hpp"
 
 namespace pkv {
 
@@ -343,6 +344,11 @@ static int launch_attend_checked(const crit_pkv_attend_params* p, hipStream_t st
     // bandwidth kernel (matrix tiles of 16 columns).
     const int tile_rows = a.fast128 && !p->blocks ? 16 / a.heads_per_wave : qr;
     a.tiles = (live_rows + tile_rows - 1) / tile_rows;
+    // Positions past the page tables do not exist: partitions that could only hold such pieces are not launched.
+    const int64_t table_keys = (int64_t)p->table_width * p->page;
+    a.max_keys = (int)(table_keys < 0x3fffffff ? table_keys : 0x3fffffff);
+    const int64_t live_parts = ((p->blocks ? (int64_t)a.listed_keys : (int64_t)a.max_keys) + (int64_t)p->piece - 1) / p->piece;
+    const unsigned gy = (unsigned)(live_parts < p->partitions ? live_parts : p->partitions);
     // Windows of several tiles of 128-wide heads over 16-bit pages, split launch: a workgroup holds four tiles (one
     // workgroup a compute unit), or the two of a window of two (two workgroups still, with two dozen registers in
     // scratch outside the steps), and reads the rows once for all of them. A tile's bits are the same however many
@@ -350,13 +356,12 @@ static int launch_attend_checked(const crit_pkv_attend_params* p, hipStream_t st
     // columns 383 -> 288 us, 5 columns 519 -> 424, 8 columns 676 -> 480; one row of 32,768: 55 -> 45, 72 -> 56 and 91 ->
     // 62. Not taken where it measured slower: four tiles of 8-bit pages (8 columns 376 -> 334 us but 5 columns 279 ->
     // 302, one row 55 -> 92: the converted rows' steps are too long a chain for one wavefront a SIMD).
-    // Three tiles where as many workgroups hold the window as with four (3, 5, 6 and 9 tiles): a step is bound by its
-    // matrix and softmax work, which the tiles that no row fills cost as well, and three leave nothing in scratch. The
-    // same 64 rows, three tiles against four: 5 columns 427 -> 365 us (a draft tree 635 -> 518), 6 columns 443 -> 380;
-    // 20 rows of 56 / 8 heads, 3 columns 142 -> 116. Three in a second workgroup's registers spill 336 bytes a lane.
+    // Three tiles, which leave nothing in scratch, in place of four where window_tiles_16bit() says so. (Three in a
+    // second workgroup's registers would spill 336 bytes a lane.)
     a.query_tiles = 1;
     if (a.fast128 && !p->blocks && !p->fused && wide128 && p->kind == 0 && a.tiles >= 2) {
-        a.query_tiles = a.tiles == 2 ? 2 : ((a.tiles + 2) / 3 == (a.tiles + 3) / 4 ? 3 : 4);
+        const bool full = !p->counts || p->window_tokens == (int64_t)p->n_rows * p->columns;
+        a.query_tiles = window_tiles_16bit(a.tiles, full, (int64_t)p->n_rows * (p->kv_heads / a.heads_per_wave) * gy, compute_units());
         a.tiles = (a.tiles + a.query_tiles - 1) / a.query_tiles;
     }
     // 8-bit pages: two tiles a workgroup, two workgroups a compute unit still (FP8 in 242-252 registers; the row-scaled
@@ -379,11 +384,6 @@ static int launch_attend_checked(const crit_pkv_attend_params* p, hipStream_t st
     }
     const int64_t gx = (int64_t)p->n_rows * (a.hkv / a.heads_per_wave) * a.tiles;
     if (gx > 0x7fffffff) return CRIT_PKV_E_GEOMETRY;
-    // Positions past the page tables do not exist: partitions that could only hold such pieces are not launched.
-    const int64_t table_keys = (int64_t)p->table_width * p->page;
-    a.max_keys = (int)(table_keys < 0x3fffffff ? table_keys : 0x3fffffff);
-    const int64_t live_parts = ((p->blocks ? (int64_t)a.listed_keys : (int64_t)a.max_keys) + (int64_t)p->piece - 1) / p->piece;
-    const unsigned gy = (unsigned)(live_parts < p->partitions ? live_parts : p->partitions);
     const dim3 grid((unsigned)gx, p->fused ? 1u : gy);
     a.units_x = a.units_y = 0;
     // The unit-pulling launches draw their units from the caller's two counters; without them units are dealt in turn.

@@ -668,6 +668,7 @@ def attend(q, key_pages, value_pages, kind, tables, rows, starts, firsts, column
     p.partitions, p.piece, p.fused, p.sliding, p.phases = parts, piece, int(bool(fused)), sliding, int(phases)
     p.scale, p.key_multiplier, p.value_multiplier = scale, km, vm
     p.int8_qk = int(bool(int8_qk))
+    p.window_tokens = 0 if offsets is None else int(tokens)
     if fresh is not None:
         fk, fv, fshift, ffirst = fresh
         if derive is not None:      # (checked as the keys the values stand for: one width)

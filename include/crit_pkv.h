@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define CRIT_PKV_ABI_VERSION 20
+#define CRIT_PKV_ABI_VERSION 21
 
 /* Page kinds: the values of KINDS in the reference module (__init__.py:78). */
 #define CRIT_PKV_KIND_16BIT 0   /* bf16 or fp16 pages (page_dtype says which) */
@@ -187,6 +187,9 @@ typedef struct crit_pkv_attend_params {
      * read as window rows); fresh positions keep the queries' 16 bits. Not with blocks or derive. Such launches take
      * the generic kernel whatever the head width. */
     int32_t int8_qk;
+    /* The columns of all rows together (the sum of counts) where the caller knows them, else 0. Only the launch's split
+     * looks at it, never a result: with n_rows * columns every row is taken to have all its columns. */
+    int64_t window_tokens;
 } crit_pkv_attend_params;
 
 int crit_pkv_attend(const crit_pkv_attend_params* p, void* stream);

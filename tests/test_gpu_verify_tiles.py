@@ -68,3 +68,24 @@ def test_trees_and_sliding_windows_over_several_ragged_rows(kind, sliding, hkv, 
         for got, up in ((out, links[:n]), (plain, None)):
             want, _ = cache.want(q[start:start + n], s, first, n, sliding=sliding, parents=up)
             torch.testing.assert_close(got[start:start + n].double().cpu(), want, atol=ATOL, rtol=RTOL, msg=f"{s} {up}")
+
+
+@pytest.mark.parametrize("columns,g", [(5, 7), (6, 7), (9, 8)])
+def test_what_the_caller_says_of_its_columns_changes_no_bit(columns, g):
+    # 65 rows of 8 KV heads: enough of them that a launch of five, six or nine tiles takes three a workgroup only where the
+    # partial rows say that every row is full; here some are (as packed rows say), some are not (as unpacked ones may be)
+    rows = 65
+    lengths = [columns + 1 + (7 * r) % 50 for r in range(rows)]
+    cache = Cache("bf16", 8, 128, 128, 16, lengths)
+    q = rand_q(rows * columns, 8 * g, 128, 34)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)
+    for counts in ([columns] * rows, [columns - r % 3 for r in range(rows)], [1 + r % columns for r in range(rows)]):
+        starts, firsts = [columns * r for r in range(rows)], [n - c for n, c in zip(lengths, counts)]
+        run = lambda **kw: cache.attend(q, list(range(rows)), starts, firsts, columns, counts=i32(counts), out=torch.zeros_like(q, dtype=torch.bfloat16), **kw)
+        plain = run()
+        packed = [sum(counts[:r]) for r in range(rows)]
+        assert torch.equal(plain, run(offsets=i32(packed), tokens=sum(counts)))
+        assert torch.equal(plain, run(offsets=i32(starts), tokens=rows * columns))
+        for r in (0, 3, 64):
+            want, _ = cache.want(q[starts[r]:starts[r] + counts[r]], r, firsts[r], counts[r])
+            torch.testing.assert_close(plain[starts[r]:starts[r] + counts[r]].double().cpu(), want, atol=ATOL, rtol=RTOL, msg=str(r))

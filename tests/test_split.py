@@ -19,6 +19,7 @@ def split(tmp_path_factory):
     (where / "split.cpp").write_text("""#include "pkv_split.hpp"
 extern "C" int xcds_log2(int64_t pairs, int64_t tiles, int64_t units, int64_t held) { return pkv::xcds_of_pair_log2(pairs, tiles, units, held); }
 extern "C" int64_t workgroups(int64_t pairs, int64_t tiles, int l) { return pkv::dealt_workgroups(pairs, tiles, l); }
+extern "C" int window_tiles(int64_t tiles, int full, int64_t places, int64_t units) { return pkv::window_tiles_16bit(tiles, full != 0, places, units); }
 extern "C" void deal(int64_t pairs, int64_t tiles, int l, int* pair, int* tile) {
     const int64_t n = pkv::dealt_workgroups(pairs, tiles, l);
     for (int64_t w = 0; w < n; ++w) {
@@ -32,6 +33,7 @@ extern "C" void deal(int64_t pairs, int64_t tiles, int l, int* pair, int* tile) 
                     str(where / "split.cpp"), "-o", out], check=True)
     lib = ctypes.CDLL(out)
     lib.xcds_log2.argtypes, lib.workgroups.argtypes = [ctypes.c_int64] * 4, [ctypes.c_int64, ctypes.c_int64, ctypes.c_int]
+    lib.window_tiles.argtypes = [ctypes.c_int64, ctypes.c_int, ctypes.c_int64, ctypes.c_int64]
     lib.workgroups.restype = ctypes.c_int64
     lib.deal.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
     return lib
@@ -84,3 +86,21 @@ def test_short_chunks_of_a_long_launch_do_not_meet_on_one_xcd(split, pairs, live
 @pytest.mark.parametrize("pairs,tiles,held", [(17, 16, 32), (21, 16, 32), (33, 16, 32), (65, 16, 32), (63, 1, 64), (66, 1, 64), (7, 64, 32), (64, 8, 32)])
 def test_many_even_pairs_and_short_chunks_stay_whole(split, pairs, tiles, held):
     assert split.xcds_log2(pairs, tiles, UNITS, held) == 0
+
+
+def test_a_row_of_four_tiles_is_not_read_twice_in_a_large_launch(split):
+    # 64 rows of 4 head pairs and 16 partitions on 256 compute units: a launch sized for 5, 6 or 9 tiles whose rows may have
+    # fewer keeps them four a workgroup; where every row has them all, three hold them in as few workgroups
+    for tiles in range(1, 33):
+        for full in (0, 1):
+            for places in (1, 16, 128, 256, 257, 4096):
+                held = split.window_tiles(tiles, full, places, 256)
+                assert held == min(tiles, 2) if tiles < 3 else held in (3, 4)
+                assert tiles < 3 or -(-tiles // held) == -(-tiles // 4)      # never more workgroups for full rows
+                if not full and places > 256:
+                    for row in range(1, tiles + 1):      # a row of fewer tiles: no more workgroups than four a workgroup
+                        assert -(-row // held) <= max(1, -(-row // 4)) or tiles < 3, (tiles, row)
+    assert [split.window_tiles(t, 1, 4096, 256) for t in (3, 4, 5, 6, 7, 8, 9, 10)] == [3, 4, 3, 3, 4, 4, 3, 4]
+    assert [split.window_tiles(t, 0, 4096, 256) for t in (3, 4, 5, 6, 7, 8, 9, 10)] == [3, 4, 4, 4, 4, 4, 4, 4]
+    # one row of 4 head pairs and 64 partitions: its second workgroups run beside its first
+    assert [split.window_tiles(t, 0, 256, 256) for t in (5, 6, 9)] == [3, 3, 4] and split.window_tiles(9, 0, 42, 256) == 3
