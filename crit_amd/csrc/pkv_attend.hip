@@ -351,7 +351,7 @@ static int launch_attend_checked(const crit_pkv_attend_params* p, hipStream_t st
     const unsigned gy = (unsigned)(live_parts < p->partitions ? live_parts : p->partitions);
     // Windows of several tiles of 128-wide heads over 16-bit pages, split launch: a workgroup holds four tiles (one
     // workgroup a compute unit), or the two of a window of two (two workgroups still, with two dozen registers in
-    // scratch outside the steps), and reads the rows once for all of them. A tile's bits are the same however many
+    // scratch, all but four of a tree's accesses outside the steps), and reads the rows once for all of them. A tile's bits are the same however many
     // share a workgroup, so this may follow the launch. Measured on MI355X (32 / 8 heads, 64 rows ~U[1024, 8192]): 4
     // columns 383 -> 288 us, 5 columns 519 -> 424, 8 columns 676 -> 480; one row of 32,768: 55 -> 45, 72 -> 56 and 91 ->
     // 62. Not taken where it measured slower: four tiles of 8-bit pages (8 columns 376 -> 334 us but 5 columns 279 ->
@@ -365,7 +365,7 @@ static int launch_attend_checked(const crit_pkv_attend_params* p, hipStream_t st
         a.tiles = (a.tiles + a.query_tiles - 1) / a.query_tiles;
     }
     // 8-bit pages: two tiles a workgroup, two workgroups a compute unit still (FP8 in 242-252 registers; the row-scaled
-    // kinds with two dozen in scratch outside the steps). 64 rows, 4 / 5 / 8 columns: FP8 207 -> 147, 279 -> 214, 376 ->
+    // kinds with two dozen in scratch, one or two accesses of them inside the steps). 64 rows, 4 / 5 / 8 columns: FP8 207 -> 147, 279 -> 214, 376 ->
     // 230 us, INT8 224 -> 167, 307 -> 264, 428 -> 287 us; one row of 32,768 (FP8): 54 -> 52 and 64 -> 52 us, but a pair
     // alone (4 columns) 40 -> 51 us, so a window of two tiles pairs them only in launches that fill the card.
     if (a.fast128 && !p->blocks && !p->fused && wide128 && p->kind >= 1 && a.tiles >= 2) {

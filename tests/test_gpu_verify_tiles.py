@@ -1,5 +1,6 @@
-"""Verify windows read three query tiles a workgroup, and draft trees whose steps lie before, across and behind the window's
-first position: every column against float64 attention over the stored values and, bit for bit, against its fused launch."""
+"""Verify windows read three query tiles a workgroup, draft trees whose steps lie before, across and behind the window's
+first position, and trees and sliding windows over several rows of fewer columns than the launch: every column against
+float64 attention over the stored values and, bit for bit, against its fused launch."""
 import pytest
 import torch
 
