@@ -584,7 +584,7 @@ __global__ __launch_bounds__(256, (DH == 2 || QT > 2) ? 1 : kMfmaWaves) void att
                         // the lane's scores: its column at positions base + r_pos + i of head r_head; another head's column sees nothing
                         const int room = lim[q] - (base + r_pos);      // visible while i <= room
                         float x[4];
-                        if constexpr (MASK == kMaskNone) {
+                        if constexpr (MASK == kMaskNone) {      // (all four first: within the loop below INT8 pages took 84.4 us for 84.0)
 #pragma unroll
                             for (int i = 0; i < 4; ++i) x[i] = (s0[q][i] + s1[q][i]) * (KIND >= 2 ? sscale * ks4[i] : sscale);
                         }
