@@ -351,13 +351,13 @@ static int launch_attend_checked(const crit_pkv_attend_params* p, hipStream_t st
     const unsigned gy = (unsigned)(live_parts < p->partitions ? live_parts : p->partitions);
     // Windows of several tiles of 128-wide heads over 16-bit pages, split launch: a workgroup holds four tiles (one
     // workgroup a compute unit), or the two of a window of two (two workgroups still, with two dozen registers in
-    // scratch, all but four of a tree's accesses outside the steps), and reads the rows once for all of them. A tile's bits are the same however many
-    // share a workgroup, so this may follow the launch. Measured on MI355X (32 / 8 heads, 64 rows ~U[1024, 8192]): 4
-    // columns 383 -> 288 us, 5 columns 519 -> 424, 8 columns 676 -> 480; one row of 32,768: 55 -> 45, 72 -> 56 and 91 ->
-    // 62. Not taken where it measured slower: four tiles of 8-bit pages (8 columns 376 -> 334 us but 5 columns 279 ->
-    // 302, one row 55 -> 92: the converted rows' steps are too long a chain for one wavefront a SIMD).
-    // Three tiles, which leave nothing in scratch, in place of four where window_tiles_16bit() says so. (Three in a
-    // second workgroup's registers would spill 336 bytes a lane.)
+    // scratch, all but four of a tree's accesses outside the steps), and reads the rows once for all of them. A tile's
+    // bits are the same however many share a workgroup, so this may follow the launch. Measured on MI355X (32 / 8 heads,
+    // 64 rows ~U[1024, 8192]): 4 columns 383 -> 288 us, 5 columns 519 -> 424, 8 columns 676 -> 480; one row of 32,768:
+    // 55 -> 45, 72 -> 56 and 91 -> 62. Not taken where it measured slower: four tiles of 8-bit pages (8 columns 376 ->
+    // 334 us but 5 columns 279 -> 302, one row 55 -> 92: the converted rows' steps are too long a chain for one
+    // wavefront a SIMD). Three tiles, which leave nothing in scratch, in place of four where window_tiles_16bit() says
+    // so. (Three in a second workgroup's registers would spill 336 bytes a lane.)
     a.query_tiles = 1;
     if (a.fast128 && !p->blocks && !p->fused && wide128 && p->kind == 0 && a.tiles >= 2) {
         const bool full = !p->counts || p->window_tokens == (int64_t)p->n_rows * p->columns;
