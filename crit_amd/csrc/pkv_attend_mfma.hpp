@@ -94,6 +94,8 @@ PKV_DEV float sum_across_quarters(float x) {      // (row 0 + row 1) + (row 2 + 
     return u2f((uint32_t)b[0]) + u2f((uint32_t)b[1]);
 }
 
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));      // four floats of a workspace that is any floats
+
 template <int KIND, int DH>
 struct Tile {
     using VVec = typename std::conditional<KIND == 0, u32x4, u32x2>::type;
@@ -158,7 +160,7 @@ __global__ __launch_bounds__(256, (DH == 2 || QT > 2) ? 1 : kMfmaWaves) void att
     constexpr int EB = KIND == 0 ? 2 : 1;
     constexpr int CPH = kTileRows / HW;      // tile columns a KV head holds
     constexpr int SPW = kTileRows / HW;      // positions a wavefront's step covers (tile rows a KV head holds)
-    constexpr int EPT = kTileRows * D / 256; // output elements a thread folds
+    constexpr int FG = D / 64;               // groups of four output elements a thread folds: dims 64 i + 4 (tid % 16) .. + 3 of column tid / 16
     __shared__ __align__(16) float s_acc[4][kTileRows][D];
     __shared__ float s_m[4][kTileRows], s_l[4][kTileRows];
     __shared__ int s_rows[kLdsRows][5];      // count, first position, table row, first token, first partial row
@@ -513,9 +515,10 @@ __global__ __launch_bounds__(256, (DH == 2 || QT > 2) ? 1 : kMfmaWaves) void att
         if (cur.valid) {
             const int part_lo = FUSED ? 0 : cur.b;
             const int part_hi = FUSED ? min(a.parts, cur.n_pieces) : cur.b + 1;
-            float run_m[FUSED ? EPT : 1], run_l[FUSED ? EPT : 1], run_a[FUSED ? EPT : 1];
+            float run_m = -INFINITY, run_l = 0.0f;
+            f32x4 run_a[FUSED ? FG : 1];
 #pragma unroll
-            for (int e = 0; e < (FUSED ? EPT : 1); ++e) run_m[e] = -INFINITY, run_l[e] = 0.0f, run_a[e] = 0.0f;
+            for (int i = 0; i < (FUSED ? FG : 1); ++i) run_a[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             for (int part = part_lo; part < part_hi; ++part) {
                 float m[QT], l[QT];                  // the lane's column of each tile: running maximum (the same in its four lanes), the lane's share of the sum
                 f32x4 acc[QT][8 * DH];               // O^T: acc[q][8 h + j][i] = dim 128 h + 32 u4 + 8 i + j of the lane's column of tile q
@@ -716,69 +719,92 @@ __global__ __launch_bounds__(256, (DH == 2 || QT > 2) ? 1 : kMfmaWaves) void att
                 }
                 if (u4 == 0) s_m[wave][c16] = m[q], s_l[wave][c16] = l_col;
                 lds_barrier();
-#pragma unroll
-                for (int e = 0; e < EPT; ++e) {
-                    const int idx = tid + e * 256;
-                    const int cc = idx / D, d = idx % D;
+                // A thread folds FG groups of four dims of one column: what follows the column (its place, the maximum, the
+                // four factors) is made once a thread, and its partials leave in 16-byte stores. (An element a thread of eight
+                // columns each, that was 90 vector instructions an element: of a unit of three tiles half of all it ran. 64
+                // rows ~U[1024, 8192], 32 / 8 heads x 128, 5 columns: 369 -> 330 us; 56 / 8, one row of 50,000, 8 columns, INT8
+                // 123 -> 113; 8 rows of 16,000, 24 / 4 x 256, fp8:row 79 -> 74. The same bits.)
+                {
+                    const int cc = tid >> 4, d0 = 4 * (tid & 15);
                     const int head_i = cc / CPH;
                     const int j = fold_col_j0 + q * CPH + cc % CPH;
-                    const int c = j / a.g;
+                    const int c = j / a.g, in_group = j - c * a.g;
                     float M = s_m[0][cc];
 #pragma unroll
                     for (int w = 1; w < 4; ++w) M = __builtin_fmaxf(M, s_m[w][cc]);
                     const float sub = M == -INFINITY ? 0.0f : M;
-                    float L = 0.0f, A = 0.0f;
+                    float L = 0.0f, fw[4];
+                    f32x4 A[FG];
+#pragma unroll
+                    for (int i = 0; i < FG; ++i) A[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                     for (int w = 0; w < 4; ++w) {
-                        const float fw = exp2_fast(s_m[w][cc] - sub);
-                        L = __builtin_fmaf(s_l[w][cc], fw, L);
-                        A = __builtin_fmaf(s_acc[w][cc][d], fw, A);
+                        fw[w] = exp2_fast(s_m[w][cc] - sub);
+                        L = __builtin_fmaf(s_l[w][cc], fw[w], L);
+#pragma unroll
+                        for (int i = 0; i < FG; ++i) {
+                            const f32x4 x = *reinterpret_cast<const f32x4*>(&s_acc[w][cc][64 * i + d0]);
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) A[i][k] = __builtin_fmaf(x[k], fw[w], A[i][k]);
+                        }
                     }
-                    // NARROW: the element is kept where its dim lies in the 64 of its column's own KV head
-                    const int odd = NARROW ? ((j % a.g) >= (a.g >> 1) ? 1 : 0) : 0;
-                    const bool kept = !NARROW || (d >> 6) == odd;
+                    // NARROW: the 64 dims of the column's own KV head are kept
+                    const int odd = NARROW ? (in_group >= (a.g >> 1) ? 1 : 0) : 0;
                     if constexpr (KIND == 1) {
-                        if constexpr (NARROW) A *= a.hm ? a.hm[2 * a.hkv + 2 * (fold_kvh0 + head_i) + odd] : a.v_mult;
-                        else A *= HW == 1 ? vm_cur[0] : (head_i == 0 ? vm_cur[0] : vm_cur[HW - 1]);
+                        float vm;
+                        if constexpr (NARROW) vm = a.hm ? a.hm[2 * a.hkv + 2 * (fold_kvh0 + head_i) + odd] : a.v_mult;
+                        else vm = HW == 1 ? vm_cur[0] : (head_i == 0 ? vm_cur[0] : vm_cur[HW - 1]);
+#pragma unroll
+                        for (int i = 0; i < FG; ++i) A[i] *= vm;
                     }
-                    if (c < cur.count && kept) {
+                    if (c < cur.count) {
                         if constexpr (FUSED) {
                             // A column folds the partitions that hold its positions, as the merge does.
                             const int held = min(a.parts, (min(cur.first + c + 1, a.max_keys) + a.piece - 1) / a.piece);
                             if (part < held) {
-                                const Fold fo = fold(run_m[e], run_l[e], M, L);
-                                run_a[e] = __builtin_fmaf(run_a[e], fo.keep, A * fo.take);
-                                run_m[e] = fo.m, run_l[e] = fo.l;
+                                const Fold fo = fold(run_m, run_l, M, L);
+#pragma unroll
+                                for (int i = 0; i < FG; ++i)
+#pragma unroll
+                                    for (int k = 0; k < 4; ++k) run_a[i][k] = __builtin_fmaf(run_a[i][k], fo.keep, A[i][k] * fo.take);
+                                run_m = fo.m, run_l = fo.l;
                             }
                         } else {
-                            const int64_t at = ((int64_t)(cur.prow + c) * a.hq + (fold_kvh0 + head_i) * a.g + j % a.g) * a.parts + cur.b;
-                            if constexpr (NARROW) a.po[at * 64 + (d & 63)] = A;
-                            else a.po[at * D + d] = A;
-                            if ((d & (NARROW ? 63 : D - 1)) == 0) a.pm[at] = M, a.pl[at] = L;
+                            const int64_t at = ((int64_t)(cur.prow + c) * a.hq + (fold_kvh0 + head_i) * a.g + in_group) * a.parts + cur.b;
+                            float* to = a.po + at * (NARROW ? 64 : D) + d0;      // (4-byte aligned: the caller's workspace may be any floats)
+#pragma unroll
+                            for (int i = 0; i < FG; ++i) {
+                                if (!NARROW || i == odd) *reinterpret_cast<f32x4_any*>(to + (NARROW ? 0 : 64 * i)) = A[i];
+                            }
+                            if (d0 == 0) a.pm[at] = M, a.pl[at] = L;
                         }
                     }
                 }
                 }
             }
             if constexpr (FUSED) {
-#pragma unroll
-                for (int e = 0; e < EPT; ++e) {
-                    const int idx = tid + e * 256;
-                    const int cc = idx / D, d = idx % D;
-                    const int j = cur.j0 + cc % CPH;
-                    const int c = j / a.g;
-                    const bool kept = !NARROW || (d >> 6) == ((j % a.g) >= (a.g >> 1) ? 1 : 0);
-                    if (c < cur.count && kept) {
-                        const int head = (cur.kvh0 + cc / CPH) * a.g + j % a.g;
-                        float M = run_m[e], L = run_l[e], A = run_a[e];
-                        if (a.sinks) {
-                            const Fold fo = fold(M, L, a.sinks[head] * kLog2e, 1.0f);
-                            A *= fo.keep, M = fo.m, L = fo.l;
-                        }
-                        const float o = L != 0.0f ? A / L : 0.0f;
-                        store_out(a.out, a.out_dtype, (int64_t)(cur.start + c) * a.o_st + (int64_t)head * a.o_sh + (NARROW ? (d & 63) : d), o);
-                        if (a.lse && (d & (NARROW ? 63 : D - 1)) == 0) a.lse[(int64_t)(cur.start + c) * a.hq + head] = L != 0.0f ? __builtin_fmaf(M, kLn2, __logf(L)) : -INFINITY;
+                const int cc = tid >> 4, d0 = 4 * (tid & 15);
+                const int j = cur.j0 + cc % CPH;
+                const int c = j / a.g, in_group = j - c * a.g;
+                const int odd = NARROW ? (in_group >= (a.g >> 1) ? 1 : 0) : 0;
+                if (c < cur.count) {
+                    const int head = (cur.kvh0 + cc / CPH) * a.g + in_group;
+                    float M = run_m, L = run_l, keep = 1.0f;
+                    if (a.sinks) {
+                        const Fold fo = fold(M, L, a.sinks[head] * kLog2e, 1.0f);
+                        keep = fo.keep, M = fo.m, L = fo.l;
                     }
+                    const int64_t to = (int64_t)(cur.start + c) * a.o_st + (int64_t)head * a.o_sh + d0;
+#pragma unroll
+                    for (int i = 0; i < FG; ++i) {
+                        if (NARROW && i != odd) continue;
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            const float A = a.sinks ? run_a[i][k] * keep : run_a[i][k];
+                            store_out(a.out, a.out_dtype, to + (NARROW ? 0 : 64 * i) + k, L != 0.0f ? A / L : 0.0f);
+                        }
+                    }
+                    if (a.lse && d0 == 0) a.lse[(int64_t)(cur.start + c) * a.hq + head] = L != 0.0f ? __builtin_fmaf(M, kLn2, __logf(L)) : -INFINITY;
                 }
             }
         }
