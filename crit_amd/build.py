@@ -21,6 +21,11 @@ OBJ_DIR = os.path.join(LIB_DIR, "obj")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-fno-fast-math", "--offload-compress",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument"]
 
+# The window kernels' accumulators are rescaled by the vector pipe between products, which cannot reach the registers that
+# the compiler keeps products in for kernels of one wavefront a SIMD (160 moves a pair of steps with three query tiles):
+# their products take ordinary registers.
+OWN_FLAGS = {"pkv_attend_": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+
 
 def sources():
     return sorted(os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith(".hip"))
@@ -28,7 +33,8 @@ def sources():
 
 def _compile(src):
     obj = os.path.join(OBJ_DIR, os.path.basename(src)[:-4] + ".o")
-    cmd = ["hipcc", *FLAGS, *os.environ.get("CRIT_PKV_EXTRA_FLAGS", "").split(), "-c", src, "-o", obj]
+    own = [f for start, flags in OWN_FLAGS.items() if os.path.basename(src).startswith(start) for f in flags]
+    cmd = ["hipcc", *FLAGS, *own, *os.environ.get("CRIT_PKV_EXTRA_FLAGS", "").split(), "-c", src, "-o", obj]
     done = subprocess.run(cmd, capture_output=True, text=True)
     noise = "is not a recognized feature for this target"
     err = "\n".join(line for line in done.stderr.splitlines() if noise not in line)

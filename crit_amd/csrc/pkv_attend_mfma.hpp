@@ -4,19 +4,19 @@
 // The kernel is bound by HBM reads of K and V; everything else is arranged so that nothing but those reads limits it.
 // The two products of a step run on the matrix pipe, which a decode kernel otherwise leaves idle, because the vector
 // pipe cannot keep up with 8-bit pages at HBM rate (one v_dot2 per two multiply-adds, plus the conversions, was two
-// thirds of its cycles): a step is 16 positions of one KV head,
-//   S^T[16 positions][16 query rows] = K[16][128] . Q^T      4 x v_mfma_f32_16x16x32 (bf16 / f16 operands)
-//   O^T[128 dims][16 query rows]    += V^T[128][16] . P^T    8 x v_mfma_f32_16x16x16
-// with operands laid out so that nothing is shuffled between memory and the matrix pipe:
-//   keys    lane (p = lane % 16, u = lane / 16) loads 16-byte pieces of the row of position p; piece c holds dims
+// thirds of its cycles): a step is 16 positions of one KV head, and steps are taken in pairs,
+//   S^T[16 positions][16 query rows] = K[16][128] . Q^T      4 x v_mfma_f32_16x16x32 a step (bf16 / f16 operands)
+//   O^T[128 dims][16 query rows]    += V^T[128][32] . P^T    8 x v_mfma_f32_16x16x32 a pair
+// with operands laid out so that nothing is shuffled between the two products:
+//   keys    lane (p = lane % 16, u = lane / 16) holds 16-byte pieces of the row of position p; piece c holds dims
 //           32 c + 8 u .. + 7, the eight contraction elements the first product's A operand wants from that lane
-//           (8-bit pages: two loads of 16 codes, converted to 16-bit pairs, exactly);
-//   values  lane (i = lane % 16, u) loads 16 bytes (dims 8 i .. 8 i + 7) of the rows of positions 4 u .. 4 u + 3: a
-//           load instruction fetches four whole rows. The second product's A operand for dims {8 i + j} is the four
-//           positions' element j as two 16-bit pairs: one v_perm_b32 each;
-//   scores  come out with lane (c = lane % 16, u) holding query row c at positions 4 u .. 4 u + 3, which is exactly
-//           the B operand layout of the second product: the probabilities go from the softmax to the matrix pipe
-//           as two packed registers, no LDS, no shuffle.
+//           (8-bit pages: two pieces of 16 codes, converted to 16-bit pairs, exactly);
+//   scores  come out with lane (c = lane % 16, u) holding query row c at positions 4 u .. 4 u + 3, which is half of
+//           the B operand of the second product, the pair's other step the other half: the probabilities go from the
+//           softmax to the matrix pipe as four packed registers, no LDS, no shuffle;
+//   values  lane (i, u) holds a dim of the rows of positions 4 u .. 4 u + 3 of both steps, as four 16-bit pairs.
+// A pair has one maximum, one factor and one sum a query row where two steps had two, and half the products for the
+// values.
 // The 16 query rows of a tile are rows of the flattened (column, group head) list, so the GQA group's heads share
 // every K/V byte read once. A wavefront serves HW adjacent KV heads (2 where the head count is even) in ONE matrix tile:
 // a step is then 8 positions of both heads (rows 0 .. 7 of the tile the first head's positions, rows 8 .. 15 the
@@ -24,11 +24,21 @@
 // other head's queries are masked), so a load instruction fetches both heads' rows of a position, 512 contiguous bytes
 // of 16-bit pages: what the HBM system streams best from randomly placed pages.
 // Softmax state: the running maximum of a query row is kept equal in the four lanes that hold the row (two
-// v_permlane swaps a step), the sums per lane until the unit's end. NT tiles are in flight per wavefront; every load
-// of the loop is unconditional, so the waits are exact counts.
+// v_permlane swaps a pair), the sums per lane until the unit's end.
 //
-// Row-exactness: position n is always read in the same step of the same wavefront of its unit, at the same place of
-// the matrix operands; the matrix pipe computes each output element from its own row and column only; every other
+// How a step's rows reach their operands. With one or two query tiles over 16-bit pages a wavefront loads them straight
+// into the operands' registers, a pair in flight beside the one in use, two workgroups a compute unit. A key operand's lanes
+// lie in 16 different rows, so such a load is 64 requests of 16 bytes to the cache instead of 16 of 64 (5.7 requests a
+// 128-byte line over the kernel, by its counters), and the registers of several tiles, of 256-wide heads or of converted
+// codes leave no room for loads in flight. So all other kernels have the memory pipe write a wavefront's rows into its
+// own ring in LDS (global_load_lds: no register holds them, a request takes 64 adjacent bytes) and read the operands from
+// there, values transposed by the LDS itself (ds_read_b64_tr_b16). Nothing is shared between wavefronts, so no barrier
+// orders the ring: the waits count loads. Against the same kernels with all rows in registers: 64 rows ~U[1024, 8192], 32
+// / 8 heads x 128, 5 columns BF16 331 -> 298 us; 8 rows of 16,000, 24 / 4 x 256, fp8:row 74 -> 67; one row of 50,000, 56 /
+// 8, 8 columns, INT8 116 -> 98.
+//
+// Row-exactness: position n is always read in the same step of the same pair of the same wavefront of its unit (pairs do
+// not cross pieces), at the same place of the matrix operands; the matrix pipe computes each output element from its own row and column only; every other
 // reduction is a fixed tree. So a column's bits depend on its own query and keys, `piece`, `partitions`, the page kind
 // and the cache geometry only: not on the rows beside it, the launch's width, the tile it falls in, which workgroup
 // served it, or `fused`.
@@ -45,17 +55,6 @@ PKV_DEV f32x4 mfma_k32(u32x4 a, u32x4 b, f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
     }
 }
-template <bool F16>
-PKV_DEV f32x4 mfma_k16(u32x2 a, u32x2 b, f32x4 c) {
-    typedef __attribute__((ext_vector_type(4))) short s16x4;
-    typedef __attribute__((ext_vector_type(4))) _Float16 f16x4;
-    if constexpr (F16) {
-        return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4, a), __builtin_bit_cast(f16x4, b), c, 0, 0, 0);
-    } else {
-        return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), c, 0, 0, 0);
-    }
-}
-
 template <bool F16>
 PKV_DEV uint32_t pair16(float a, float b) {      // two FP32 values as one 16-bit pair, round to nearest even
     if constexpr (F16) return pack_f16(a, b);
@@ -96,23 +95,67 @@ PKV_DEV float sum_across_quarters(float x) {      // (row 0 + row 1) + (row 2 + 
 
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));      // four floats of a workspace that is any floats
 
-template <int KIND, int DH>
-struct Tile {
-    using VVec = typename std::conditional<KIND == 0, u32x4, u32x2>::type;
-    u32x4 k[(KIND == 0 ? 4 : 2) * DH];      // the lane's pieces of its position's K row
-    VVec v[4][DH];                           // the lane's 8 dims (of each 128-wide half) of the V rows of its quarter's four positions
-    float ks[KIND >= 2 ? 4 : 1], vs[KIND >= 2 ? 4 : 1];      // row-scaled kinds: the scales of positions 4 u .. 4 u + 3
+struct Tile {      // a step in registers (16-bit pages, 128-wide heads)
+    u32x4 k[4];      // the lane's pieces of its position's key row
+    u32x4 v[4];      // the lane's 8 dims of the value rows of its quarter's four positions
 };
+
+// Piece c of a lane's key row as the first product's A operand: 16-bit values as they are, codes as 16-bit pairs, exactly.
+template <int KIND>
+PKV_DEV u32x4 key_operand(const u32x4* k, int c) {
+    if constexpr (KIND == 0) {
+        return k[c];
+    } else {
+        const uint32_t w0 = c % 2 ? k[c / 2].z : k[c / 2].x, w1 = c % 2 ? k[c / 2].w : k[c / 2].y;
+        const u32x2 lo = codes4_to_pairs<KIND>(w0), hi = codes4_to_pairs<KIND>(w1);
+        return u32x4{lo.x, lo.y, hi.x, hi.y};
+    }
+}
 
 constexpr int kMaskNone = 0, kMaskTree = 1, kMaskSliding = 2;
 constexpr int kTileRows = 16;      // query rows (columns of S^T) a tile holds
 constexpr int kLdsRows = 512;      // batch rows whose descriptors a workgroup keeps in LDS (the others are read from memory)
 
-// Wavefronts a SIMD holds (workgroups a compute unit) and steps a wavefront keeps in flight. Measured on MI355X: three
-// workgroups a unit (fewer registers each) and four steps in flight both stream less (the memory system is saturated by
-// two and two; more concurrent streams cost DRAM locality).
+// Workgroups a compute unit holds where one or two tiles a wavefront leave the registers for them. Measured on MI355X:
+// three of them (fewer registers each) and four steps in flight a wavefront both stream less (the memory system is
+// saturated by two and two; more concurrent streams cost DRAM locality).
 constexpr int kMfmaWaves = 2;
-constexpr int kMfmaTiles = 2;
+
+// Where a kernel keeps the steps in flight. 16-bit pages of 128-wide heads with one query tile or two: in registers, two
+// workgroups a compute unit. Everything else: in LDS, sent there by the memory pipe itself (a ring of a wavefront's own).
+template <int KIND, int DH, int QT>
+struct MfmaShape {
+    static constexpr bool kRing = KIND != 0 || DH == 2 || QT > 2;
+    static constexpr int kGroups = DH == 2 || QT > 2 ? 1 : kMfmaWaves;      // workgroups a compute unit
+    static constexpr int kPairs = kRing && kGroups == 1 && !(DH == 2 && KIND == 0) ? 2 : 1;      // pairs of steps in flight a wavefront
+};
+
+// 64 lanes x 16 bytes from base + offset (a lane's own) to LDS bytes lds .. lds + 1023 (ONCE: not kept in the caches), and
+// 4 bytes a lane to lds + 4 lane. Spelled in assembly so that the compiler neither counts these loads nor waits for them:
+// the waits are the kernel's own (wait_dma), and "memory" clobbers, which keeps the reads of LDS behind them.
+template <bool ONCE>
+PKV_DEV void dma_rows(uint32_t offset, const uint8_t* base, unsigned lds) {
+    lds = (unsigned)__builtin_amdgcn_readfirstlane((int)lds);      // (uniform; it may have been kept in a vector register)
+    if constexpr (ONCE) asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(offset), "s"(base), "s"(lds));
+    else asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds));
+}
+PKV_DEV void dma_words(const float* from, unsigned lds) {
+    lds = (unsigned)__builtin_amdgcn_readfirstlane((int)lds);
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(from), "s"(lds));
+}
+template <int N>
+PKV_DEV void wait_dma() {
+    static_assert(N >= 0 && N < 64, "vmcnt is six bits");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// The wavefront's own LDS reads have returned: what they read may be overwritten.
+PKV_DEV void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+// 4 consecutive rows of one value, transposed on the way out of LDS: lane 4 j + c of a 16-lane group points at row j's
+// values 4 c .. 4 c + 3; lane i of the group receives value i of rows 0 .. 3.
+PKV_DEV u32x2 read_transposed(const uint8_t* p) {
+    typedef short v4 __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4*)(p)));
+}
 
 // The launch: as many workgroups as the card holds at once, each working through units of the list (row, KV head
 // group, query tile, partition) until it is exhausted. The hardware's own dispatcher binds a workgroup to an XCD by its
@@ -139,9 +182,8 @@ constexpr int kMfmaTiles = 2;
 // state and accumulators, so a tile's bits are what they are alone and the rows are read once for QT tiles instead of
 // once a tile. More than one tile takes the registers of a second workgroup on the compute unit (one stays). Built for
 // four or three tiles (or a window's two) of 128-wide heads over 16-bit pages and two over 8-bit pages (pairs still fit two
-// workgroups a compute unit), where it measured faster (64 rows ~U[1024, 8192] of 32 / 8 heads, 8 columns: 676 -> 480 us, FP8 376 -> 224);
-// pairs of tiles of 256-wide heads keep one step in flight a wavefront instead of two (NT), or their registers spill;
-// four tiles of 8-bit pages measured slower.
+// workgroups a compute unit) or of 256-wide heads, where it measured faster (64 rows ~U[1024, 8192] of 32 / 8 heads, 8
+// columns: 676 -> 480 us, FP8 376 -> 224); four tiles of 8-bit pages measured slower.
 // NARROW: 64-wide heads, read as 128-wide ones. Two adjacent KV heads' rows of a position are 128 contiguous values,
 // which is what a 128-wide head's row is: the launcher hands the kernel half the KV heads at twice the width and GQA
 // groups twice as large (a group's first half the query heads of the even KV head, its second half the odd one's: the
@@ -151,22 +193,35 @@ constexpr int kMfmaTiles = 2;
 // the 128-wide kernel's loads: 512 contiguous bytes a position and wavefront. What follows a KV head (row scales, an
 // FP8 pool's multipliers) is looked up by the column's own head.
 template <int KIND, bool F16, int HW, bool FUSED, int MASK, int DH = 1, int QT = 1, bool NARROW = false>
-__global__ __launch_bounds__(256, (DH == 2 || QT > 2) ? 1 : kMfmaWaves) void attend_mfma_kernel(AttendArgs a) {
+__global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void attend_mfma_kernel(AttendArgs a) {
     static_assert(!NARROW || (DH == 1 && QT == 1), "64-wide heads: one 128-wide pair a tile row, one tile a workgroup");
-    constexpr int NT = DH == 2 && QT == 2 ? 1 : kMfmaTiles;
+    constexpr bool RING = MfmaShape<KIND, DH, QT>::kRing;
+    constexpr int NP = MfmaShape<KIND, DH, QT>::kPairs, NT = 2 * NP;      // pairs of steps in flight, steps
     constexpr int D = 128 * DH;
     static_assert(DH == 1 || (DH == 2 && HW == 1), "heads of 128 or 256; one KV head a wavefront at 256");
     static_assert(QT == 1 || !FUSED, "several query tiles: the split launch");
     constexpr int EB = KIND == 0 ? 2 : 1;
     constexpr int CPH = kTileRows / HW;      // tile columns a KV head holds
     constexpr int SPW = kTileRows / HW;      // positions a wavefront's step covers (tile rows a KV head holds)
-    constexpr int FG = D / 64;               // groups of four output elements a thread folds: dims 64 i + 4 (tid % 16) .. + 3 of column tid / 16
-    __shared__ __align__(16) float s_acc[4][kTileRows][D];
+    constexpr int FW = RING ? 64 : D;        // output dims folded at a time
+    constexpr int FG = FW / 64;              // groups of four of them a thread folds: dims 64 i + 4 (tid % 16) .. + 3 of column tid / 16
+    constexpr int ROWB = D * EB;             // bytes of a key or value row
+    constexpr int CPR = ROWB / 16;           // its 16-byte chunks
+    constexpr int HALF = 16 * ROWB;          // a step's keys (its values follow)
+    constexpr int NKI = HALF / 1024;         // loads of a wavefront they take
+    constexpr int SCI = KIND >= 2 ? 1 : 0;   // ... and their rows' scales
+    constexpr int NK = 2 * (NKI + SCI), NV = 2 * NKI;      // ... a pair's keys with all scales, its values
+    constexpr int SCN = NARROW ? 64 : 32;    // scales of a step: keys', values' (NARROW: the even heads', the odd ones', twice)
+    __shared__ __align__(16) float s_acc[4][kTileRows][FW];
+    __shared__ __align__(1024) uint8_t s_ring[RING ? 4 : 1][RING ? NT : 1][RING ? 2 * HALF : 16];
+    __shared__ __align__(16) float s_scales[RING && KIND >= 2 ? 4 : 1][RING && KIND >= 2 ? NT : 1][RING && KIND >= 2 ? SCN : 4];
     __shared__ float s_m[4][kTileRows], s_l[4][kTileRows];
     __shared__ int s_rows[kLdsRows][5];      // count, first position, table row, first token, first partial row
     __shared__ int s_before[kLdsRows + 1];   // the dense list: partitions but the last of the rows before row r
     __shared__ int s_wave_sum[4];
-    __shared__ int s_key[kLdsRows], s_order[kLdsRows];      // the dense list: the rows by the size of their last partition
+    __shared__ uint16_t s_order[kLdsRows];   // the dense list: the rows by the size of their last partition
+    int* const s_key = reinterpret_cast<int*>(&s_acc[0][0][0]);      // ... (while the list is made)
+    static_assert(sizeof(s_acc) >= kLdsRows * sizeof(int), "the list's keys lie in the fold's array");
     __shared__ unsigned s_unit;
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -247,7 +302,7 @@ __global__ __launch_bounds__(256, (DH == 2 || QT > 2) ? 1 : kMfmaWaves) void att
                     rank += (other > key || (other == key && o < r)) ? 1 : 0;
                 }
             }
-            s_order[rank] = r;
+            s_order[rank] = (uint16_t)r;
         }
         lds_barrier();
     }
@@ -345,70 +400,105 @@ __global__ __launch_bounds__(256, (DH == 2 || QT > 2) ? 1 : kMfmaWaves) void att
     uint32_t vvo[4];
 #pragma unroll
     for (int p = 0; p < 4; ++p) vvo[p] = (uint32_t)((r_pos + p) * slot_bytes + r_head * D * EB + c16 * 8 * EB);
-    const uint32_t svo = (uint32_t)(r_pos * a.hkv + r_head);      // row-scaled kinds: the lane's first score row's scale
+    // A ring's step in LDS: the tile's 16 key rows (row i: position i % SPW of head i / SPW), then its value rows. The memory
+    // pipe writes lane i's 16 bytes at byte 16 i of a kilobyte, whatever it fetched for that lane, so a load's lanes take
+    // adjacent chunks of a row (four lanes a 64-byte request, where the operand's own layout would be a request a lane)
+    // and the chunks of a row are stored permuted, chunk c of row i at place c ^ turn(i) (in its low four bits), which
+    // spreads the operands' reads (16 rows, one chunk each) over all banks. 8-bit values are not permuted, but row
+    // 4 u + p lies in place 4 p + u: a read takes rows p, 4 + p, 8 + p, 12 + p.
+    auto turn = [](int row) __attribute__((always_inline)) -> int { return CPR == 8 ? (row >> 1) & 7 : 2 * (row & 7) + (row >> 3); };
+    uint32_t k_from[NKI], v_from[NKI];
+    if constexpr (RING) {
+#pragma unroll
+        for (int j = 0; j < NKI; ++j) {
+            const int place = 64 * j + lane, row = place / CPR, c = place % CPR;
+            k_from[j] = (uint32_t)((row % SPW) * slot_bytes + (row / SPW) * ROWB + 16 * (c ^ turn(row)));
+            if constexpr (KIND == 0) {
+                v_from[j] = k_from[j];
+            } else {
+                const int vrow = 4 * (row & 3) + (row >> 2);
+                v_from[j] = (uint32_t)((vrow % SPW) * slot_bytes + (vrow / SPW) * ROWB + 16 * c);
+            }
+        }
+    }
+    const unsigned ring_at = (unsigned)__builtin_amdgcn_readfirstlane((int)(uintptr_t)&s_ring[RING ? wave : 0][0][0]);
+    const unsigned scales_at = (unsigned)__builtin_amdgcn_readfirstlane((int)(uintptr_t)&s_scales[RING && KIND >= 2 ? wave : 0][0][0]);
+    const uint32_t k_read = (uint32_t)(c16 * ROWB + 16 * (u4 ^ turn(c16)));      // chunk 4 l + u4 of row c16: ^ 64 l (+ 256 from l = 4 on)
+    const int t_row = 4 * u4 + (c16 >> 2);      // 16-bit values, transposed: four values of row t_row, of every 16 dims
+    const uint32_t t_read = (uint32_t)(t_row * ROWB + 8 * (c16 & 1)), t_turn = (uint32_t)(16 * (((c16 & 3) >> 1) ^ turn(t_row)));
+    // the scale this lane sends to LDS: of which head's keys or values, and of which row of the tile
+    const int sc_row = lane & 15, sc_odd = NARROW ? (lane >> 4) & 1 : 0;
+    const float* sc_from = (lane >> (NARROW ? 5 : 4)) & 1 ? a.vs : a.ks;
+    if constexpr (RING && KIND >= 2)
+        sc_from += NARROW ? (sc_row % SPW) * 2 * a.hkv + 2 * (sc_row / SPW) + sc_odd : (sc_row % SPW) * a.hkv + sc_row / SPW;
 
-    // -- a wavefront's walk over a partition's steps: steps wave, wave + 4, ... of pieces part, part + parts, ...
-    // (positions stay below 2^31: the launcher bounds partitions x piece)
-    struct Walk {
-        int pi, st;
+    // -- a wavefront's steps of a partition: steps wave, wave + 4, ... of pieces part, part + parts, ..., taken in pairs
+    // within a piece (a piece's last pair may lack its second step). Lane 2 i + r holds the first position and the table
+    // entry of step r of pair from + i, for 32 pairs at a time: one load of the page table, and no wait on it in the loop.
+    // A step that is not there has position -1 and the entry of one that is.
+    struct Steps {
+        int base, entry, in_page, from, first_piece;
+        uint32_t slot;
     };
-    auto walk_base = [&](const Unit& un, const Walk& w) __attribute__((always_inline)) -> int {
-        if (w.st * SPW >= a.piece) return -1;
-        const int base = w.pi * a.piece + w.st * SPW;
-        return base < un.n_keys ? base : -1;
+    const int steps_a_piece = a.piece / SPW;
+    const int pairs_a_piece = ((steps_a_piece - wave + 3) / 4 + 1) / 2;      // this wavefront's (0: too short a piece for it)
+    auto hold = [&](const Unit& un, int first_piece, int from) __attribute__((always_inline)) -> Steps {
+        Steps s;
+        s.from = from, s.first_piece = first_piece;
+        const int n = from + (lane >> 1), r = lane & 1;
+        const int turns = n / max(pairs_a_piece, 1), k = n - turns * pairs_a_piece;
+        const int piece = first_piece + turns * a.parts;
+        const int st = wave + 8 * k;
+        const bool there = pairs_a_piece > 0 && piece < un.n_pieces;
+        const int at = there ? piece * a.piece + st * SPW : 0x7fffffff - 8 * SPW;      // (pieces of the row: positions below 2^31)
+        const bool one = at < un.n_keys, two = one && st + 4 < steps_a_piece && at + 4 * SPW < un.n_keys;
+        s.base = r == 0 ? (one ? at : -1) : (two ? at + 4 * SPW : -1);
+        const int of = s.base >= 0 ? s.base : (one ? at : 0);
+        const int page = of >> a.page_shift;
+        s.entry = a.tables[un.trow + (page < a.tab_width ? page : a.tab_width - 1)];
+        s.in_page = of & (a.page - 1);
+        s.slot = 0u;
+        return s;
     };
-    auto walk_advance = [&](const Unit& un, Walk& w) __attribute__((always_inline)) -> int {
-        w.st += 4;
-        if (w.st * SPW >= a.piece) w.pi += a.parts, w.st = wave;
-        return walk_base(un, w);
-    };
-    auto entry = [&](const Unit& un, int base) __attribute__((always_inline)) -> int {     // the page table entry of a step (uniform over the wavefront)
-        int pidx = base >> a.page_shift;
-        pidx = pidx < a.tab_width ? pidx : a.tab_width - 1;
-        return a.tables[un.trow + pidx];
-    };
-    // The first steps of a partition with their page table entries: NT steps to fill the buffers and the NT after them.
-    struct Lead {
-        int base[2 * NT], e[2 * NT];
-        Walk w;
-    };
-    auto lead_of = [&](const Unit& un, int part) __attribute__((always_inline)) -> Lead {
-        Lead f;
-        f.w.pi = part, f.w.st = wave;
+    auto resolve = [&](Steps& s) __attribute__((always_inline)) { s.slot = (uint32_t)s.entry * (uint32_t)a.page + (uint32_t)s.in_page; };
+    auto steps_of = [&](const Unit& un, int part) __attribute__((always_inline)) -> Steps {
+        int first_piece = part;
         if (win > 0) {      // pieces wholly below the tile's window are skipped (no row sees them)
             const int wlo = un.first + un.c_lo - win + 1;
             const int below = (wlo > 0 ? wlo : 0) / a.piece - part;
-            if (below > 0) f.w.pi = part + (below + a.parts - 1) / a.parts * a.parts;
+            if (below > 0) first_piece = part + (below + a.parts - 1) / a.parts * a.parts;
         }
-        f.base[0] = walk_base(un, f.w);
-        const int again = f.base[0] >= 0 ? f.base[0] : 0;      // (a wavefront without a step reads position 0's entry)
-        f.e[0] = entry(un, again);
-#pragma unroll
-        for (int i = 1; i < 2 * NT; ++i) {
-            f.base[i] = f.base[i - 1] >= 0 ? walk_advance(un, f.w) : -1;
-            f.e[i] = entry(un, f.base[i] >= 0 ? f.base[i] : again);
-        }
-        return f;
+        return hold(un, first_piece, 0);
     };
-    // A step's positions lie in one page (pages are powers of two from 16 up): its first slot, uniform.
-    auto first_slot = [&](int base, int e) __attribute__((always_inline)) -> int64_t {
-        return (int64_t)__builtin_amdgcn_readfirstlane(e) * a.page + (base & (a.page - 1));
+    struct Pair {
+        int base, second;      // the steps' first positions; -1: no such step
+        uint32_t s0, s1;       // their first slots (of a step that is not there: another's)
+    };
+    auto pair_no = [&](const Unit& un, Steps& s, int n) __attribute__((always_inline)) -> Pair {
+        if (n - s.from >= 32) s = hold(un, s.first_piece, s.from + 32), resolve(s);
+        const int l = 2 * (n - s.from);
+        Pair p;
+        p.base = __builtin_amdgcn_readlane(s.base, l), p.second = __builtin_amdgcn_readlane(s.base, l + 1);
+        p.s0 = (uint32_t)__builtin_amdgcn_readlane((int)s.slot, l), p.s1 = (uint32_t)__builtin_amdgcn_readlane((int)s.slot, l + 1);
+        return p;
     };
     // Loads of one step from its first slot. Every lane loads its place of the step whether the row holds that
     // position or not (the page does; a step past the row's keys is never listed): what such a place holds is dropped
     // where it is used (keys: the score is masked; values and scales: zeroed, see sanitize()).
     // (NARROW: `odd`, whether this lane's column is a query row of the pair's odd KV head; the scales are per KV head)
-    auto fetch_k = [&](const Unit& un, int64_t slot0, Tile<KIND, DH>& t, int odd) __attribute__((always_inline)) {
-        const uint8_t* sbase = a.kp + slot0 * slot_bytes + un.kvh0 * D * EB;
+    Tile t[RING ? 1 : NT];
+    auto fetch_k = [&](const Unit& un, uint32_t slot0, int i) __attribute__((always_inline)) {
+        const uint8_t* sbase = a.kp + (int64_t)slot0 * slot_bytes + un.kvh0 * ROWB;
+        if constexpr (RING) {
 #pragma unroll
-        for (int c = 0; c < (KIND == 0 ? 4 : 2) * DH; ++c) t.k[c] = *reinterpret_cast<const u32x4*>(sbase + kvo + 64 * c);
-        if constexpr (KIND >= 2) {
-            const int heads = NARROW ? 2 * a.hkv : a.hkv;      // scales a slot
-            const int first = NARROW ? (int)svo * 2 + odd : (int)svo;      // (svo = r_pos * hkv + r_head)
-            const float* ks = a.ks + slot0 * heads + (NARROW ? 2 * un.kvh0 : un.kvh0);
-            const float* vs = a.vs + slot0 * heads + (NARROW ? 2 * un.kvh0 : un.kvh0);
+            for (int j = 0; j < NKI; ++j) dma_rows<false>(k_from[j], sbase, ring_at + (unsigned)(i * 2 * HALF + 1024 * j));
+            if constexpr (KIND >= 2) {
+                if (SCN == 64 || lane < SCN)
+                    dma_words(sc_from + ((int64_t)slot0 * a.hkv + un.kvh0) * (NARROW ? 2 : 1), scales_at + (unsigned)(i * SCN * 4));
+            }
+        } else {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) t.ks[i] = ks[first + i * heads], t.vs[i] = vs[first + i * heads];
+            for (int c = 0; c < 4; ++c) t[i].k[c] = *reinterpret_cast<const u32x4*>(sbase + kvo + 64 * c);
         }
     };
     // NARROW: whether this lane's tile column (a query row of the flattened list) belongs to the pair's odd KV head.
@@ -416,13 +506,14 @@ __global__ __launch_bounds__(256, (DH == 2 || QT > 2) ? 1 : kMfmaWaves) void att
         if constexpr (!NARROW) return 0;
         return ((un.j0 + c16 % CPH) % a.g) >= (a.g >> 1) ? 1 : 0;
     };
-    auto fetch_v = [&](const Unit& un, int64_t slot0, Tile<KIND, DH>& t) __attribute__((always_inline)) {
-        const uint8_t* sbase = a.vp + slot0 * slot_bytes + un.kvh0 * D * EB;
+    auto fetch_v = [&](const Unit& un, uint32_t slot0, int i) __attribute__((always_inline)) {
+        const uint8_t* sbase = a.vp + (int64_t)slot0 * slot_bytes + un.kvh0 * ROWB;
+        if constexpr (RING) {
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
+            for (int j = 0; j < NKI; ++j) dma_rows<true>(v_from[j], sbase, ring_at + (unsigned)(i * 2 * HALF + HALF + 1024 * j));
+        } else {
 #pragma unroll
-            for (int h = 0; h < DH; ++h)
-                t.v[p][h] = __builtin_nontemporal_load(reinterpret_cast<const typename Tile<KIND, DH>::VVec*>(sbase + vvo[p] + h * 128 * EB));
+            for (int p = 0; p < 4; ++p) t[i].v[p] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(sbase + vvo[p]));
         }
     };
 
@@ -446,6 +537,14 @@ __global__ __launch_bounds__(256, (DH == 2 || QT > 2) ? 1 : kMfmaWaves) void att
     auto lane_values = [&](const Unit& un) __attribute__((always_inline)) {
         const int odd = odd_of(un);
         if constexpr (KIND == 1) sscale = a.sscale * (a.hm ? a.hm[NARROW ? 2 * (un.kvh0 + hsel) + odd : un.kvh0 + hsel] : a.k_mult);
+        // (16-bit and FP8 pages: the scale rides on the exponent's multiply-add and on the maximum, so it is kept positive,
+        // its sign in the queries, and above zero: a hidden position's score of -inf times it stays -inf)
+        uint32_t flip = 0u;
+        if constexpr (KIND < 2) {
+            const float given = KIND == 1 ? sscale : a.sscale;
+            flip = given < 0.0f ? 0x80008000u : 0u;
+            sscale = __builtin_fmaxf(__builtin_fabsf(given), 0x1p-126f);
+        }
 #pragma unroll
         for (int q = 0; q < QT; ++q) {
             const int jr = un.j0 + q * CPH + c16 % CPH;
@@ -465,28 +564,28 @@ __global__ __launch_bounds__(256, (DH == 2 || QT > 2) ? 1 : kMfmaWaves) void att
                 } else {
                     if (live) qb[q][c] = *reinterpret_cast<const u32x4*>(row + dim * 2);
                 }
+                if constexpr (KIND < 2) qb[q][c] ^= u32x4{flip, flip, flip, flip};
             }
         }
     };
 
-    Tile<KIND, DH> t[NT];
-    auto fill = [&](const Unit& un, const Lead& f) __attribute__((always_inline)) {      // a partition's first NT steps
-        const int again = f.base[0] >= 0 ? f.base[0] : 0;
-        const int odd = odd_of(un);
+    auto fill = [&](const Unit& un, Steps& s) __attribute__((always_inline)) {      // a partition's first NP pairs
 #pragma unroll
-        for (int i = 0; i < NT; ++i) {
-            const int64_t slot = first_slot(f.base[i] >= 0 ? f.base[i] : again, f.e[i]);
-            fetch_k(un, slot, t[i], odd), fetch_v(un, slot, t[i]);
+        for (int i = 0; i < NP; ++i) {
+            const Pair p = pair_no(un, s, i);
+            fetch_k(un, p.s0, 2 * i), fetch_k(un, p.s1, 2 * i + 1);
+            fetch_v(un, p.s0, 2 * i), fetch_v(un, p.s1, 2 * i + 1);
         }
     };
 
     unsigned u_next = blockIdx.x + grid;
     Unit cur = decode(blockIdx.x);
-    Lead lead_cur;
+    Steps steps = {};
     if (cur.valid) {
-        lead_cur = lead_of(cur, FUSED ? 0 : cur.b);
+        steps = steps_of(cur, FUSED ? 0 : cur.b);
         value_multipliers(cur);
-        fill(cur, lead_cur);
+        resolve(steps);
+        fill(cur, steps);
         lane_values(cur);
 #pragma unroll
         for (int h = 0; h < HW; ++h) vm_cur[h] = vm_nxt[h];
@@ -494,9 +593,9 @@ __global__ __launch_bounds__(256, (DH == 2 || QT > 2) ? 1 : kMfmaWaves) void att
     for (;;) {
         // The next unit: its first steps' page table entries are requested now and wait in registers.
         const Unit nxt = decode(u_next);
-        Lead lead_nxt = {};
+        Steps steps_nxt = {};
         if (nxt.valid) {
-            lead_nxt = lead_of(nxt, FUSED ? 0 : nxt.b);
+            steps_nxt = steps_of(nxt, FUSED ? 0 : nxt.b);
             value_multipliers(nxt);
         }
         // The ticket of the unit after the next is drawn when the current unit's steps are done (a returning atomic
@@ -506,7 +605,8 @@ __global__ __launch_bounds__(256, (DH == 2 || QT > 2) ? 1 : kMfmaWaves) void att
         auto hand_over = [&]() __attribute__((always_inline)) {
             if (pulled && tid == 0) drawn = atomicAdd(a.ticket, 1u);
             if (nxt.valid) {
-                fill(nxt, lead_nxt);
+                resolve(steps_nxt);
+                fill(nxt, steps_nxt);
                 lane_values(nxt);
             }
             sent = true;
@@ -516,9 +616,9 @@ __global__ __launch_bounds__(256, (DH == 2 || QT > 2) ? 1 : kMfmaWaves) void att
             const int part_lo = FUSED ? 0 : cur.b;
             const int part_hi = FUSED ? min(a.parts, cur.n_pieces) : cur.b + 1;
             float run_m = -INFINITY, run_l = 0.0f;
-            f32x4 run_a[FUSED ? FG : 1];
+            f32x4 run_a[FUSED ? D / 64 : 1];
 #pragma unroll
-            for (int i = 0; i < (FUSED ? FG : 1); ++i) run_a[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int i = 0; i < (FUSED ? D / 64 : 1); ++i) run_a[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             for (int part = part_lo; part < part_hi; ++part) {
                 float m[QT], l[QT];                  // the lane's column of each tile: running maximum (the same in its four lanes), the lane's share of the sum
                 f32x4 acc[QT][8 * DH];               // O^T: acc[q][8 h + j][i] = dim 128 h + 32 u4 + 8 i + j of the lane's column of tile q
@@ -529,257 +629,344 @@ __global__ __launch_bounds__(256, (DH == 2 || QT > 2) ? 1 : kMfmaWaves) void att
                     for (int j = 0; j < 8 * DH; ++j) acc[q][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                 }
 
-                auto step = [&](int base, Tile<KIND, DH>& tl, auto&& refill_k, auto&& refill_v) __attribute__((always_inline)) {
-                    if (base + SPW > cur.n_keys) {
-                        // The row's last step: what lies past its keys may be anything, and a probability of zero
-                        // times a NaN is a NaN.
-#pragma unroll
-                        for (int p = 0; p < 4; ++p) {
-                            if (base + r_pos + p >= cur.n_keys) {
-#pragma unroll
-                                for (int h = 0; h < DH; ++h) {
-                                    if constexpr (KIND == 0) tl.v[p][h] = u32x4{0, 0, 0, 0};
-                                    else tl.v[p][h] = u32x2{0, 0};
-                                }
-                                if constexpr (KIND >= 2) tl.vs[p] = 0.0f;
-                            }
-                        }
-                    }
-                    // -- scores
-                    u32x4 ka[4 * DH];
-                    if constexpr (KIND == 0) {
-#pragma unroll
-                        for (int c = 0; c < 4 * DH; ++c) ka[c] = tl.k[c];
-                    } else {
-#pragma unroll
-                        for (int c = 0; c < 4 * DH; ++c) {
-                            const uint32_t w0 = c % 2 ? tl.k[c / 2].z : tl.k[c / 2].x, w1 = c % 2 ? tl.k[c / 2].w : tl.k[c / 2].y;
-                            const u32x2 lo = codes4_to_pairs<KIND>(w0), hi = codes4_to_pairs<KIND>(w1);
-                            ka[c] = u32x4{lo.x, lo.y, hi.x, hi.y};
-                        }
-                    }
+                const int odd_cur = odd_of(cur);
+                // A pair of steps, in places 2 i and 2 i + 1: positions base .. + SPW - 1 and second .. + SPW - 1 (second < 0: no such
+                // step). keys_here and values_here wait until the pair's have landed.
+                auto step = [&](int base, int second, int i, auto&& keys_here, auto&& values_here, auto&& refill_k, auto&& refill_v) __attribute__((always_inline)) {
+                    const int base_b = second >= 0 ? second : 0x3fffff00;      // (past every column's last position)
+                    keys_here();
+                    // -- scores: the two steps' are two chains of products
                     f32x4 s0[QT], s1[QT];
 #pragma unroll
-                    for (int q = 0; q < QT; ++q) {
-                        s0[q] = mfma_k32<F16>(ka[0], qb[q][0], f32x4{0.0f, 0.0f, 0.0f, 0.0f});
-                        s1[q] = mfma_k32<F16>(ka[1], qb[q][1], f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+                    for (int q = 0; q < QT; ++q) s0[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f}, s1[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    const uint8_t* const place_a = &s_ring[RING ? wave : 0][RING ? 2 * i : 0][0];
+                    const uint8_t* const place_b = &s_ring[RING ? wave : 0][RING ? 2 * i + 1 : 0][0];
+                    u32x4 held[2][RING ? CPR / 4 : 1];
+                    if constexpr (RING) {
+#pragma unroll
+                        for (int l = 0; l < CPR / 4; ++l) {
+                            const uint32_t at = (k_read ^ (uint32_t)(64 * (l & 3))) + (uint32_t)(256 * (l >> 2));
+                            held[0][l] = *reinterpret_cast<const u32x4*>(place_a + at);
+                            held[1][l] = *reinterpret_cast<const u32x4*>(place_b + at);
+                        }
                     }
 #pragma unroll
-                    for (int c = 2; c < 4 * DH; c += 2) {      // (two chains, the even pieces and the odd ones)
+                    for (int c = 0; c < 4 * DH; ++c) {
+                        const u32x4 ka = key_operand<KIND>(RING ? held[0] : t[RING ? 0 : 2 * i].k, c), kb = key_operand<KIND>(RING ? held[1] : t[RING ? 0 : 2 * i + 1].k, c);
 #pragma unroll
                         for (int q = 0; q < QT; ++q) {
-                            s0[q] = mfma_k32<F16>(ka[c], qb[q][c], s0[q]);
-                            s1[q] = mfma_k32<F16>(ka[c + 1], qb[q][c + 1], s1[q]);
+                            s0[q] = mfma_k32<F16>(ka, qb[q][c], s0[q]);
+                            s1[q] = mfma_k32<F16>(kb, qb[q][c], s1[q]);
                         }
                     }
-                    float ks4[4], vs4[4];
+                    float ks8[8], vs8[8];
+                    if constexpr (KIND >= 2) {
+                        const int first = NARROW ? 16 * odd_cur : 0;
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) ks4[i] = KIND >= 2 ? tl.ks[i] : 1.0f, vs4[i] = KIND >= 2 ? tl.vs[i] : 1.0f;
-                    refill_k();      // (the keys' registers are free: the loads of NT steps ahead go out)
-                    u32x2 pb[QT];
-                    // A draft tree's step wholly before the window's first position: every column of the row sees all of
-                    // it, so nothing is asked a position (a shift by 64 bits and three comparisons each, on the vector
-                    // pipe that 8-bit pages keep busy: one row of 50,000, 56 / 8 heads, 8 columns, INT8 179 -> 124 us; 64
-                    // rows ~U[1024, 8192], 32 / 8 heads, 5 columns INT8 370 -> 283 us, BF16 518 -> 393; the same bits).
-                    const bool before = MASK == kMaskTree && win <= 0 && base + SPW <= min(cur.first, cur.n_keys);
+                        for (int r = 0; r < 2; ++r) {
+                            const float* sc = s_scales[wave][2 * i + r];
+                            const f32x4 k4 = *reinterpret_cast<const f32x4*>(sc + first + 4 * u4), v4 = *reinterpret_cast<const f32x4*>(sc + SCN / 2 + first + 4 * u4);
+#pragma unroll
+                            for (int p = 0; p < 4; ++p) ks8[4 * r + p] = k4[p], vs8[4 * r + p] = v4[p];
+                        }
+                        if (base_b + SPW > cur.n_keys) {      // (scales past the row's keys may be anything)
+#pragma unroll
+                            for (int p = 0; p < 8; ++p) vs8[p] = (p < 4 ? base : base_b) + r_pos + (p & 3) < cur.n_keys ? vs8[p] : 0.0f;
+                        }
+                    }
+                    if constexpr (RING) wait_lds();
+                    refill_k();      // (the keys' registers are free: the loads of NP pairs ahead go out)
+                    // Both steps wholly seen by every column of the tiles (a draft tree's: before the window's first
+                    // position): nothing is asked of a position.
+                    const bool whole = MASK != kMaskSliding && win <= 0 &&
+                                       base_b + SPW <= min(MASK == kMaskTree ? cur.first : cur.first + cur.c_lo + 1, cur.n_keys);
+                    // The lane's scores: its column at positions base + r_pos + i, second + r_pos + i of head r_head. Another
+                    // head's column (a lane that is not `mine`) sees nothing: its scores stay out of the maximum, its
+                    // probabilities become zeros (chosen, not multiplied: the other head's values may be anything).
+                    float x[QT][8], top[QT];
 #pragma unroll
                     for (int q = 0; q < QT; ++q) {
-                        // the lane's scores: its column at positions base + r_pos + i of head r_head; another head's column sees nothing
-                        const int room = lim[q] - (base + r_pos);      // visible while i <= room
-                        float x[4];
-                        if constexpr (MASK == kMaskNone) {      // (all four first: within the loop below INT8 pages took 84.4 us for 84.0)
 #pragma unroll
-                            for (int i = 0; i < 4; ++i) x[i] = (s0[q][i] + s1[q][i]) * (KIND >= 2 ? sscale * ks4[i] : sscale);
+                        for (int i = 0; i < 8; ++i) {
+                            const float raw = i < 4 ? s0[q][i & 3] : s1[q][i & 3];
+                            x[q][i] = KIND >= 2 ? raw * (sscale * ks8[i]) : raw;
                         }
-                        if (MASK == kMaskTree && before) {
-                            const bool vis = mine && lim[q] >= 0;
+                        if (!whole) {
+                            const int room = lim[q] - r_pos;      // position n (of the step's first) is visible while n + i <= room
 #pragma unroll
-                            for (int i = 0; i < 4; ++i) x[i] = vis ? (s0[q][i] + s1[q][i]) * (KIND >= 2 ? sscale * ks4[i] : sscale) : -INFINITY;
-                        } else {
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) {
-                                if constexpr (MASK != kMaskNone) x[i] = (s0[q][i] + s1[q][i]) * (KIND >= 2 ? sscale * ks4[i] : sscale);
-                                bool vis = mine && i <= room;
+                            for (int i = 0; i < 8; ++i) {
+                                const int at = (i < 4 ? base : base_b) + (i & 3);
+                                bool vis = at <= room;
                                 if constexpr (MASK != kMaskNone) {
-                                    const int n = base + r_pos + i;
+                                    const int n = at + r_pos;
                                     if (tree) vis = vis && (n < cur.first || ((anc[q] >> ((n - cur.first) & 63)) & 1ull) != 0);
                                     if (win > 0) vis = vis && n > cur.first + col[q] - win;
                                 }
-                                x[i] = vis ? x[i] : -INFINITY;
+                                x[q][i] = vis ? x[q][i] : -INFINITY;
                             }
                         }
-                        const float top = max_across_quarters(__builtin_fmaxf(__builtin_fmaxf(x[0], x[1]), __builtin_fmaxf(x[2], x[3])));
-                        const float m_new = __builtin_fmaxf(m[q], top);
-                        const float sub = m_new == -INFINITY ? 0.0f : m_new;
-                        const float alpha = m[q] == -INFINITY ? 1.0f : exp2_fast(m[q] - sub);      // (nothing summed yet: nothing to rescale)
-                        float p[4];
+                        float y = __builtin_fmaxf(__builtin_fmaxf(__builtin_fmaxf(x[q][0], x[q][1]), __builtin_fmaxf(x[q][2], x[q][3])),
+                                                  __builtin_fmaxf(__builtin_fmaxf(x[q][4], x[q][5]), __builtin_fmaxf(x[q][6], x[q][7])));
+                        if constexpr (KIND < 2) y *= sscale;      // (positive: -inf stays -inf)
+                        if constexpr (HW > 1) y = mine ? y : -INFINITY;
+                        top[q] = max_across_quarters(y);
+                    }
+                    bool moved[QT], any = false;
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) p[i] = exp2_fast(x[i] - sub);
-                        l[q] = __builtin_fmaf(l[q], alpha, (p[0] + p[1]) + (p[2] + p[3]));
-                        m[q] = m_new;
-                        if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {     // some row's maximum moved: rescale
+                    for (int q = 0; q < QT; ++q) moved[q] = top[q] > m[q], any = any || moved[q];
+                    if (__builtin_amdgcn_ballot_w64(any) != 0) {
+#pragma unroll
+                        for (int q = 0; q < QT; ++q) {
+                            const float alpha = moved[q] ? exp2_fast(m[q] - top[q]) : 1.0f;
+                            m[q] = moved[q] ? top[q] : m[q];
+                            l[q] *= alpha;
 #pragma unroll
                             for (int j = 0; j < 8 * DH; ++j) acc[q][j] *= alpha;
                         }
-                        pb[q] = u32x2{pair16<F16>(p[0] * vs4[0], p[1] * vs4[1]), pair16<F16>(p[2] * vs4[2], p[3] * vs4[3])};
                     }
-                    // -- values: dims {8 i + j} of the lane's four rows as two 16-bit pairs (one v_perm each), then O^T += V^T P^T
+                    u32x4 pb[QT];
 #pragma unroll
-                    for (int h = 0; h < DH; ++h) {
-                    if constexpr (KIND == 0) {
+                    for (int q = 0; q < QT; ++q) {
+                        const float sub = m[q] == -INFINITY ? 0.0f : m[q];
+                        float p[8];
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) p[i] = exp2_fast(KIND >= 2 ? x[q][i] - sub : __builtin_fmaf(x[q][i], sscale, -sub));
+                        const float sum = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+                        l[q] += HW == 1 || mine ? sum : 0.0f;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const uint32_t w = KIND >= 2 ? pair16<F16>(p[2 * i] * vs8[2 * i], p[2 * i + 1] * vs8[2 * i + 1]) : pair16<F16>(p[2 * i], p[2 * i + 1]);
+                            pb[q][i] = HW == 1 || mine ? w : 0u;
+                        }
+                    }
+                    values_here();
+                    // The row's last steps: what lies past its keys may be anything, and a probability of zero times a NaN is a
+                    // NaN. Such values become zeros.
+                    auto clean = [&](int at, int place) __attribute__((always_inline)) {
+                        if (at + SPW > cur.n_keys) {
+                            if constexpr (RING) {
+                                uint8_t* values = &s_ring[wave][place][HALF];
+                                for (int row = 0; row < 16; ++row) {
+                                    if (at + row % SPW < cur.n_keys) continue;
+                                    uint8_t* to = values + (KIND == 0 ? row : 4 * (row & 3) + (row >> 2)) * ROWB;
+                                    for (int b = lane * 4; b < ROWB; b += 256) *reinterpret_cast<uint32_t*>(to + b) = 0u;
+                                }
+                            } else {
+#pragma unroll
+                                for (int p = 0; p < 4; ++p)
+                                    if (at + r_pos + p >= cur.n_keys) t[RING ? 0 : place].v[p] = u32x4{0, 0, 0, 0};
+                            }
+                        }
+                    };
+                    clean(base, 2 * i), clean(base_b, 2 * i + 1);
+                    // -- values: the lane's dims of the eight rows as four 16-bit pairs, then O^T += V^T P^T
+                    if constexpr (!RING) {      // dims {8 i + j}: a v_perm a pair
+                        const Tile&ta = t[RING ? 0 : 2 * i], &tb = t[RING ? 0 : 2 * i + 1];
 #pragma unroll
                         for (int w = 0; w < 4; ++w) {
-                            const u32x2 lo = {__builtin_amdgcn_perm(tl.v[1][h][w], tl.v[0][h][w], 0x05040100), __builtin_amdgcn_perm(tl.v[3][h][w], tl.v[2][h][w], 0x05040100)};
-                            const u32x2 hi = {__builtin_amdgcn_perm(tl.v[1][h][w], tl.v[0][h][w], 0x07060302), __builtin_amdgcn_perm(tl.v[3][h][w], tl.v[2][h][w], 0x07060302)};
+                            u32x4 lo, hi;
+#pragma unroll
+                            for (int r = 0; r < 2; ++r) {
+                                const Tile& tl = r == 0 ? ta : tb;
+                                lo[2 * r] = __builtin_amdgcn_perm(tl.v[1][w], tl.v[0][w], 0x05040100), lo[2 * r + 1] = __builtin_amdgcn_perm(tl.v[3][w], tl.v[2][w], 0x05040100);
+                                hi[2 * r] = __builtin_amdgcn_perm(tl.v[1][w], tl.v[0][w], 0x07060302), hi[2 * r + 1] = __builtin_amdgcn_perm(tl.v[3][w], tl.v[2][w], 0x07060302);
+                            }
 #pragma unroll
                             for (int q = 0; q < QT; ++q) {
-                                acc[q][8 * h + 2 * w] = mfma_k16<F16>(lo, pb[q], acc[q][8 * h + 2 * w]);
-                                acc[q][8 * h + 2 * w + 1] = mfma_k16<F16>(hi, pb[q], acc[q][8 * h + 2 * w + 1]);
+                                acc[q][2 * w] = mfma_k32<F16>(lo, pb[q], acc[q][2 * w]);
+                                acc[q][2 * w + 1] = mfma_k32<F16>(hi, pb[q], acc[q][2 * w + 1]);
                             }
                         }
-                    } else {
+                    } else if constexpr (KIND == 0) {      // dims 16 b + (0 .. 15): transposed by the LDS
 #pragma unroll
-                        for (int w = 0; w < 2; ++w) {
-                            // bytes (a0 b0 a1 b1) and (a2 b2 a3 b3): two rows' codes of one dim side by side
-                            const uint32_t lo01 = __builtin_amdgcn_perm(tl.v[1][h][w], tl.v[0][h][w], 0x05010400), hi01 = __builtin_amdgcn_perm(tl.v[1][h][w], tl.v[0][h][w], 0x07030602);
-                            const uint32_t lo23 = __builtin_amdgcn_perm(tl.v[3][h][w], tl.v[2][h][w], 0x05010400), hi23 = __builtin_amdgcn_perm(tl.v[3][h][w], tl.v[2][h][w], 0x07030602);
-                            // (dims 4 w + 0, 1 from the low halves, 2, 3 from the high ones; .x: rows 0, 1; .y: rows 2, 3)
-                            const u32x2 a01 = codes4_to_pairs<KIND>(lo01), a23 = codes4_to_pairs<KIND>(lo23);
-                            const u32x2 b01 = codes4_to_pairs<KIND>(hi01), b23 = codes4_to_pairs<KIND>(hi23);
-                            const u32x2 va[4] = {u32x2{a01.x, a23.x}, u32x2{a01.y, a23.y}, u32x2{b01.x, b23.x}, u32x2{b01.y, b23.y}};
+                        for (int b = 0; b < 8 * DH; ++b) {
+                            const uint32_t at = (uint32_t)HALF + t_read + (t_turn ^ (uint32_t)(32 * (b & 7))) + (uint32_t)(256 * (b >> 3));
+                            const u32x2 x = read_transposed(place_a + at), y = read_transposed(place_b + at);
+                            const u32x4 va = {x.x, x.y, y.x, y.y};
 #pragma unroll
-                            for (int q = 0; q < QT; ++q) {
+                            for (int q = 0; q < QT; ++q) acc[q][b] = mfma_k32<F16>(va, pb[q], acc[q][b]);
+                        }
+                    } else {      // dims {8 i + j}: codes of adjacent rows side by side, then as 16-bit pairs
 #pragma unroll
-                                for (int j = 0; j < 4; ++j) acc[q][8 * h + 4 * w + j] = mfma_k16<F16>(va[j], pb[q], acc[q][8 * h + 4 * w + j]);
+                        for (int h = 0; h < DH; ++h) {
+                            u32x2 v[2][4];
+#pragma unroll
+                            for (int p = 0; p < 4; ++p) {
+                                const uint32_t at = (uint32_t)(HALF + (4 * p + u4) * ROWB + 128 * h + 8 * c16);
+                                v[0][p] = *reinterpret_cast<const u32x2*>(place_a + at), v[1][p] = *reinterpret_cast<const u32x2*>(place_b + at);
+                            }
+#pragma unroll
+                            for (int w = 0; w < 2; ++w) {
+                                u32x4 va[4];
+#pragma unroll
+                                for (int r = 0; r < 2; ++r) {
+                                    // bytes (a0 b0 a1 b1) and (a2 b2 a3 b3): two rows' codes of one dim side by side
+                                    const uint32_t lo01 = __builtin_amdgcn_perm(v[r][1][w], v[r][0][w], 0x05010400), hi01 = __builtin_amdgcn_perm(v[r][1][w], v[r][0][w], 0x07030602);
+                                    const uint32_t lo23 = __builtin_amdgcn_perm(v[r][3][w], v[r][2][w], 0x05010400), hi23 = __builtin_amdgcn_perm(v[r][3][w], v[r][2][w], 0x07030602);
+                                    // (dims 4 w + 0, 1 from the low halves, 2, 3 from the high ones; .x: rows 0, 1; .y: rows 2, 3)
+                                    const u32x2 a01 = codes4_to_pairs<KIND>(lo01), a23 = codes4_to_pairs<KIND>(lo23);
+                                    const u32x2 b01 = codes4_to_pairs<KIND>(hi01), b23 = codes4_to_pairs<KIND>(hi23);
+                                    va[0][2 * r] = a01.x, va[0][2 * r + 1] = a23.x, va[1][2 * r] = a01.y, va[1][2 * r + 1] = a23.y;
+                                    va[2][2 * r] = b01.x, va[2][2 * r + 1] = b23.x, va[3][2 * r] = b01.y, va[3][2 * r + 1] = b23.y;
+                                }
+#pragma unroll
+                                for (int q = 0; q < QT; ++q) {
+#pragma unroll
+                                    for (int j = 0; j < 4; ++j) acc[q][8 * h + 4 * w + j] = mfma_k32<F16>(va[j], pb[q], acc[q][8 * h + 4 * w + j]);
+                                }
                             }
                         }
                     }
-                    }
+                    if constexpr (RING) wait_lds();
                     refill_v();
                 };
 
-                // Software pipeline over NT steps: a step's keys are reloaded (for NT steps ahead) as soon as its
-                // scores are issued, its values as soon as its second product is; the page table entries run NT steps
-                // further ahead. While the NT steps ahead all exist the loop's loads are unconditional (exact waits);
-                // the wavefront's last steps are peeled: no step is loaded that is not used (a re-read of an earlier
-                // step would come from HBM again: the caches have long turned over).
-                Lead f = lead_cur;
-                const int odd_cur = odd_of(cur);
                 if (part != part_lo) {
-                    f = lead_of(cur, part);
-                    fill(cur, f);
+                    steps = steps_of(cur, part);
+                    resolve(steps);
+                    fill(cur, steps);
                 }
-                if (f.base[0] >= 0) {
-                    const int again = f.base[0];
-                    int at[NT], ahead[NT], e_ahead[NT];
+                Pair at[NP];
 #pragma unroll
-                    for (int i = 0; i < NT; ++i) at[i] = f.base[i], ahead[i] = f.base[NT + i], e_ahead[i] = f.e[NT + i];
-                    while (ahead[NT - 1] >= 0) {
+                for (int i = 0; i < NP; ++i) at[i] = pair_no(cur, steps, i);
+                int n = NP;      // the next pair to send for
+                if constexpr (RING) {
+                    // A pair's keys are sent for again (NP pairs ahead) as soon as its scores are issued, its values as soon as
+                    // its second product is; loads return in order, so a wait counts the younger ones that are surely there.
 #pragma unroll
-                        for (int i = 0; i < NT; ++i) {
-                            const int after = walk_advance(cur, f.w);      // NT steps past the one this buffer is refilled with
-                            const int e_after = entry(cur, after >= 0 ? after : again);
-                            const int64_t slot = first_slot(ahead[i], e_ahead[i]);
-                            step(at[i], t[i], [&]() __attribute__((always_inline)) { fetch_k(cur, slot, t[i], odd_cur); },
-                                 [&]() __attribute__((always_inline)) { fetch_v(cur, slot, t[i]); });
-                            at[i] = ahead[i], ahead[i] = after, e_ahead[i] = e_after;
+                    for (int q = 0; q < QT; ++q)      // (the queries are waited for here: the compiler's count knows only them)
+#pragma unroll
+                        for (int c = 0; c < 4 * DH; ++c) asm volatile("" ::"v"(qb[q][c].x), "v"(qb[q][c].y), "v"(qb[q][c].z), "v"(qb[q][c].w));
+                    bool alive = true;
+                    while (alive) {
+#pragma unroll
+                        for (int i = 0; i < NP; ++i) {
+                            if (at[i].base < 0) {
+                                alive = false;
+                                break;
+                            }
+                            const Pair ahead = pair_no(cur, steps, n);
+                            const bool more = ahead.base >= 0, follows = NP == 2 && at[NP - 1 - i].base >= 0;
+                            step(at[i].base, at[i].second, i,
+                                 [&]() __attribute__((always_inline)) { if (follows) wait_dma<NV + NK + NV>(); else wait_dma<NV>(); },
+                                 [&]() __attribute__((always_inline)) {
+                                     if constexpr (NP == 2) { if (more) wait_dma<NK + NV + NK>(); else if (follows) wait_dma<NK + NV>(); else wait_dma<0>(); }
+                                     else { if (more) wait_dma<NK>(); else wait_dma<0>(); }
+                                 },
+                                 [&]() __attribute__((always_inline)) { if (more) fetch_k(cur, ahead.s0, 2 * i), fetch_k(cur, ahead.s1, 2 * i + 1); },
+                                 [&]() __attribute__((always_inline)) { if (more) fetch_v(cur, ahead.s0, 2 * i), fetch_v(cur, ahead.s1, 2 * i + 1); });
+                            at[i] = ahead, ++n;
                         }
                     }
-#pragma unroll
-                    for (int i = 0; i < NT; ++i) {
-                        if (at[i] >= 0) {
-                            const bool again_i = ahead[i] >= 0;
-                            const int64_t slot = first_slot(again_i ? ahead[i] : again, e_ahead[i]);
-                            step(at[i], t[i], [&]() __attribute__((always_inline)) { if (again_i) fetch_k(cur, slot, t[i], odd_cur); },
-                                 [&]() __attribute__((always_inline)) { if (again_i) fetch_v(cur, slot, t[i]); });
-                        }
+                } else if (at[0].base >= 0) {
+                    // In registers the compiler counts the loads: the loop's are unconditional (exact waits), the last pair is peeled.
+                    static_assert(RING || NP == 1, "one pair in registers");
+                    const auto none = []() {};
+                    Pair ahead = pair_no(cur, steps, n);
+                    while (ahead.base >= 0) {
+                        step(at[0].base, at[0].second, 0, none, none,
+                             [&]() __attribute__((always_inline)) { fetch_k(cur, ahead.s0, 0), fetch_k(cur, ahead.s1, 1); },
+                             [&]() __attribute__((always_inline)) { fetch_v(cur, ahead.s0, 0), fetch_v(cur, ahead.s1, 1); });
+                        at[0] = ahead;
+                        ahead = pair_no(cur, steps, ++n);
                     }
-#pragma unroll
-                    for (int i = 0; i < NT; ++i) {
-                        if (ahead[i] >= 0) step(ahead[i], t[i], []() {}, []() {});
-                    }
+                    step(at[0].base, at[0].second, 0, none, none, none, none);
                 }
                 // The unit's steps are done: the next unit's first keys, values and queries go out before the fold.
                 const int fold_col_j0 = cur.j0, fold_kvh0 = cur.kvh0;
                 if (part == part_hi - 1) hand_over();
 
                 // A tile's column sums over its four lanes, then the four wavefronts through LDS, in wavefront order; tile
-                // after tile through the same arrays.
+                // after tile (and FW dims after FW dims) through the same arrays. A thread folds FG groups of four dims of one
+                // column: what follows the column (its place, the maximum, the four factors) is made once a thread. Four
+                // adjacent dims lie together, group g of column c at place g ^ c (the columns' rows start in one bank).
 #pragma unroll
                 for (int q = 0; q < QT; ++q) {
-                const float l_col = sum_across_quarters(l[q]);
-                if (part != part_lo || q > 0) lds_barrier();      // the fold before has read the LDS
-#pragma unroll
-                for (int h = 0; h < DH; ++h) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        *reinterpret_cast<f32x4*>(&s_acc[wave][c16][128 * h + 32 * u4 + 8 * i]) = f32x4{acc[q][8 * h][i], acc[q][8 * h + 1][i], acc[q][8 * h + 2][i], acc[q][8 * h + 3][i]};
-                        *reinterpret_cast<f32x4*>(&s_acc[wave][c16][128 * h + 32 * u4 + 8 * i + 4]) = f32x4{acc[q][8 * h + 4][i], acc[q][8 * h + 5][i], acc[q][8 * h + 6][i], acc[q][8 * h + 7][i]};
-                    }
-                }
-                if (u4 == 0) s_m[wave][c16] = m[q], s_l[wave][c16] = l_col;
-                lds_barrier();
-                // A thread folds FG groups of four dims of one column: what follows the column (its place, the maximum, the
-                // four factors) is made once a thread, and its partials leave in 16-byte stores. (An element a thread of eight
-                // columns each, that was 90 vector instructions an element: of a unit of three tiles half of all it ran. 64
-                // rows ~U[1024, 8192], 32 / 8 heads x 128, 5 columns: 369 -> 330 us; 56 / 8, one row of 50,000, 8 columns, INT8
-                // 123 -> 113; 8 rows of 16,000, 24 / 4 x 256, fp8:row 79 -> 74. The same bits.)
-                {
-                    const int cc = tid >> 4, d0 = 4 * (tid & 15);
+                    const float l_col = sum_across_quarters(l[q]);
+                    const int cc = tid >> 4, g0 = tid & 15;
                     const int head_i = cc / CPH;
                     const int j = fold_col_j0 + q * CPH + cc % CPH;
                     const int c = j / a.g, in_group = j - c * a.g;
-                    float M = s_m[0][cc];
-#pragma unroll
-                    for (int w = 1; w < 4; ++w) M = __builtin_fmaxf(M, s_m[w][cc]);
-                    const float sub = M == -INFINITY ? 0.0f : M;
-                    float L = 0.0f, fw[4];
-                    f32x4 A[FG];
-#pragma unroll
-                    for (int i = 0; i < FG; ++i) A[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                    for (int w = 0; w < 4; ++w) {
-                        fw[w] = exp2_fast(s_m[w][cc] - sub);
-                        L = __builtin_fmaf(s_l[w][cc], fw[w], L);
-#pragma unroll
-                        for (int i = 0; i < FG; ++i) {
-                            const f32x4 x = *reinterpret_cast<const f32x4*>(&s_acc[w][cc][64 * i + d0]);
-#pragma unroll
-                            for (int k = 0; k < 4; ++k) A[i][k] = __builtin_fmaf(x[k], fw[w], A[i][k]);
-                        }
-                    }
-                    // NARROW: the 64 dims of the column's own KV head are kept
-                    const int odd = NARROW ? (in_group >= (a.g >> 1) ? 1 : 0) : 0;
+                    const int odd = NARROW ? (in_group >= (a.g >> 1) ? 1 : 0) : 0;      // NARROW: the 64 dims of the column's own KV head are kept
+                    float M = 0.0f, L = 0.0f, fw[4];
+                    float vm = 1.0f;
                     if constexpr (KIND == 1) {
-                        float vm;
                         if constexpr (NARROW) vm = a.hm ? a.hm[2 * a.hkv + 2 * (fold_kvh0 + head_i) + odd] : a.v_mult;
                         else vm = HW == 1 ? vm_cur[0] : (head_i == 0 ? vm_cur[0] : vm_cur[HW - 1]);
-#pragma unroll
-                        for (int i = 0; i < FG; ++i) A[i] *= vm;
                     }
-                    if (c < cur.count) {
+                    Fold fo = {};
+                    // A column folds the partitions that hold its positions, as the merge does.
+                    const int held = FUSED ? min(a.parts, (min(cur.first + c + 1, a.max_keys) + a.piece - 1) / a.piece) : 0;
+                    auto group = [&](int w, int col_, int g) __attribute__((always_inline)) -> f32x4* { return reinterpret_cast<f32x4*>(&s_acc[w][col_][4 * (g ^ col_)]); };
+#pragma unroll
+                    for (int sl = 0; sl < D / FW; ++sl) {
+                        if (part != part_lo || q > 0 || sl > 0) lds_barrier();      // the fold before has read the LDS
+                        if constexpr (RING && KIND == 0) {      // (acc[b][i] = dim 16 b + 4 u4 + i)
+#pragma unroll
+                            for (int b = 0; b < 4; ++b) *group(wave, c16, 4 * b + u4) = acc[q][4 * sl + b];
+                        } else if constexpr (RING) {            // (acc[8 h + j][i] = dim 128 h + 32 u4 + 8 i + j)
+                            if ((u4 >> 1) == (sl & 1)) {
+#pragma unroll
+                                for (int i = 0; i < 4; ++i) {
+                                    const f32x4* x = &acc[q][8 * (sl >> 1)];
+                                    *group(wave, c16, 8 * (u4 & 1) + 2 * i) = f32x4{x[0][i], x[1][i], x[2][i], x[3][i]};
+                                    *group(wave, c16, 8 * (u4 & 1) + 2 * i + 1) = f32x4{x[4][i], x[5][i], x[6][i], x[7][i]};
+                                }
+                            }
+                        } else {
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                *group(wave, c16, 8 * u4 + 2 * i) = f32x4{acc[q][0][i], acc[q][1][i], acc[q][2][i], acc[q][3][i]};
+                                *group(wave, c16, 8 * u4 + 2 * i + 1) = f32x4{acc[q][4][i], acc[q][5][i], acc[q][6][i], acc[q][7][i]};
+                            }
+                        }
+                        if (sl == 0 && u4 == 0) s_m[wave][c16] = m[q], s_l[wave][c16] = l_col;
+                        lds_barrier();
+                        if (sl == 0) {
+                            M = s_m[0][cc];
+#pragma unroll
+                            for (int w = 1; w < 4; ++w) M = __builtin_fmaxf(M, s_m[w][cc]);
+                            const float sub = M == -INFINITY ? 0.0f : M;
+#pragma unroll
+                            for (int w = 0; w < 4; ++w) {
+                                fw[w] = exp2_fast(s_m[w][cc] - sub);
+                                L = __builtin_fmaf(s_l[w][cc], fw[w], L);
+                            }
+                            if (FUSED && c < cur.count && part < held) {
+                                fo = fold(run_m, run_l, M, L);
+                                run_m = fo.m, run_l = fo.l;
+                            }
+                        }
+                        f32x4 A[FG];
+#pragma unroll
+                        for (int i = 0; i < FG; ++i) {
+                            A[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                            for (int w = 0; w < 4; ++w) {
+                                const f32x4 x = *group(w, cc, 16 * i + g0);
+#pragma unroll
+                                for (int k = 0; k < 4; ++k) A[i][k] = __builtin_fmaf(x[k], fw[w], A[i][k]);
+                            }
+                            if constexpr (KIND == 1) A[i] *= vm;
+                        }
+                        if (c >= cur.count) continue;
                         if constexpr (FUSED) {
-                            // A column folds the partitions that hold its positions, as the merge does.
-                            const int held = min(a.parts, (min(cur.first + c + 1, a.max_keys) + a.piece - 1) / a.piece);
                             if (part < held) {
-                                const Fold fo = fold(run_m, run_l, M, L);
 #pragma unroll
                                 for (int i = 0; i < FG; ++i)
 #pragma unroll
-                                    for (int k = 0; k < 4; ++k) run_a[i][k] = __builtin_fmaf(run_a[i][k], fo.keep, A[i][k] * fo.take);
-                                run_m = fo.m, run_l = fo.l;
+                                    for (int k = 0; k < 4; ++k) run_a[FG * sl + i][k] = __builtin_fmaf(run_a[FG * sl + i][k], fo.keep, A[i][k] * fo.take);
                             }
                         } else {
                             const int64_t at = ((int64_t)(cur.prow + c) * a.hq + (fold_kvh0 + head_i) * a.g + in_group) * a.parts + cur.b;
-                            float* to = a.po + at * (NARROW ? 64 : D) + d0;      // (4-byte aligned: the caller's workspace may be any floats)
 #pragma unroll
                             for (int i = 0; i < FG; ++i) {
-                                if (!NARROW || i == odd) *reinterpret_cast<f32x4_any*>(to + (NARROW ? 0 : 64 * i)) = A[i];
+                                const int d = FW * sl + 64 * i;      // (NARROW: the half d / 64 of the pair)
+                                if (!NARROW || d / 64 == odd) *reinterpret_cast<f32x4_any*>(a.po + at * (NARROW ? 64 : D) + (NARROW ? 0 : d) + 4 * g0) = A[i];
                             }
-                            if (d0 == 0) a.pm[at] = M, a.pl[at] = L;
+                            if (sl == 0 && g0 == 0) a.pm[at] = M, a.pl[at] = L;
                         }
                     }
-                }
                 }
             }
             if constexpr (FUSED) {
@@ -796,7 +983,7 @@ __global__ __launch_bounds__(256, (DH == 2 || QT > 2) ? 1 : kMfmaWaves) void att
                     }
                     const int64_t to = (int64_t)(cur.start + c) * a.o_st + (int64_t)head * a.o_sh + d0;
 #pragma unroll
-                    for (int i = 0; i < FG; ++i) {
+                    for (int i = 0; i < D / 64; ++i) {
                         if (NARROW && i != odd) continue;
 #pragma unroll
                         for (int k = 0; k < 4; ++k) {
@@ -819,17 +1006,18 @@ __global__ __launch_bounds__(256, (DH == 2 || QT > 2) ? 1 : kMfmaWaves) void att
                 s_unit = found;
             }
             lds_barrier();      // (and every thread is done with the fold's shared arrays)
-            u_after = s_unit;
+            u_after = (unsigned)__builtin_amdgcn_readfirstlane((int)s_unit);
         } else {
             lds_barrier();
         }
         if (!nxt.valid && u_next >= total && u_after >= total) break;
-        cur = nxt, lead_cur = lead_nxt;
+        cur = nxt, steps = steps_nxt;
 #pragma unroll
         for (int h = 0; h < HW; ++h) vm_cur[h] = vm_nxt[h];
         u_next = u_after;
         lds_barrier();      // every thread has read s_unit before the next round's draw is published
     }
+    if constexpr (RING) wait_dma<0>();      // (LDS must not be written for a workgroup that has gone)
     if (!pulled) return;
     if (threadIdx.x == 0) {
         if (atomicAdd(a.ticket + 1, 1u) == grid - 1) {
