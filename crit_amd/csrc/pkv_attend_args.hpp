@@ -41,6 +41,7 @@ struct AttendArgs {
     int tab_width, n_rows, columns, hq, hkv, g, page, page_shift, parts, piece, sliding, out_dtype, tiles, max_keys, heads_per_wave, units_x, units_y, query_tiles;
     int blocks_k, block_size, listed_keys;      // listed_keys = blocks_k * block_size: the positions a list's run holds
     Div32 block_div;
+    Div32 group_div, piece_div, tiles_div, row_div;      // the bandwidth kernel's quotients: by g, piece, tiles, a row's units a partition
     float sscale, k_mult, v_mult;
     // Fresh rows (attend's fresh=): row r reads its positions from f_firsts[r * f_per_row] on from rows
     // position - f_shifts[r * f_per_row] of fk / fv ([f_rows][kv_heads][dim], q's 16-bit type, unscaled) instead of the

@@ -167,6 +167,8 @@ static int launch_mfma(const AttendArgs& a, bool fused, dim3 grid, hipStream_t s
     u.units_x = (int)grid.x, u.units_y = fused ? (int)grid.y : (int)grid.y + kTailClasses - 1;
     const int64_t units = (int64_t)u.units_x * u.units_y;
     if (units > 0x7fffffff) return CRIT_PKV_E_GEOMETRY;
+    u.group_div = make_div32((uint32_t)a.g), u.piece_div = make_div32((uint32_t)a.piece), u.tiles_div = make_div32((uint32_t)a.tiles);
+    u.row_div = make_div32((uint32_t)(a.hkv / a.heads_per_wave * a.tiles));
     const int64_t resident = (int64_t)compute_units() * (a.dk == 256 || a.query_tiles > 2 ? 1 : kMfmaWaves);
     const dim3 pgrid((unsigned)(units < resident ? units : resident));
     // A unit a workgroup at most: nothing to draw, and no counter touched (a draw's round trip and the count of the

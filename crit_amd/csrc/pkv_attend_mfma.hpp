@@ -242,6 +242,10 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
     // its steps so that 98 registers a lane go to scratch instead of 39, 64 rows of 8 columns 600 us instead of 520.)
     const int win = MASK == kMaskSliding || (MASK == kMaskTree && QT > 3) ? a.sliding : 0;
 
+    // Quotients by the launch's own numbers (none of them a power of two in general: a division is forty instructions).
+    auto by_group = [&](int x) __attribute__((always_inline)) -> int { return (int)div32(a.group_div, (uint32_t)x); };
+    auto pieces_of = [&](int n_keys) __attribute__((always_inline)) -> int { return (int)div32(a.piece_div, (uint32_t)(n_keys + a.piece - 1)); };
+
     // -- every row's descriptors, once per workgroup
     auto row_from_memory = [&](int r, int (&d)[5]) __attribute__((always_inline)) {
         const int count = a.counts ? a.counts[r] : a.columns;
@@ -265,7 +269,7 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
         if (count <= 0) return 0;
         if constexpr (FUSED) return 1;
         const int n_keys = min(s_rows[r][1] + count, a.max_keys);
-        return min((n_keys + a.piece - 1) / a.piece, a.parts);
+        return min(pieces_of(n_keys), a.parts);
     };
     if (dense) {      // s_before[r] = sum over r' < r of max(partitions(r') - 1, 0): thread i sums rows 2 i and 2 i + 1
         const int r0 = 2 * tid, r1 = 2 * tid + 1;
@@ -286,23 +290,30 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
             int key = -1;
             if (count > 0) {
                 const int n_keys = min(s_rows[r][1] + count, a.max_keys);
-                const int n_pieces = (n_keys + a.piece - 1) / a.piece;
+                const int n_pieces = pieces_of(n_keys);
                 key = FUSED ? n_keys : (n_pieces > a.parts ? a.piece + 1 : n_keys - (n_pieces - 1) * a.piece);
             }
             s_key[r] = key;
         }
         lds_barrier();
-        for (int r = tid; r < a.n_rows; r += 256) {
-            int rank = r;
-            if (a.n_rows <= 256) {      // (larger launches keep the rows' order: ranking them costs more than it returns)
-                const int key = s_key[r];
-                rank = 0;
-                for (int o = 0; o < a.n_rows; ++o) {
-                    const int other = s_key[o];
-                    rank += (other > key || (other == key && o < r)) ? 1 : 0;
+        if (a.n_rows <= 256) {
+            // A row's place is the number of rows before it. A wavefront holds 64 rows' keys, a lane each, and goes through them by
+            // v_readlane: no round trip to LDS a row (64 rows: 4,800 of a workgroup's 22,000 clocks before its first step as a
+            // loop over LDS; with the quotients and the search by multiplications and ballots, 64 rows ~U[1024, 8192], 5 columns
+            // 298 -> 294 us, of 24 / 2 heads x 256 BF16, one column, 159 -> 154).
+            if (64 * wave < a.n_rows) {
+                const int key = tid < a.n_rows ? s_key[tid] : 0;
+                int rank = 0;
+                for (int r0 = 0; r0 < a.n_rows; r0 += 64) {
+                    const int keys = r0 + lane < a.n_rows ? s_key[r0 + lane] : 0;
+                    const int upto = min(64, a.n_rows - r0);
+#pragma unroll 4
+                    for (int o = 0; o < upto; ++o) rank += __builtin_amdgcn_readlane(keys, o) + (r0 + o < tid ? 1 : 0) > key ? 1 : 0;
                 }
+                if (tid < a.n_rows) s_order[rank] = (uint16_t)tid;
             }
-            s_order[rank] = (uint16_t)r;
+        } else {      // (larger launches keep the rows' order: ranking them costs more than it returns)
+            for (int r = tid; r < a.n_rows; r += 256) s_order[r] = (uint16_t)r;
         }
         lds_barrier();
     }
@@ -323,27 +334,25 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
         bool last = false;      // dense list: the row's last partition
         if (dense) {
             if (unit < phase1) {
-                const int q = (int)(unit / per_row);      // the q-th of all rows' partitions but their last
-                bx = (int)(unit % per_row);
-                int lo = 0, hi = a.n_rows;                // the row: s_before[r] <= q < s_before[r + 1]
-                while (hi - lo > 1) {
-                    const int mid = (lo + hi) >> 1;
-                    if (__builtin_amdgcn_readfirstlane(s_before[mid]) <= q) lo = mid;
-                    else hi = mid;
-                }
-                r = lo, b = q - __builtin_amdgcn_readfirstlane(s_before[lo]);
+                const int q = (int)div32(a.row_div, unit);      // the q-th of all rows' partitions but their last
+                bx = (int)(unit - (unsigned)q * per_row);
+                int n = 0;      // the row: the last with s_before[r] <= q (64 rows a look)
+                for (int r0 = 0; r0 < a.n_rows; r0 += 64)
+                    n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(r0 + lane < a.n_rows && s_before[min(r0 + lane, kLdsRows)] <= q));
+                r = n - 1, b = q - __builtin_amdgcn_readfirstlane(s_before[r]);
             } else {
                 const unsigned rest = unit - phase1;
-                r = __builtin_amdgcn_readfirstlane(s_order[rest / per_row]), bx = (int)(rest % per_row), b = 0, last = true;
+                const unsigned at = div32(a.row_div, rest);
+                r = __builtin_amdgcn_readfirstlane(s_order[at]), bx = (int)(rest - at * per_row), b = 0, last = true;
             }
         } else {
             bx = (int)(unit % (unsigned)a.units_x);
             b = (int)(unit / (unsigned)a.units_x);
-            r = bx / (int)per_row;
-            bx %= (int)per_row;
+            r = (int)div32(a.row_div, (uint32_t)bx);
+            bx -= r * (int)per_row;
         }
-        const int tile = bx % a.tiles;
-        un.kvh0 = (bx / a.tiles) * HW;      // the first of the wavefronts' KV heads
+        const int tiles_before = (int)div32(a.tiles_div, (uint32_t)bx), tile = bx - tiles_before * a.tiles;
+        un.kvh0 = tiles_before * HW;      // the first of the wavefronts' KV heads
         int d[5];
         if (r < kLdsRows) {
 #pragma unroll
@@ -357,10 +366,10 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
         un.trow = (int64_t)d[2] * a.tab_stride;
         un.j0 = tile * (QT * CPH);           // the first row of the unit's tiles in the flattened (column, group head) list
         if (un.j0 >= un.count * a.g) return un;
-        un.c_lo = un.j0 / a.g;
-        const int c_hi = min(un.count, (un.j0 + QT * CPH - 1) / a.g + 1);
+        un.c_lo = by_group(un.j0);
+        const int c_hi = min(un.count, by_group(un.j0 + QT * CPH - 1) + 1);
         un.n_keys = min(un.first + c_hi, a.max_keys);
-        un.n_pieces = (un.n_keys + a.piece - 1) / a.piece;
+        un.n_pieces = pieces_of(un.n_keys);
         if constexpr (!FUSED) {
             // Units are taken in list order, y slowest, and a launch's tail is as long as its last units: the row's
             // last partition (usually a partial piece, the smallest unit of work) is listed after every other
@@ -446,7 +455,7 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
         Steps s;
         s.from = from, s.first_piece = first_piece;
         const int n = from + (lane >> 1), r = lane & 1;
-        const int turns = n / max(pairs_a_piece, 1), k = n - turns * pairs_a_piece;
+        const int turns = n < pairs_a_piece ? 0 : n / max(pairs_a_piece, 1), k = n - turns * pairs_a_piece;
         const int piece = first_piece + turns * a.parts;
         const int st = wave + 8 * k;
         const bool there = pairs_a_piece > 0 && piece < un.n_pieces;
@@ -504,7 +513,8 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
     // NARROW: whether this lane's tile column (a query row of the flattened list) belongs to the pair's odd KV head.
     auto odd_of = [&](const Unit& un) __attribute__((always_inline)) -> int {
         if constexpr (!NARROW) return 0;
-        return ((un.j0 + c16 % CPH) % a.g) >= (a.g >> 1) ? 1 : 0;
+        const int j = un.j0 + c16 % CPH;
+        return j - by_group(j) * a.g >= (a.g >> 1) ? 1 : 0;
     };
     auto fetch_v = [&](const Unit& un, uint32_t slot0, int i) __attribute__((always_inline)) {
         const uint8_t* sbase = a.vp + (int64_t)slot0 * slot_bytes + un.kvh0 * ROWB;
@@ -548,9 +558,9 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
 #pragma unroll
         for (int q = 0; q < QT; ++q) {
             const int jr = un.j0 + q * CPH + c16 % CPH;
-            col[q] = jr / a.g;
+            col[q] = by_group(jr);
             const bool live = col[q] < un.count;
-            const int qhead = (un.kvh0 + hsel) * a.g + jr % a.g;
+            const int qhead = (un.kvh0 + hsel) * a.g + jr - col[q] * a.g;
             lim[q] = live ? min(un.first + col[q], un.n_keys - 1) : -1;
             anc[q] = (tree && live) ? ancestors(a, un.start, col[q]) : 0ull;
             const uint8_t* row = a.q + ((int64_t)(un.start + col[q]) * a.q_st + (int64_t)qhead * a.q_sh) * 2;
@@ -886,7 +896,7 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
                     const int cc = tid >> 4, g0 = tid & 15;
                     const int head_i = cc / CPH;
                     const int j = fold_col_j0 + q * CPH + cc % CPH;
-                    const int c = j / a.g, in_group = j - c * a.g;
+                    const int c = by_group(j), in_group = j - c * a.g;
                     const int odd = NARROW ? (in_group >= (a.g >> 1) ? 1 : 0) : 0;      // NARROW: the 64 dims of the column's own KV head are kept
                     float M = 0.0f, L = 0.0f, fw[4];
                     float vm = 1.0f;
@@ -896,7 +906,7 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
                     }
                     Fold fo = {};
                     // A column folds the partitions that hold its positions, as the merge does.
-                    const int held = FUSED ? min(a.parts, (min(cur.first + c + 1, a.max_keys) + a.piece - 1) / a.piece) : 0;
+                    const int held = FUSED ? min(a.parts, pieces_of(min(cur.first + c + 1, a.max_keys))) : 0;
                     auto group = [&](int w, int col_, int g) __attribute__((always_inline)) -> f32x4* { return reinterpret_cast<f32x4*>(&s_acc[w][col_][4 * (g ^ col_)]); };
 #pragma unroll
                     for (int sl = 0; sl < D / FW; ++sl) {
@@ -972,7 +982,7 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
             if constexpr (FUSED) {
                 const int cc = tid >> 4, d0 = 4 * (tid & 15);
                 const int j = cur.j0 + cc % CPH;
-                const int c = j / a.g, in_group = j - c * a.g;
+                const int c = by_group(j), in_group = j - c * a.g;
                 const int odd = NARROW ? (in_group >= (a.g >> 1) ? 1 : 0) : 0;
                 if (c < cur.count) {
                     const int head = (cur.kvh0 + cc / CPH) * a.g + in_group;
@@ -1000,10 +1010,13 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
         // The unit after the next: the ticket drawn above, or, while it names a unit without work, the ones after it.
         unsigned u_after = u_next + grid;
         if (pulled) {
-            if (tid == 0) {
-                unsigned found = 2 * grid + drawn;
-                while (found < total && !decode(found).valid) found = 2 * grid + atomicAdd(a.ticket, 1u);
-                s_unit = found;
+            if (wave == 0) {      // (the whole wavefront: decode() looks at 64 rows at once)
+                unsigned found = 2 * grid + (unsigned)__builtin_amdgcn_readfirstlane((int)drawn);
+                while (found < total && !decode(found).valid) {
+                    if (lane == 0) drawn = atomicAdd(a.ticket, 1u);
+                    found = 2 * grid + (unsigned)__builtin_amdgcn_readfirstlane((int)drawn);
+                }
+                if (lane == 0) s_unit = found;
             }
             lds_barrier();      // (and every thread is done with the fold's shared arrays)
             u_after = (unsigned)__builtin_amdgcn_readfirstlane((int)s_unit);
