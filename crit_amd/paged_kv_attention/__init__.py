@@ -172,7 +172,7 @@ def _launch_state(device, stream):
     a replaying graph never meets an eager launch or another graph in its counters, whatever streams they run on.
     The pairs come from a zeroed block the owner holds; a launch leaves its pair zero."""
     holding = _holding(device)
-    capture = _abi.capture_id(stream)
+    capture = _capture_of(device, stream)
     if not capture and (holding.counters is None or holding.pairs_used > COUNTER_PAIRS - COUNTER_HEADROOM):
         # An eager launch tops the block up while there is still room for the captures that may follow it: a block is
         # zeroed memory, which a capture cannot allocate. The pairs handed out stay where they are (`kept`).
@@ -198,6 +198,16 @@ def _ptr(t):
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)      # (the stream's handle without a Stream object)
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)      # (without the check that CUDA is up)
+_capturing = getattr(torch._C, "_cuda_isCurrentStreamCapturing", lambda: True)
+
+
+def _capture_of(device, stream):
+    """The id of the capture `stream`, the caller's current one on `device`, records into; 0 outside a capture (asked of
+    torch first, which answers for the current device's stream in a tenth of the library call's time)."""
+    if (device.index is None or device.index == _current_device()) and not _capturing():
+        return 0
+    return _abi.capture_id(stream)
 
 
 def _stream_of(device):
@@ -213,7 +223,7 @@ def _launch(device, name, what, *args, stream=None):
     entry = getattr(_abi.load(), name)
     if stream is None:
         stream = _stream_of(device)
-    if device.index is None or device.index == torch.cuda.current_device():
+    if device.index is None or device.index == _current_device():
         code = entry(*args, stream)
     else:
         with torch.cuda.device(device):
@@ -349,8 +359,9 @@ def workspace_floats(tokens, heads, partitions, value_dim):
 
 
 def _workspace(device, tokens, heads, parts, dv, given=None):
-    """(partial outputs, maxima, sums) of a split launch: three views of the caller's FP32 workspace, or of the one the
-    current owner holds on the device."""
+    """The addresses of a split launch's partial outputs, maxima and sums, one behind another in the caller's FP32
+    workspace, or in the one the current owner holds on the device. (Addresses: three views of the workspace were a fifth
+    of a small launch's time on the host.)"""
     states = tokens * heads * parts
     floats = states * (dv + 2)
     if given is None:
@@ -359,8 +370,8 @@ def _workspace(device, tokens, heads, parts, dv, given=None):
     elif given.dtype != torch.float32 or not given.is_contiguous() or given.numel() < floats:
         raise ValueError(f"workspace: {floats} contiguous FP32 floats for this launch (workspace_floats()), "
                          f"{given.numel()} given")
-    outs, rest = given[:states * dv], given[states * dv:]
-    return outs, rest[:states], rest[states:2 * states]
+    base = given.data_ptr()
+    return base, base + 4 * states * dv, base + 4 * states * (dv + 1)
 
 
 # -- writes ----------------------------------------------------------------------------------------------------------------
@@ -403,13 +414,18 @@ def write(keys, values, slots, key_pages, value_pages, kind, key_scales=None, va
         return write(None, values, slots, None, value_pages, kind, None, value_scales, multipliers=multipliers)
     if keys.dtype not in _DTYPE:
         keys = keys.float()
-    if keys.stride(-1) != 1:
+    k_step = keys.stride()
+    if k_step[-1] != 1:
         keys = keys.contiguous()
+        k_step = keys.stride()
+    v_step = (0, 0)
     if values is not None:
         if values.dtype != keys.dtype:
             values = values.to(keys.dtype)
-        if values.stride(-1) != 1:
+        v_step = values.stride()
+        if v_step[-1] != 1:
             values = values.contiguous()
+            v_step = values.stride()
         if value_pages is None or (k_kind >= 2 and value_scales is None):
             raise ValueError("values come with their pages (and their scales for fp8:row and int8)")
     if slots.dtype != torch.int64 or not slots.is_contiguous():
@@ -417,19 +433,12 @@ def write(keys, values, slots, key_pages, value_pages, kind, key_scales=None, va
     if not key_pages.is_contiguous() or (value_pages is not None and not value_pages.is_contiguous()):
         raise ValueError("a layer's pages are contiguous ([slots][kv_heads][dim] storage)")
     km, vm, per_head = _multipliers(multipliers, hkv, keys.device)
-    p = _abi.WriteParams()
-    p.keys, p.values, p.slots = keys.data_ptr(), _ptr(values), slots.data_ptr()
-    p.key_pages, p.value_pages = key_pages.data_ptr(), _ptr(value_pages)
-    p.key_scales, p.value_scales = _ptr(key_scales), _ptr(value_scales)
-    p.head_multipliers = _ptr(per_head)
-    p.tokens = T
-    p.key_stride_t, p.key_stride_h = keys.stride(0), keys.stride(1)
-    if values is not None:
-        p.value_stride_t, p.value_stride_h = values.stride(0), values.stride(1)
-    p.kv_heads, p.head_dim = hkv, d
-    p.value_dim = values.shape[-1] if values is not None else 0
-    p.kind, p.page_dtype, p.in_dtype = k_kind, _page_dtype(key_pages, kind), _DTYPE[keys.dtype]
-    p.key_multiplier, p.value_multiplier = km, vm
+    # (the fields in the structure's order: one call instead of a Python assignment each)
+    p = _abi.WriteParams(keys.data_ptr(), _ptr(values), slots.data_ptr(), key_pages.data_ptr(), _ptr(value_pages),
+                         _ptr(key_scales), _ptr(value_scales), _ptr(per_head),
+                         T, k_step[0], k_step[1], v_step[0], v_step[1],
+                         hkv, d, 0 if values is None else values.shape[-1], k_kind, _page_dtype(key_pages, kind),
+                         _DTYPE[keys.dtype], km, vm)
     if rope is not None:
         if not 2 <= len(rope) <= 4:
             raise ValueError("rope is (table, positions), with a style and a scale if not half and 1")
@@ -600,7 +609,8 @@ def attend(q, key_pages, value_pages, kind, tables, rows, starts, firsts, column
     R = int(starts.shape[0])
     if hq % hkv or not 1 <= columns <= MAX_COLUMNS or R == 0:
         raise ValueError("query heads a multiple of the KV heads, 1..64 columns a row, one row or more")
-    if q.stride(-1) != 1:
+    q_step = q.stride()      # (a tensor's strides are asked for once: a question is a quarter of a microsecond)
+    if q_step[-1] != 1:
         raise ValueError("q's last dimension is contiguous")
     if d not in HEAD_WIDTHS or dv not in HEAD_WIDTHS or key_pages.shape[-1] != d:
         raise ValueError(f"head widths are powers of two from 16 to 256 (q's, keys' and values'), not {d} and {dv}")
@@ -609,7 +619,8 @@ def attend(q, key_pages, value_pages, kind, tables, rows, starts, firsts, column
         raise ValueError(f"q is {want_q} over {kind} pages, not {q.dtype}")
     if (offsets is None) != (tokens is None):
         raise ValueError("offsets come with the partial rows they take (tokens)")
-    if tables.dtype != torch.int32 or tables.stride(-1) != 1 or rows.dtype not in (torch.int32, torch.int64) or \
+    table_step, rows_dtype = tables.stride(), rows.dtype
+    if tables.dtype != torch.int32 or table_step[-1] != 1 or rows_dtype not in (torch.int32, torch.int64) or \
             starts.dtype != torch.int32 or firsts.dtype != torch.int64:
         raise ValueError("tables and starts are int32, rows int32 or int64 and firsts int64")
     if counts is not None and counts.dtype != torch.int32 or offsets is not None and offsets.dtype != torch.int32:
@@ -639,36 +650,34 @@ def attend(q, key_pages, value_pages, kind, tables, rows, starts, firsts, column
         po, pm, pl = _workspace(device, partial_rows, hq, parts, dv, workspace)
     if out is None:
         out = torch.empty(T, hq, dv, dtype=q.dtype, device=device)
-    if out.dtype not in _DTYPE or out.stride(-1) != 1 or out.shape[-1] != dv:
+    out_dtype, out_step = _DTYPE.get(out.dtype), out.stride()
+    if out_dtype is None or out_step[-1] != 1 or out.shape[-1] != dv:
         raise ValueError("out is [tokens][heads][value_dim] BF16, FP16 or FP32, its last dimension contiguous")
     if lse is not None and (lse.dtype != torch.float32 or not lse.is_contiguous()):
         raise ValueError("lse is contiguous FP32 [tokens][heads]")
     km, vm, per_head = _multipliers(multipliers, hkv, device)
-    p = _abi.AttendParams()
-    p.q, p.key_pages, p.value_pages = q.data_ptr(), key_pages.data_ptr(), value_pages.data_ptr()
-    p.key_scales, p.value_scales, p.head_multipliers = _ptr(key_scales), _ptr(value_scales), _ptr(per_head)
+    parents32 = parents is not None and parents.dtype == torch.int32
+    # (the fields in the structure's order: one call instead of a Python assignment each)
+    p = _abi.AttendParams(q.data_ptr(), key_pages.data_ptr(), value_pages.data_ptr(), _ptr(key_scales), _ptr(value_scales),
+                          _ptr(per_head), tables.data_ptr(), rows.data_ptr(), starts.data_ptr(), _ptr(counts),
+                          firsts.data_ptr(), _ptr(offsets), po, pm, pl, out.data_ptr(), _ptr(lse), _ptr(sinks),
+                          parents.data_ptr() if parents32 else None, None if parents is None or parents32 else parents.data_ptr(),
+                          _ptr(blocks), q_step[0], q_step[1], out_step[0], out_step[1], table_step[0],
+                          0 if blocks is None else blocks.stride(0),
+                          tables.shape[1], R, int(columns), hq, hkv, d, dv, int(page), k_kind, _page_dtype(key_pages, kind),
+                          out_dtype, parts, piece, int(bool(fused)), sliding, int(phases),
+                          0 if blocks is None else int(blocks.shape[1]), 0 if blocks is None else int(block_size),
+                          scale, km, vm)
     if derived is not None:
         p.key_pages = p.key_scales = None
         p.derive_table, p.derive_eps = derived.table.data_ptr(), derived.eps
         p.derive_rot, p.derive_weighted = derived.rotary_dim, int(has_weight)
-    p.tables, p.rows, p.starts, p.counts = tables.data_ptr(), rows.data_ptr(), starts.data_ptr(), _ptr(counts)
-    p.rows_are_64 = int(rows.dtype == torch.int64)
-    p.firsts, p.offsets = firsts.data_ptr(), _ptr(offsets)
-    p.partial_out, p.partial_max, p.partial_sum = _ptr(po), _ptr(pm), _ptr(pl)
-    p.out, p.lse, p.sinks = out.data_ptr(), _ptr(lse), _ptr(sinks)
-    if parents is not None:
-        p.parents, p.parents64 = (parents.data_ptr(), None) if parents.dtype == torch.int32 else (None, parents.data_ptr())
-    if blocks is not None:
-        p.blocks, p.blocks_stride = blocks.data_ptr(), blocks.stride(0)
-        p.blocks_k, p.block_size = int(blocks.shape[1]), int(block_size)
-    p.q_stride_t, p.q_stride_h, p.out_stride_t, p.out_stride_h = q.stride(0), q.stride(1), out.stride(0), out.stride(1)
-    p.table_stride, p.table_width = tables.stride(0), tables.shape[1]
-    p.n_rows, p.columns, p.heads, p.kv_heads, p.head_dim, p.value_dim, p.page = R, int(columns), hq, hkv, d, dv, int(page)
-    p.kind, p.page_dtype, p.out_dtype = k_kind, _page_dtype(key_pages, kind), _DTYPE[out.dtype]
-    p.partitions, p.piece, p.fused, p.sliding, p.phases = parts, piece, int(bool(fused)), sliding, int(phases)
-    p.scale, p.key_multiplier, p.value_multiplier = scale, km, vm
-    p.int8_qk = int(bool(int8_qk))
-    p.window_tokens = 0 if offsets is None else int(tokens)
+    if rows_dtype == torch.int64:
+        p.rows_are_64 = 1
+    if int8_qk:
+        p.int8_qk = 1
+    if offsets is not None:
+        p.window_tokens = int(tokens)
     if fresh is not None:
         fk, fv, fshift, ffirst = fresh
         if derive is not None:      # (checked as the keys the values stand for: one width)

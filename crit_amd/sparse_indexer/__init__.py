@@ -26,7 +26,7 @@ from typing import Optional
 import torch
 
 from ..paged_kv_attention import _abi
-from ..paged_kv_attention import _launch, _ptr, _require_device
+from ..paged_kv_attention import _current_device, _launch, _ptr, _require_device
 
 __all__ = ["scores", "select", "topk"]
 
@@ -120,20 +120,24 @@ def scores(q, keys, weights, ends, *, key_scales=None, scale=None, out: Optional
             scores(q[first:last], keys, weights[first:last], ends[first:last], key_scales=key_scales, scale=scale,
                    out=out[first:last], slots=these)
         return out
-    p = _abi.IndexScoresParams()
-    p.q, p.keys, p.weights, p.ends, p.out = (x.data_ptr() for x in (q, keys, weights, ends, out))
-    p.key_scales = _ptr(key_scales) if coded else None
-    p.slots = _ptr(slots)
-    p.q_stride_t, p.q_stride_h = q.stride(0), q.stride(1)
-    p.key_stride, p.weights_stride, p.out_stride = keys.stride(0), weights.stride(0), out.stride(0)
-    p.slots_stride = slots.stride(0) if slots is not None and slots.dim() == 2 else 0
-    p.tokens, p.n, p.group, p.heads, p.dim = tokens, n, group, heads, dim
-    p.key_dtype = 2 if coded else int(keys.dtype == torch.float16)
-    p.q_dtype = _abi.F16 if q.dtype == torch.float16 else _abi.BF16
-    p.slots_are_64 = int(slots is not None and slots.dtype == torch.int64)
-    p.scale = float(dim ** -0.5 if scale is None else scale)
-    _launch(q.device, "crit_pkv_index_scores", "sparse_indexer.scores", p)
+    _score(q, keys, weights, ends, key_scales if coded else None, scale, out.data_ptr(), out.stride(0), slots, n, group)
     return out
+
+
+def _score(q, keys, weights, ends, key_scales, scale, out, out_stride, slots, n, group):
+    """The launch of checked operands' scores into the FP32 rows at address `out`."""
+    tokens, heads, dim = q.shape
+    q_step = q.stride()
+    # (the fields in the structure's order)
+    p = _abi.IndexScoresParams(q.data_ptr(), keys.data_ptr(), _ptr(key_scales), weights.data_ptr(), ends.data_ptr(), _ptr(slots), out,
+                               q_step[0], q_step[1], keys.stride(0), weights.stride(0), out_stride,
+                               slots.stride(0) if slots is not None and slots.dim() == 2 else 0,
+                               tokens, n, group, heads, dim,
+                               2 if key_scales is not None else int(keys.dtype == torch.float16),
+                               _abi.F16 if q.dtype == torch.float16 else _abi.BF16,
+                               int(slots is not None and slots.dtype == torch.int64),
+                               float(dim ** -0.5 if scale is None else scale))
+    _launch(q.device, "crit_pkv_index_scores", "sparse_indexer.scores", p)
 
 
 def topk(s, ends, k, *, out: Optional[torch.Tensor] = None):
@@ -150,17 +154,24 @@ def topk(s, ends, k, *, out: Optional[torch.Tensor] = None):
     out = _picks_buffer(out, tokens, k, s.device)
     if tokens == 0:
         return out
-    # A long row is selected in slices whose candidates go through a buffer; the library says how large.
-    with torch.cuda.device(s.device):
-        room = int(_abi.load().crit_pkv_index_topk_work_bytes(tokens, n, k))
+    room = _candidates(s.device, tokens, n, k)
     work = torch.empty(room // 4, dtype=torch.int32, device=s.device) if room else None
-    p = _abi.IndexTopkParams()
-    p.scores, p.ends, p.out = s.data_ptr(), ends.data_ptr(), out.data_ptr()
-    p.work, p.work_bytes = _ptr(work), room
-    p.scores_stride, p.out_stride = s.stride(0), out.stride(0)
-    p.tokens, p.n, p.k = tokens, n, k
-    _launch(s.device, "crit_pkv_index_topk", "sparse_indexer.topk", p)
+    _pick(s.device, s.data_ptr(), s.stride(0), ends, out, _ptr(work), room, tokens, n, k)
     return out
+
+
+def _candidates(device, tokens, n, k):
+    """Bytes of the buffer a long row's selection takes: it goes in slices whose candidates pass through memory."""
+    if device.index is None or device.index == _current_device():
+        return int(_abi.load().crit_pkv_index_topk_work_bytes(tokens, n, k))
+    with torch.cuda.device(device):
+        return int(_abi.load().crit_pkv_index_topk_work_bytes(tokens, n, k))
+
+
+def _pick(device, scores_at, scores_stride, ends, out, work_at, room, tokens, n, k):
+    """The launch of checked operands' picks from the FP32 rows at address `scores_at`."""
+    p = _abi.IndexTopkParams(scores_at, ends.data_ptr(), out.data_ptr(), work_at, scores_stride, out.stride(0), room, tokens, n, k)
+    _launch(device, "crit_pkv_index_topk", "sparse_indexer.topk", p)
 
 
 def select(q, keys, weights, ends, k, *, key_scales=None, scale=None, out: Optional[torch.Tensor] = None,
@@ -168,7 +179,7 @@ def select(q, keys, weights, ends, k, *, key_scales=None, scale=None, out: Optio
     """topk(scores(...), ends, k) without ever holding the whole score matrix: tokens are taken in batches whose scores
     fit `workspace` (FP32, any shape; by default a fresh buffer of at most workspace_bytes). The picks are those of the
     two calls made separately. `slots` here is one list [n] for every token."""
-    tokens, _, _, _ = _score_operands(q, keys, weights, ends, key_scales)
+    tokens, _, _, coded = _score_operands(q, keys, weights, ends, key_scales)
     if slots is not None and slots.dim() != 1:
         raise ValueError("slots: select takes one list [n]; per-group lists [groups][n] are for scores()")
     n = keys.shape[0] if slots is None else slots.shape[0]
@@ -177,6 +188,17 @@ def select(q, keys, weights, ends, k, *, key_scales=None, scale=None, out: Optio
         return out
     if n == 0:
         out.fill_(-1)
+        return out
+    if workspace is None and tokens <= min((workspace_bytes // 4) // n, _LAUNCH_TOKENS) and int(k) >= 1:
+        # One batch, checked already: the scores and the candidates in one buffer of this call's, two launches.
+        if slots is not None:
+            _slot_groups(slots, tokens)
+        k = int(k)
+        device, room = q.device, _candidates(q.device, tokens, n, k)
+        held = torch.empty((tokens * n + 3) // 4 * 4 + room // 4, dtype=torch.float32, device=device)
+        at = held.data_ptr()
+        _score(q, keys, weights, ends, key_scales if coded else None, scale, at, n, slots, n, tokens)
+        _pick(device, at, n, ends, out, at + (tokens * n + 3) // 4 * 16 if room else None, room, tokens, n, k)
         return out
     if workspace is None:
         batch = min(tokens, max(1, (workspace_bytes // 4) // n))
