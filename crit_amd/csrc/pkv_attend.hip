@@ -18,7 +18,9 @@ int launch_attend_int8(const AttendArgs& a, int lpr, int qr, bool fused, bool pa
 // Lane `at`'s value of x (at: the same in every lane).
 PKV_DEV float lane_value(float x, int at) { return u2f((uint32_t)__builtin_amdgcn_readlane((int)f2u(x), at)); }
 
-template <int DV>
+// MANY: launches of more wavefronts than the card holds at once of the other form, whose batches of 32 partitions take 160
+// registers: batches of 8, three times the wavefronts (10,240 of up to 17 partitions: 18.7 -> 13.3 us).
+template <int DV, bool MANY>
 __global__ __launch_bounds__(64) void merge_kernel(AttendArgs a) {
     constexpr int EPL = DV < 64 ? 1 : DV / 64;      // (value rows narrower than a wavefront: the lanes past them idle)
     const int c = blockIdx.x, head = blockIdx.y, r = blockIdx.z;
@@ -64,7 +66,7 @@ __global__ __launch_bounds__(64) void merge_kernel(AttendArgs a) {
         // (exact in any order), then keep, take and l * take a lane each. What stays in order is one fused
         // multiply-add for the sum and one multiply and one fused multiply-add a value dim, their factors read from
         // the lane that holds them. The next batch's states are loaded while this one is folded.
-        constexpr int U = EPL > 2 ? 16 : 32;
+        constexpr int U = MANY ? 8 : EPL > 2 ? 16 : 32;
         float po[2][U][EPL], pm_next, pl_next;
         auto load_scalars = [&](int b0) __attribute__((always_inline)) {
             const int b = min(b0 + ((int)threadIdx.x & (U - 1)), nb - 1);      // (the thread's own place: `lane` is clamped to the value row)
@@ -134,6 +136,81 @@ __global__ __launch_bounds__(64) void merge_kernel(AttendArgs a) {
         if (DV >= 64 || (int)threadIdx.x < DV) store_out(a.out, a.out_dtype, token * a.o_st + (int64_t)head * a.o_sh + e * 64 + lane, o);
     }
     if (a.lse && threadIdx.x == 0) a.lse[token * a.hq + head] = L != 0.0f ? __builtin_fmaf(M, kLn2, __logf(L)) : -INFINITY;
+}
+
+// The same fold for few (column, head, row) triples of many partitions (long rows): a workgroup each. One wavefront would
+// fetch its partials a batch after another, at a round trip to memory a batch (200,000 positions in splits of 1,024, 40
+// heads: 15.3 us in 40 wavefronts, 10.7 here). Here 256 threads bring up to a hundred kilobytes of them into LDS at once,
+// make every partition's factors (a prefix maximum over the threads, exact in any order), and a thread a value dim folds
+// them in order: the operations of merge_kernel on the same values.
+template <int DV>
+__global__ __launch_bounds__(256) void merge_long_kernel(AttendArgs a) {
+    typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));      // (four floats of a workspace that is any floats)
+    constexpr int CH = DV == 256 ? 128 : 256;      // partitions at a time
+    __shared__ __align__(16) float s_val[CH * DV];
+    __shared__ __align__(16) float4 s_factor[CH];     // keep, take, l * take
+    __shared__ float s_top[4];
+    const int c = blockIdx.x, head = blockIdx.y, r = blockIdx.z;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    int count = a.columns;
+    if (a.counts) count = min(a.counts[r], a.columns);
+    if (c >= count) return;
+    int64_t first = a.firsts[r];
+    first = first < 0 ? 0 : (first > (int64_t)0x3fffffff ? (int64_t)0x3fffffff : first);
+    const int64_t seen = min(first + c + 1, (int64_t)a.max_keys);
+    const uint32_t run = a.blocks ? (uint32_t)a.listed_keys : (uint32_t)seen;
+    const int nb = (int)min((uint32_t)a.parts, (run + (uint32_t)a.piece - 1u) / (uint32_t)a.piece);
+    const int64_t prow = a.offsets ? (int64_t)(a.offsets[r] - a.offsets[0]) : (int64_t)r * a.columns;
+    const int64_t at = ((prow + c) * a.hq + head) * a.parts;
+    float M = -INFINITY, L = 0.0f, A = 0.0f;
+    for (int b0 = 0; b0 < nb; b0 += CH) {
+        const int n = min(CH, nb - b0);
+        const float* src = a.po + (at + b0) * DV;      // (a triple's partials lie side by side)
+        const int vecs = n * (DV / 4);
+        for (int v0 = 0; v0 < vecs; v0 += 256 * 16) {
+            f32x4_any x[16];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) x[k] = *reinterpret_cast<const f32x4_any*>(src + 4 * min(v0 + 256 * k + tid, vecs - 1));
+#pragma unroll
+            for (int k = 0; k < 16; ++k)
+                if (v0 + 256 * k + tid < vecs) *reinterpret_cast<f32x4*>(&s_val[4 * (v0 + 256 * k + tid)]) = x[k];
+        }
+        float pm = -INFINITY, pl = 0.0f;
+        if (tid < n) pm = a.pm[at + b0 + tid], pl = a.pl[at + b0 + tid];
+        float upto = pm;      // the maximum of the wavefront's partitions up to this one
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const float other = __shfl_up(upto, o);
+            if (lane >= o) upto = __builtin_fmaxf(upto, other);
+        }
+        if (lane == 63) s_top[wave] = upto;
+        __syncthreads();
+        float before = M;     // the maximum of every partition before the wavefront's first
+        for (int w = 0; w < wave; ++w) before = __builtin_fmaxf(before, s_top[w]);
+        const float m_new = __builtin_fmaxf(before, upto);
+        float m_old = __shfl_up(m_new, 1);
+        if (lane == 0) m_old = before;
+        const float sub = m_new == -INFINITY ? 0.0f : m_new;
+        const float keep = exp2_fast(m_old - sub), take = exp2_fast(pm - sub);
+        if (tid < n) s_factor[tid] = make_float4(keep, take, pl * take, 0.0f);
+        for (int w = 0; w < 4; ++w) M = __builtin_fmaxf(M, s_top[w]);
+        __syncthreads();
+#pragma unroll 8
+        for (int i = 0; i < n; ++i) {
+            const float4 f = s_factor[i];
+            L = __builtin_fmaf(L, f.x, f.z);
+            A = __builtin_fmaf(A, f.x, s_val[i * DV + (tid & (DV - 1))] * f.y);
+        }
+        __syncthreads();      // (the next partitions go where these were)
+    }
+    if (a.sinks) {
+        const Fold f = fold(M, L, a.sinks[head] * kLog2e, 1.0f);
+        A *= f.keep;
+        M = f.m, L = f.l;
+    }
+    const int64_t token = a.starts[r] + c;
+    if (tid < DV) store_out(a.out, a.out_dtype, token * a.o_st + (int64_t)head * a.o_sh + tid, L != 0.0f ? A / L : 0.0f);
+    if (a.lse && tid == 0) a.lse[token * a.hq + head] = L != 0.0f ? __builtin_fmaf(M, kLn2, __logf(L)) : -INFINITY;
 }
 
 // Shard merge: outs [parts][rows][DV], lses [parts][rows] (natural log) -> out FP32, lse; one wavefront per row.
@@ -407,13 +484,28 @@ static int launch_attend_checked(const crit_pkv_attend_params* p, hipStream_t st
     if (p->phases != 2) rc = split(false);
     if (rc || p->phases == 1) return rc;
     const dim3 mgrid((unsigned)p->columns, (unsigned)p->heads, (unsigned)p->n_rows);
-    switch (p->value_dim) {
-        case 16: hipLaunchKernelGGL((merge_kernel<16>), mgrid, dim3(64), 0, stream, a); break;
-        case 32: hipLaunchKernelGGL((merge_kernel<32>), mgrid, dim3(64), 0, stream, a); break;
-        case 64: hipLaunchKernelGGL((merge_kernel<64>), mgrid, dim3(64), 0, stream, a); break;
-        case 128: hipLaunchKernelGGL((merge_kernel<128>), mgrid, dim3(64), 0, stream, a); break;
-        case 256: hipLaunchKernelGGL((merge_kernel<256>), mgrid, dim3(64), 0, stream, a); break;
+    // Which merge: by the wavefronts of the launch and the partitions a row may have (the bits are the same). Up to a
+    // triple a compute unit of more than 32 partitions, a workgroup each; more than 8 wavefronts a compute unit (what the card
+    // holds of the form with batches of 32), batches of 8.
+    const int64_t triples = (int64_t)p->columns * p->heads * p->n_rows, units = compute_units();
+    const bool long_rows = triples <= units && gy > 32, many = triples > 8 * units;
+#define PKV_MERGE(W)                                                                                                        \
+    case W:                                                                                                                 \
+        if (many) hipLaunchKernelGGL((merge_kernel<W, true>), mgrid, dim3(64), 0, stream, a);                               \
+        else hipLaunchKernelGGL((merge_kernel<W, false>), mgrid, dim3(64), 0, stream, a);                                   \
+        break;
+    if (long_rows && p->value_dim >= 64) {
+        switch (p->value_dim) {
+            case 64: hipLaunchKernelGGL((merge_long_kernel<64>), mgrid, dim3(256), 0, stream, a); break;
+            case 128: hipLaunchKernelGGL((merge_long_kernel<128>), mgrid, dim3(256), 0, stream, a); break;
+            case 256: hipLaunchKernelGGL((merge_long_kernel<256>), mgrid, dim3(256), 0, stream, a); break;
+        }
+        return hip_code(hipGetLastError());
     }
+    switch (p->value_dim) {
+        PKV_MERGE(16) PKV_MERGE(32) PKV_MERGE(64) PKV_MERGE(128) PKV_MERGE(256)
+    }
+#undef PKV_MERGE
     return hip_code(hipGetLastError());
 }
 
