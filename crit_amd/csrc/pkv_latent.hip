@@ -465,7 +465,10 @@ __global__ __launch_bounds__(256, 1) void latent_heads_kernel(LatentArgs a) {
     int b, r;
     if (a.n_rows >= kRowsToAnXcd) {
         const int64_t pair = place / a.tiles;
-        b = (int)(pair % a.gy), r = (int)(pair / a.gy) * 8 + (int)(blockIdx.x & 7);
+        // (every second round of rows is dealt in the opposite order: the rows come longest first, and the same XCD would
+        // take the longest of every eight)
+        const int round = (int)(pair / a.gy), xcd = (int)(blockIdx.x & 7);
+        b = (int)(pair % a.gy), r = round * 8 + (round & 1 ? 7 - xcd : xcd);
         if (r >= a.n_rows) return;
     } else {
         const int64_t pair = (place / a.tiles) * 8 + (int64_t)(blockIdx.x & 7);
