@@ -18,7 +18,7 @@ int launch_attend_int8(const AttendArgs& a, int lpr, int qr, bool fused, bool pa
 // Lane `at`'s value of x (at: the same in every lane).
 PKV_DEV float lane_value(float x, int at) { return u2f((uint32_t)__builtin_amdgcn_readlane((int)f2u(x), at)); }
 
-// MANY: launches of more wavefronts than the card holds at once of the other form, whose batches of 32 partitions take 160
+// MANY: launches of as many wavefronts as the card holds at once of the other form, or more, whose batches of 32 partitions take 160
 // registers: batches of 8, three times the wavefronts (10,240 of up to 17 partitions: 18.7 -> 13.3 us).
 template <int DV, bool MANY>
 __global__ __launch_bounds__(64) void merge_kernel(AttendArgs a) {
@@ -485,10 +485,10 @@ static int launch_attend_checked(const crit_pkv_attend_params* p, hipStream_t st
     if (rc || p->phases == 1) return rc;
     const dim3 mgrid((unsigned)p->columns, (unsigned)p->heads, (unsigned)p->n_rows);
     // Which merge: by the wavefronts of the launch and the partitions a row may have (the bits are the same). Up to a
-    // triple a compute unit of more than 32 partitions, a workgroup each; more than 8 wavefronts a compute unit (what the card
-    // holds of the form with batches of 32), batches of 8.
+    // triple a compute unit of more than 32 partitions, a workgroup each; 8 wavefronts a compute unit (what the card holds of
+    // the form with batches of 32) or more, batches of 8.
     const int64_t triples = (int64_t)p->columns * p->heads * p->n_rows, units = compute_units();
-    const bool long_rows = triples <= units && gy > 32, many = triples > 8 * units;
+    const bool long_rows = triples <= units && gy > 32, many = triples >= 8 * units;
 #define PKV_MERGE(W)                                                                                                        \
     case W:                                                                                                                 \
         if (many) hipLaunchKernelGGL((merge_kernel<W, true>), mgrid, dim3(64), 0, stream, a);                               \

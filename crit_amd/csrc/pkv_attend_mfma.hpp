@@ -44,6 +44,7 @@
 // served it, or `fused`.
 #pragma once
 #include "pkv_attend_args.hpp"
+#include "pkv_dma.hpp"
 
 namespace pkv {
 
@@ -129,33 +130,6 @@ struct MfmaShape {
     static constexpr int kGroups = DH == 2 || QT > 2 ? 1 : kMfmaWaves;      // workgroups a compute unit
     static constexpr int kPairs = kRing && kGroups == 1 && !(DH == 2 && KIND == 0) ? 2 : 1;      // pairs of steps in flight a wavefront
 };
-
-// 64 lanes x 16 bytes from base + offset (a lane's own) to LDS bytes lds .. lds + 1023 (ONCE: not kept in the caches), and
-// 4 bytes a lane to lds + 4 lane. Spelled in assembly so that the compiler neither counts these loads nor waits for them:
-// the waits are the kernel's own (wait_dma), and "memory" clobbers, which keeps the reads of LDS behind them.
-template <bool ONCE>
-PKV_DEV void dma_rows(uint32_t offset, const uint8_t* base, unsigned lds) {
-    lds = (unsigned)__builtin_amdgcn_readfirstlane((int)lds);      // (uniform; it may have been kept in a vector register)
-    if constexpr (ONCE) asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(offset), "s"(base), "s"(lds));
-    else asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds));
-}
-PKV_DEV void dma_words(const float* from, unsigned lds) {
-    lds = (unsigned)__builtin_amdgcn_readfirstlane((int)lds);
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(from), "s"(lds));
-}
-template <int N>
-PKV_DEV void wait_dma() {
-    static_assert(N >= 0 && N < 64, "vmcnt is six bits");
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-// The wavefront's own LDS reads have returned: what they read may be overwritten.
-PKV_DEV void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-// 4 consecutive rows of one value, transposed on the way out of LDS: lane 4 j + c of a 16-lane group points at row j's
-// values 4 c .. 4 c + 3; lane i of the group receives value i of rows 0 .. 3.
-PKV_DEV u32x2 read_transposed(const uint8_t* p) {
-    typedef short v4 __attribute__((ext_vector_type(4)));
-    return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4*)(p)));
-}
 
 // The launch: as many workgroups as the card holds at once, each working through units of the list (row, KV head
 // group, query tile, partition) until it is exhausted. The hardware's own dispatcher binds a workgroup to an XCD by its
@@ -296,7 +270,7 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
             s_key[r] = key;
         }
         lds_barrier();
-        if (a.n_rows <= 256) {
+        if (a.n_rows <= 256 && (unsigned)a.units_x * (unsigned)a.units_y > grid) {
             // A row's place is the number of rows before it. A wavefront holds 64 rows' keys, a lane each, and goes through them by
             // v_readlane: no round trip to LDS a row (64 rows: 4,800 of a workgroup's 22,000 clocks before its first step as a
             // loop over LDS; with the quotients and the search by multiplications and ballots, 64 rows ~U[1024, 8192], 5 columns
@@ -312,7 +286,7 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
                 }
                 if (tid < a.n_rows) s_order[rank] = (uint16_t)tid;
             }
-        } else {      // (larger launches keep the rows' order: ranking them costs more than it returns)
+        } else {      // (more rows: ranking them costs more than it returns; a unit a workgroup: all start at once)
             for (int r = tid; r < a.n_rows; r += 256) s_order[r] = (uint16_t)r;
         }
         lds_barrier();

@@ -29,8 +29,6 @@
 namespace pkv {
 namespace {
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-
 struct LatentArgs {
     const uint8_t* q;
     const uint8_t* cache;
@@ -54,13 +52,6 @@ struct LatentArgs {
     int tile_rows;      // the caller's choice: 0 (the geometry decides), 16, 128
     int out16;          // 16-bit results whose rows start on 16 bytes
 };
-
-// 4 consecutive positions (rows of the LDS tile) of one value, transposed on the way out of LDS: lane 4 j + c of a
-// 16-lane group points at row j's values 4 c .. 4 c + 3; lane i of the group receives value i of rows 0 .. 3.
-PKV_DEV u32x2 lds_transposed(const uint8_t* p) {
-    const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(p));
-    return __builtin_bit_cast(u32x2, v);
-}
 
 // NT: query tiles (of 16 rows) a workgroup serves over one staging of the cache rows: 1 where a row's columns times
 // heads fit one tile, else 2 (each tile is then two wavefronts' work: the staging, the barriers and half of the softmax
@@ -314,8 +305,8 @@ __global__ __launch_bounds__(256, NT == 1 ? 3 : 2) void latent_kernel(LatentArgs
             u32x2 va[VR][2];
             auto read_v = [&](auto ic) __attribute__((always_inline)) {
                 constexpr int t = decltype(ic)::value;
-                va[t % VR][0] = lds_transposed(vrow + t * 32);
-                va[t % VR][1] = lds_transposed(vrow + 16 * ROWB + t * 32);
+                va[t % VR][0] = read_transposed(vrow + t * 32);
+                va[t % VR][1] = read_transposed(vrow + 16 * ROWB + t * 32);
             };
             static_for<VR - 1>([&](auto ic) __attribute__((always_inline)) { read_v(ic); });
             static_for<FT>([&](auto ic) __attribute__((always_inline)) {
@@ -400,17 +391,6 @@ PKV_DEV f32x16 mfma_32(u32x4 a, u32x4 b, f32x16 c) {
 // 64 lanes x 16 bytes from base + offset (a lane's own) to LDS bytes lds .. lds + 1023.
 PKV_DEV void dma_row(uint32_t offset, const uint8_t* base, unsigned lds) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds));
-}
-PKV_DEV void dma_any(const uint8_t* from, unsigned lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(lds));
-}
-PKV_DEV void dma_word(const float* from, unsigned lds) {      // 4 bytes a lane, to LDS bytes lds + 4 lane
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(from), "s"(lds));
-}
-template <int N>
-PKV_DEV void wait_loads() {
-    static_assert(N >= 0 && N < 64, "vmcnt is six bits");
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 // The score products and their operand reads are spelled out too, with the accumulators in ordinary registers (the
 // compiler would put them where the value accumulators are and move 16 of those out and back every step) and the waits
@@ -575,7 +555,7 @@ __global__ __launch_bounds__(256, 1) void latent_heads_kernel(LatentArgs a) {
                     dma_any(plan_row0 + (uint32_t)(min(row, plan_room) * W + (c - row * CPR) * 16), plan_to + (unsigned)(k * 1024));
                 }
             } else if constexpr (k == 5) {
-                if (ln < 16) dma_word(plan_scale0 + min(ln & 7, plan_room) * a.scales_per_row + (ln >> 3) * (a.scales_per_row - 1), plan_scale_to);
+                if (ln < 16) dma_words(plan_scale0 + min(ln & 7, plan_room) * a.scales_per_row + (ln >> 3) * (a.scales_per_row - 1), plan_scale_to);
             }
         } else if constexpr (k < 8) {
             const uint32_t place = (uint32_t)(ln ^ ((2 * wave + k / 4) & 3)) * 16u;
@@ -652,7 +632,7 @@ __global__ __launch_bounds__(256, 1) void latent_heads_kernel(LatentArgs a) {
         static_for<5>([&](auto jc) __attribute__((always_inline)) { convert_part(jc, from, to); });
     };
     if constexpr (FP8) {
-        wait_loads<2 * LPT>();      // (its own rows of the first tile are all a wavefront converts: no barrier)
+        wait_dma<2 * LPT>();      // (its own rows of the first tile are all a wavefront converts: no barrier)
         convert(0, 0);
     }
     int raw_stage = 0;      // E4M3: the raw tile that held tile t (tile t + 3 goes there)
@@ -671,7 +651,7 @@ __global__ __launch_bounds__(256, 1) void latent_heads_kernel(LatentArgs a) {
             const int stage = t & (NSTAGE - 1);
             // 16-bit: the tile's loads of this wavefront have landed, those of the next two may be in flight. E4M3: the next
             // tile's have (it is converted at the end of this step), the one after may be in flight.
-            wait_loads<FP8 ? LPT : 2 * LPT>();
+            wait_dma<FP8 ? LPT : 2 * LPT>();
             lds_barrier();              // everybody's have, and nobody reads the tile before any more, nor the last probabilities
             const int base3 = plan(t + 3, FP8 ? raw_stage : (t + 3) & (NSTAGE - 1));
             const uint8_t* tile = ring + stage * TILE;
@@ -827,7 +807,7 @@ __global__ __launch_bounds__(256, 1) void latent_heads_kernel(LatentArgs a) {
 #pragma unroll
                     for (int e = 0; e < 2; ++e) {
                         const uint32_t at = v_lane + 64u * (uint32_t)(vb ^ (i16 >> 2)) + 16u * (v_low ^ (uint32_t)((2 * h + e) & 3));
-                        va[i % RING][e] = lds_transposed(tile + at + (16 * g + 4 * e) * (R * 2));
+                        va[i % RING][e] = read_transposed(tile + at + (16 * g + 4 * e) * (R * 2));
                     }
                 };
                 static_for<RING - 1>([&](auto ic) __attribute__((always_inline)) { read_v(ic); });
@@ -1011,7 +991,7 @@ __global__ __launch_bounds__(256, 1) void latent_heads_kernel(LatentArgs a) {
 #pragma unroll
                 for (int e = 0; e < 2; ++e) {
                     const uint32_t at = L.v_lane + 64u * (uint32_t)(vb ^ (L.i16 >> 2)) + 16u * (L.v_low ^ (uint32_t)((2 * L.h + e) & 3));
-                    va[i % RING][e] = lds_transposed(tile + at + (16 * g + 4 * e) * (R * 2));
+                    va[i % RING][e] = read_transposed(tile + at + (16 * g + 4 * e) * (R * 2));
                 }
             };
             static_for<RING - 1>([&](auto ic) __attribute__((always_inline)) { read_v(ic); });
@@ -1052,7 +1032,7 @@ __global__ __launch_bounds__(256, 1) void latent_heads_kernel(LatentArgs a) {
         const std::false_type no;
         // step 0: no values yet
         {
-            wait_loads<LPT>();
+            wait_dma<LPT>();
             lds_barrier();
             const int base2 = plan(2, 2);
             const Lane L = lane_now();
@@ -1068,7 +1048,7 @@ __global__ __launch_bounds__(256, 1) void latent_heads_kernel(LatentArgs a) {
         // the masked ones, each kind in a loop of its own (a branch around the products inside one loop sends the
         // accumulators to scratch).
         auto step = [&](int t, auto mask_c) __attribute__((always_inline)) {
-            wait_loads<LPT>();      // the tile's loads of this wavefront have landed: those of the next may be in flight
+            wait_dma<LPT>();      // the tile's loads of this wavefront have landed: those of the next may be in flight
             lds_barrier();          // A
             const int base2 = plan(t + 2, (t + 2) & (NSTAGE - 1));
             const Lane L = lane_now();
@@ -1089,7 +1069,7 @@ __global__ __launch_bounds__(256, 1) void latent_heads_kernel(LatentArgs a) {
             values(ring + ((n_tiles - 1) & (NSTAGE - 1)) * TILE, L, no, no, no, 0);
         }
     }
-    wait_loads<0>();      // (the loads past the last tile: LDS must not be written for a workgroup that has gone)
+    wait_dma<0>();      // (the loads past the last tile: LDS must not be written for a workgroup that has gone)
     {
         const int w = (int)f2u(l);
         const auto both = __builtin_amdgcn_permlane32_swap(w, w, false, false);

@@ -12,6 +12,7 @@
 // the B operand it must feed to the second product: no shuffle, no LDS round trip for P.
 //
 // A token's bits follow its own positions only: the key blocks are absolute, masked keys contribute exact zeros.
+#include "pkv_dma.hpp"
 #include "pkv_launch.hpp"
 #include "pkv_prefill.hpp"
 
@@ -44,8 +45,19 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 1 : 8 / WAVES) void prefill_
     // K blocks alternate between two buffers. V blocks too with four wavefronts; with eight, half of the wavefronts
     // multiply by a block's values one iteration after the other half (below), so V blocks go round three buffers.
     constexpr int VBUFS = WAVES == 8 ? 3 : 2;
-    __shared__ __align__(16) uint16_t k_lds[2][BN * KSTR];
-    __shared__ __align__(16) uint16_t v_lds[VBUFS][D * BN];
+    // 16-bit rows of 128- and 256-wide heads reach LDS without passing through registers (DMA): K and V blocks alike as [64
+    // keys][D], the 16-byte chunks of a row permuted, chunk c of key n at place c ^ dma_turn(n) (its low four bits, which
+    // spreads the operands' reads over all banks), and the second product's operand is transposed by the LDS on the way out.
+    // Chunks of 256-wide heads, one wavefront a SIMD, spent 2,600 of a block's 4,900 clocks on 1,000 clocks of score
+    // products and the staging among them: 777 tokens after 1,024, 24 / 2 heads, 92.0 -> 80.9 us, 2,048 tokens 165.8 -> 149.8;
+    // 128-wide ones gain up to 3 % (600 tokens after 2,048 72.8 -> 71.0) or nothing (8 chunks of 512). The others pass
+    // through registers, K rows padded and V transposed there.
+    constexpr bool DMA = KIND == 0 && D >= 128;
+    constexpr int ROWB = 2 * D;                          // DMA: bytes of a row
+    constexpr int DROWS = 1024 / ROWB, DCH = ROWB / 16;   // ... rows a load of a wavefront takes, chunks of a row
+    constexpr int NI = 64 / DROWS / WAVES;               // ... loads of a block's keys (values) a wavefront issues
+    __shared__ __align__(1024) uint16_t k_lds[2][DMA ? BN * D : BN * KSTR];
+    __shared__ __align__(1024) uint16_t v_lds[VBUFS][D * BN];
     __shared__ float ks_lds[2][BN], vs_lds[VBUFS][BN];
 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n32 = lane & 31, h = lane >> 5;
@@ -290,6 +302,9 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 1 : 8 / WAVES) void prefill_
         for (int kb = 0; kb < 2; ++kb) {
             if constexpr (IQK) {
                 dst[kb] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint8_t*>(kl) + (32 * kb + n32) * KSTR8 + 32 * i + 16 * h);
+            } else if constexpr (DMA) {
+                const uint32_t row = (uint32_t)(n32 * ROWB + 16 * (h ^ (4 * (n32 & 3) + ((n32 >> 2) & 3))));
+                dst[kb] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint8_t*>(kl) + (row ^ (32u * (i & 7))) + 256 * (i >> 3) + 32 * kb * ROWB);
             } else {
                 dst[kb] = *reinterpret_cast<const u32x4*>(&kl[(32 * kb + n32) * KSTR + 16 * i + 8 * h]);
             }
@@ -305,11 +320,38 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 1 : 8 / WAVES) void prefill_
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int nb = 2 * (i % (NB / 2)) + j;
+            if constexpr (DMA) {      // groups 4 g + h and 4 g + 2 + h of four keys: two transposing reads
+                const int key = 4 * h + ((lane & 15) >> 2);
+                const uint32_t at = ((uint32_t)(key * ROWB + 8 * (lane & 1) + 16 * ((2 * ((lane >> 4) & 1) + ((lane >> 1) & 1)) ^ (4 * (key & 3) + ((key >> 2) & 3)))) ^ (64u * (nb & 3))) + 256u * (nb >> 2);
+                const u32x2 x = read_transposed(vb + at + 16 * g * ROWB), y = read_transposed(vb + (at ^ 32u) + (16 * g + 8) * ROWB);
+                dst[j] = u32x4{x.x, x.y, y.x, y.y};
+                continue;
+            }
             const u32x4 w = *reinterpret_cast<const u32x4*>(vb + (v_read ^ (16u * ((2 * g) ^ (4 * (nb & 1))))) + 32 * BN * 2 * nb);
             dst[j] = w;
         }
     };
 
+    // DMA. Load j of a wavefront takes rows DROWS (NI wave + j) .. of a block; lane i's 16 bytes go to byte 16 i of the
+    // kilobyte, so a lane fetches the chunk that belongs there. row_of: its row of the block.
+    auto dma_turn = [](int n) __attribute__((always_inline)) -> int { return 4 * (n & 3) + ((n >> 2) & 3); };
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    uint32_t send_slot[DMA ? NI : 1];      // the slots of the lane's rows of the block that is sent for next
+    auto dma_slots = [&]() __attribute__((always_inline)) {      // ... from the entries, lane i holding position i's
+        const uint32_t slot = (uint32_t)ent * (uint32_t)a.page + (uint32_t)inp;
+#pragma unroll
+        for (int j = 0; j < NI; ++j)
+            send_slot[j] = (uint32_t)__builtin_amdgcn_ds_bpermute((DROWS * (NI * wave_u + j) + lane / DCH) << 2, (int)slot);
+    };
+    const unsigned k_at = (unsigned)(uintptr_t)&k_lds[0][0], v_at = (unsigned)(uintptr_t)&v_lds[0][0];
+    auto send = [&](auto ic, int kbuf, int vbuf) __attribute__((always_inline)) {      // load ic of a block's 2 NI: its keys', then its values'
+        constexpr int j = decltype(ic)::value % NI;
+        constexpr bool values = decltype(ic)::value >= NI;
+        const int row = DROWS * (NI * wave_u + j) + lane / DCH;
+        const uint32_t chunk = (uint32_t)((lane % DCH) ^ dma_turn(row));
+        const uint8_t* from = (values ? vbase : kbase) + (uint64_t)send_slot[j] * (values ? v_slot_bytes : k_slot_bytes) + 16 * chunk;
+        dma_any(from, (values ? v_at + (unsigned)(vbuf * 64 * ROWB) : k_at + (unsigned)(kbuf * 64 * ROWB)) + (unsigned)(1024 * (NI * wave_u + j)));
+    };
     f32x16 o[NB];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
@@ -336,7 +378,27 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 1 : 8 / WAVES) void prefill_
     // load of the loop is unconditional (past the last block it repeats the last one), so the compiler counts the
     // outstanding loads exactly instead of waiting for all of them.
     auto upto = [&](int kt) __attribute__((always_inline)) { return kt < kt_hi ? kt : kt_hi; };
-    if (any_block) {
+    // DMA: block kt + 1 is sent for between the products of block kt's scores, its table entries a block earlier; a block starts
+    // when its own rows have landed and everybody is past the one before. Its entries are looked at there, where every load
+    // is waited for anyway (the compiler's own wait on them counts none of the others).
+    auto begin = [&](int kt) __attribute__((always_inline)) {
+        if constexpr (DMA) {
+            wait_dma<0>();
+            dma_slots();
+            load_entries(upto(kt + 2));
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        }
+    };
+    auto end = [&](int kt) __attribute__((always_inline)) {
+        if constexpr (!DMA) __syncthreads();
+    };
+    if (DMA && any_block) {
+        load_entries(kt_lo);
+        dma_slots();
+        static_for<2 * NI>([&](auto ic) __attribute__((always_inline)) { send(ic, kt_lo & 1, WAVES == 8 ? 0 : kt_lo & 1); });
+        load_entries(upto(kt_lo + 1));
+    }
+    if (!DMA && any_block) {
         load_entries(kt_lo);
         take_slots();
         load_k();
@@ -395,13 +457,16 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 1 : 8 / WAVES) void prefill_
                 s[0] = mfma<F16>(ka[i % RING][0], qreg[i], s[0]);
                 s[1] = mfma<F16>(ka[i % RING][1], qreg[i], s[1]);
             }
-            if constexpr (i == 0) store_k(buf ^ 1), load_k();
-            if constexpr (i == KSTEPS / 2 - 1) store_v(vnext), load_v();
-            if constexpr (WAVES == 8 && i == KSTEPS - 2) {      // the slots of block kt + 3 for the next iteration's loads, the entries of kt + 4
+            if constexpr (DMA) {
+                if constexpr (i < 2 * NI) send(ic, buf ^ 1, vnext);      // (past the last block that one again, to a place nobody reads)
+            }
+            if constexpr (!DMA && i == 0) store_k(buf ^ 1), load_k();
+            if constexpr (!DMA && i == KSTEPS / 2 - 1) store_v(vnext), load_v();
+            if constexpr (!DMA && WAVES == 8 && i == KSTEPS - 2) {      // the slots of block kt + 3 for the next iteration's loads, the entries of kt + 4
                 take_slots();
                 load_entries(upto(kt + 4));
             }
-            if constexpr (KIND != 0) PKV_SB();
+            if constexpr (KIND != 0 || DMA) PKV_SB();
         });
         if constexpr (IQK) {      // exact integer dot products of the codes; the rows' and keys' scales follow below
 #pragma unroll
@@ -411,7 +476,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 1 : 8 / WAVES) void prefill_
         }
         // one product, then a share of the staging work (LDS reads of later operands, the stores' permutes and
         // writes, the row loads) in its shadow
-        if constexpr (KIND == 0 && D != 256) {      // (8-bit pages: the conversions' temporaries make this order spill)
+        if constexpr (KIND == 0 && !DMA) {      // (8-bit pages: the conversions' temporaries make this order spill)
             __builtin_amdgcn_sched_group_barrier(0x100, 2 * (RING - 1), 0);
             static_for<2 * KS>([&](auto) __attribute__((always_inline)) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -528,7 +593,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 1 : 8 / WAVES) void prefill_
                 if constexpr (i == 1) pairs(vbuf, std::integral_constant<int, 2>{}, c0), pairs(vbuf, std::integral_constant<int, 2>{}, c1);
                 if constexpr (i == 2) pairs(vbuf, std::integral_constant<int, 3>{}, c0), pairs(vbuf, std::integral_constant<int, 3>{}, c1);
             }
-            if constexpr (WAVES == 4 && i == VSTEPS - 2) {      // the slots of block kt + 3 for the next iteration's loads, the entries of kt + 4
+            if constexpr (!DMA && WAVES == 4 && i == VSTEPS - 2) {      // the slots of block kt + 3 for the next iteration's loads, the entries of kt + 4
                 take_slots();
                 load_entries(upto(kt + 4));
             }
@@ -550,17 +615,14 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 1 : 8 / WAVES) void prefill_
         int kt = kt_lo;
         if constexpr (RESUME) {
             for (; kt < kt_lead; ++kt) {
-                scores(kt, (kt & 1) ^ 1), weigh(kt, kt & 1, c1), values(kt, kt & 1);
-                __syncthreads();
+                begin(kt), scores(kt, (kt & 1) ^ 1), weigh(kt, kt & 1, c1), values(kt, kt & 1), end(kt);
             }
         }
         for (; kt < kt_full; ++kt) {
-            scores(kt, (kt & 1) ^ 1), weigh(kt, kt & 1, c0), values(kt, kt & 1);
-            __syncthreads();          // every wavefront is done with this buffer; the other one is stored
+            begin(kt), scores(kt, (kt & 1) ^ 1), weigh(kt, kt & 1, c0), values(kt, kt & 1), end(kt);
         }
         for (; kt <= kt_hi; ++kt) {
-            scores(kt, (kt & 1) ^ 1), weigh(kt, kt & 1, c1), values(kt, kt & 1);
-            __syncthreads();
+            begin(kt), scores(kt, (kt & 1) ^ 1), weigh(kt, kt & 1, c1), values(kt, kt & 1), end(kt);
         }
     } else {
         // Eight wavefronts, two a SIMD, and the barrier keeps them in step: were both of a SIMD in the same phase, its
@@ -576,46 +638,40 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 1 : 8 / WAVES) void prefill_
             int vcur = 0, kt = kt_lo;
             if constexpr (RESUME) {
                 for (; kt < kt_lead; ++kt) {
-                    scores(kt, after(vcur)), weigh(kt, vcur, c1), values(kt, vcur);
-                    __syncthreads();
+                    begin(kt), scores(kt, after(vcur)), weigh(kt, vcur, c1), values(kt, vcur), end(kt);
                     vcur = after(vcur);
                 }
             }
             for (; kt < kt_full; ++kt) {
-                scores(kt, after(vcur)), weigh(kt, vcur, c0), values(kt, vcur);
-                __syncthreads();
+                begin(kt), scores(kt, after(vcur)), weigh(kt, vcur, c0), values(kt, vcur), end(kt);
                 vcur = after(vcur);
             }
             for (; kt <= kt_hi; ++kt) {
-                scores(kt, after(vcur)), weigh(kt, vcur, c1), values(kt, vcur);
-                __syncthreads();
+                begin(kt), scores(kt, after(vcur)), weigh(kt, vcur, c1), values(kt, vcur), end(kt);
                 vcur = after(vcur);
             }
         } else {
             // iteration kt weighs block kt - 1: masked while that block is below kt_lead or from kt_full on
-            scores(kt_lo, 1);
-            __syncthreads();
+            begin(kt_lo), scores(kt_lo, 1), end(kt_lo);
             int vprev = 0, vcur = 1, kt = kt_lo + 1;
             if constexpr (RESUME) {
                 for (; kt <= min(kt_lead, kt_hi); ++kt) {
-                    weigh(kt - 1, vprev, c1), values(kt - 1, vprev), scores(kt, after(vcur));
-                    __syncthreads();
+                    begin(kt), weigh(kt - 1, vprev, c1), values(kt - 1, vprev), scores(kt, after(vcur)), end(kt);
                     vprev = vcur, vcur = after(vcur);
                 }
             }
             for (; kt <= min(kt_full, kt_hi); ++kt) {
-                weigh(kt - 1, vprev, c0), values(kt - 1, vprev), scores(kt, after(vcur));
-                __syncthreads();
+                begin(kt), weigh(kt - 1, vprev, c0), values(kt - 1, vprev), scores(kt, after(vcur)), end(kt);
                 vprev = vcur, vcur = after(vcur);
             }
             for (; kt <= kt_hi; ++kt) {
-                weigh(kt - 1, vprev, c1), values(kt - 1, vprev), scores(kt, after(vcur));
-                __syncthreads();
+                begin(kt), weigh(kt - 1, vprev, c1), values(kt - 1, vprev), scores(kt, after(vcur)), end(kt);
                 vprev = vcur, vcur = after(vcur);
             }
             weigh(kt_hi, vprev, c1), values(kt_hi, vprev);      // (a mask over a wholly visible block changes nothing)
         }
     }
+    if constexpr (DMA) wait_dma<0>();      // (LDS must not be written for a workgroup that has gone)
     // The two half-waves hold the same row's sums over different keys.
     l += __shfl_xor(l, 32);
     if (!live) return;
