@@ -453,6 +453,21 @@ PKV_DEV unsigned waves_before(const unsigned* s_wave, int wave, int lane, unsign
     return wave > 0 ? upto : 0u;
 }
 
+// The largest (smallest, of the complements) of x over the wavefront, in every lane: data-parallel-primitive steps as in
+// wave_inclusive_sum, then lane 63's value.
+PKV_DEV uint32_t wave_max(uint32_t x) {
+    uint32_t v = x;
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+constexpr int kShortList = 512;      // keys of one bin that are ranked against each other
+
 template <int LEVEL, int EPT>
 __global__ __launch_bounds__(1024) void index_topk_runs_kernel(TopkArgs a) {
     // Four copies of the histogram, a lane's by its number; a copy's bins side by side (a wavefront's lanes that fall into
@@ -461,7 +476,10 @@ __global__ __launch_bounds__(1024) void index_topk_runs_kernel(TopkArgs a) {
     constexpr int COPIES = 4, COPY_WORDS = 2048 + 16;
     __shared__ __align__(16) unsigned s_hist[COPIES * COPY_WORDS];
     __shared__ __align__(16) unsigned s_wave[16];
-    __shared__ unsigned s_pick[2];
+    __shared__ unsigned s_pick[3];
+    __shared__ unsigned s_range[2][16];
+    __shared__ unsigned s_count;
+    __shared__ __align__(16) uint32_t s_list[kShortList];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int t = blockIdx.x, part = LEVEL == 1 ? blockIdx.y : 0;
     const int end = min(max(a.ends[t], 0), a.n);
@@ -534,18 +552,17 @@ __global__ __launch_bounds__(1024) void index_topk_runs_kernel(TopkArgs a) {
     unsigned want = 0u;               // of the keys equal to the k-th, the `want` first are taken
     if (!all) {
         want = (unsigned)k;
-        static_for<3>([&](auto pass) {
-            constexpr int p = pass;
-            constexpr int kShift[3] = {21, 10, 0}, kDigit[3] = {11, 11, 10};
-            constexpr int shift = kShift[p], bins = 1 << kDigit[p], done = shift + kDigit[p];      // `done`: the bits below the digits already chosen
+        // A pass: the keys by their digit `of(key)`, below `bins`, where `in(key)` says; s_pick: the bin that holds the
+        // want-th of them from the top, the want that is left for that bin, the bin's keys.
+        auto pass = [&](auto bins_c, auto&& in, auto&& of) __attribute__((always_inline)) {
+            constexpr int bins = decltype(bins_c)::value;
             for (int i = tid; i < COPIES * COPY_WORDS / 4; i += 1024) reinterpret_cast<u32x4*>(s_hist)[i] = u32x4{0u, 0u, 0u, 0u};
             lds_barrier();
             if (mine) {
                 unsigned* const copy = s_hist + (lane & (COPIES - 1)) * COPY_WORDS;
 #pragma unroll
                 for (int j = 0; j < EPT; ++j) {
-                    if constexpr (p == 0) atomicAdd(&copy[key[j] >> 21], 1u);
-                    else if ((key[j] >> (done & 31)) == (prefix >> (done & 31))) atomicAdd(&copy[(key[j] >> shift) & (unsigned)(bins - 1)], 1u);
+                    if (in(key[j])) atomicAdd(&copy[of(key[j])], 1u);
                 }
             }
             lds_barrier();
@@ -558,13 +575,7 @@ __global__ __launch_bounds__(1024) void index_topk_runs_kernel(TopkArgs a) {
 #pragma unroll
             for (int c = 0; c < COPIES; ++c) {
                 const unsigned* mine_of = s_hist + c * COPY_WORDS + per * tid;
-                if constexpr (per % 4 == 0) {
-#pragma unroll
-                    for (int i = 0; i < per; i += 4) {
-                        const u32x4 v = *reinterpret_cast<const u32x4*>(mine_of + i);
-                        h[i] += v.x, h[i + 1] += v.y, h[i + 2] += v.z, h[i + 3] += v.w;
-                    }
-                } else if constexpr (per == 2) {
+                if constexpr (per == 2) {
                     const u32x2 v = *reinterpret_cast<const u32x2*>(mine_of);
                     h[0] += v.x, h[1] += v.y;
                 } else {
@@ -582,13 +593,58 @@ __global__ __launch_bounds__(1024) void index_topk_runs_kernel(TopkArgs a) {
 #pragma unroll
             for (int i = per - 1; i >= 0; --i) {
                 const unsigned upto = before + h[i];
-                if (upto >= want && before < want) s_pick[0] = (unsigned)(tid * per + i), s_pick[1] = want - before;
+                if (upto >= want && before < want) s_pick[0] = (unsigned)(tid * per + i), s_pick[1] = want - before, s_pick[2] = h[i];
                 before = upto;
             }
             lds_barrier();
-            prefix |= s_pick[0] << shift;
-            want = s_pick[1];
-        });
+        };
+        // The first digit is taken from the keys' own range: the bits below the highest that differs between the candidates'
+        // smallest and largest key, 2,048 bins over what lies between them, where the top bits of the keys as they are put a
+        // row of scores into a few dozen bins (which its atomics then meet in) and leave thousands of keys to two more
+        // digits. A bin then holds a few dozen keys around the k-th, which are ranked against each other at once.
+        uint32_t hi = 0u, lo_not = 0u;      // (elements that are no candidates count as keys of 0: below the range, in bin 0)
+#pragma unroll
+        for (int j = 0; j < EPT; ++j) {
+            hi = max(hi, key[j]);
+            lo_not = max(lo_not, ((ok >> j) & 1u) ? ~key[j] : 0u);
+        }
+        hi = wave_max(hi), lo_not = wave_max(lo_not);
+        if (lane == 0) s_range[0][wave] = hi, s_range[1][wave] = lo_not;
+        if (tid == 0) s_count = 0u;
+        lds_barrier();
+        hi = wave_max(s_range[0][lane & 15]), lo_not = wave_max(s_range[1][lane & 15]);
+        const uint32_t low = ~lo_not, span = hi - low;
+        const int shift0 = span < 2048u ? 0 : 21 - __builtin_clz(span);      // (span >> shift0 is below 2,048)
+        auto digit = [&](uint32_t x) __attribute__((always_inline)) -> uint32_t { return x < low ? 0u : (x - low) >> shift0; };
+        pass(std::integral_constant<int, 2048>{}, [](uint32_t) { return true; }, digit);
+        const unsigned bin = s_pick[0], left = s_pick[1], held = s_pick[2];
+        if (held <= (unsigned)kShortList) {
+            if (mine) {
+#pragma unroll
+                for (int j = 0; j < EPT; ++j)
+                    if (digit(key[j]) == bin) s_list[atomicAdd(&s_count, 1u)] = key[j];
+            }
+            lds_barrier();
+            if (tid < (int)held) {      // the key with fewer than `left` above it and, with its equals, at least `left`
+                const uint32_t x = s_list[tid];
+                unsigned above = 0u, equal = 0u;
+                for (unsigned i = 0; i < held; ++i) above += s_list[i] > x ? 1u : 0u, equal += s_list[i] == x ? 1u : 0u;
+                if (above < left && above + equal >= left) s_pick[0] = x, s_pick[1] = left - above;
+            }
+            lds_barrier();
+            prefix = s_pick[0], want = s_pick[1];
+        } else {      // (many equal or nearly equal keys: digits of 11, 11 and 10 bits from the top)
+            static_for<3>([&](auto step) {
+                constexpr int p = step;
+                constexpr int kShift[3] = {21, 10, 0}, kDigit[3] = {11, 11, 10};
+                constexpr int shift = kShift[p], bins = 1 << kDigit[p], done = shift + kDigit[p];      // `done`: the bits below the digits already chosen
+                pass(std::integral_constant<int, bins>{},
+                     [&](uint32_t x) { return p == 0 || (x >> (done & 31)) == (prefix >> (done & 31)); },
+                     [&](uint32_t x) { return (x >> shift) & (unsigned)(bins - 1); });
+                prefix |= s_pick[0] << shift;
+                want = s_pick[1];
+            });
+        }
     }
     // What each thread writes (above the k-th key | equal to it << 16), then the places before each thread's. A key of
     // 0 is a NaN's or that of an element that is no candidate: only where the k-th key is 0 (or everything is picked)
