@@ -12,7 +12,8 @@
 // the four quarters of the wavefront as (0 + 1) + (2 + 3). That order is the same in both kernels, so a token's bits
 // are its own: not its neighbours', not the launch's shape.
 //   index_scores_kernel: a workgroup is one token and a block of keys, its four wavefronts take tiles of 16 keys in
-//     turn and load them where they lie (from their slots where the keys are read in place): calls of few tokens.
+//     turn and load them where they lie (from their slots where the keys are read in place): calls of few tokens or keys,
+//     and of tokens that read keys of their own.
 //   index_scores_tokens_kernel: a workgroup is 4 or 8 tokens (one or two a wavefront) and a block of keys; 64 keys a
 //     step go through LDS once for all of them (two buffers, one barrier a step, the next step's loads in flight
 //     under the products), so the keys cross the L2 once per 4 or 8 tokens.
@@ -688,9 +689,33 @@ __global__ __launch_bounds__(1024) void index_topk_runs_kernel(TopkArgs a) {
     for (int i = picks + tid; i < k; i += 1024) out[i] = -1;
 }
 
+// Which tokens share the keys of a workgroup: none (a workgroup is one token's), four (a wavefront each), or as many as the
+// registers of four wavefronts hold.
+constexpr int kSharedNone = 0, kSharedFew = 1, kSharedMany = 2;
+
+template <bool F16, bool FP8, int HT, int KS, int TW>
+int launch_scores_shared(const ScoreArgs& a, hipStream_t stream) {
+    constexpr int E = FP8 ? 1 : 2;
+    constexpr size_t lds = (size_t)4 * TW * HT * 16 * 4 + 2 * 64 * (KS * 32 * E + 16);
+    if (lds > 48 * 1024) {
+        static bool raised[16] = {};      // per device: the kernel's LDS limit
+        int device = 0;
+        if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 16) return CRIT_PKV_E_GEOMETRY;
+        if (!raised[device]) {
+            if (hipFuncSetAttribute(reinterpret_cast<const void*>(&index_scores_tokens_kernel<F16, FP8, HT, KS, TW>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+                return CRIT_PKV_E_GEOMETRY;
+            raised[device] = true;
+        }
+    }
+    const dim3 grid((unsigned)((a.n + a.block - 1) / a.block), (unsigned)((a.tokens + 4 * TW - 1) / (4 * TW)));
+    hipLaunchKernelGGL((index_scores_tokens_kernel<F16, FP8, HT, KS, TW>), grid, dim3(256), lds, stream, a);
+    return hip_code(hipGetLastError());
+}
+
 template <bool F16, bool FP8, int HT, int KS>
-int launch_scores_shape(ScoreArgs a, bool many, int cus, hipStream_t stream) {
-    if (!many) {
+int launch_scores_shape(ScoreArgs a, int shared, int cus, hipStream_t stream) {
+    if (shared == kSharedNone) {
         // A block of keys a workgroup, sized so that the workgroups are as many as the chip holds at once (or a whole
         // number of times that many): every one runs from the start and they end together. Three tiles in flight a
         // wavefront where the queries leave the registers room and a wavefront has 64 tiles or more (measured: 64
@@ -725,32 +750,23 @@ int launch_scores_shape(ScoreArgs a, bool many, int cus, hipStream_t stream) {
         return hip_code(hipGetLastError());
     }
     constexpr int TW = HT * KS <= 16 && HT <= 4 ? 2 : 1;      // two tokens a wavefront where their queries fit its registers
-    constexpr int E = FP8 ? 1 : 2;
-    constexpr size_t lds = (size_t)4 * TW * HT * 16 * 4 + 2 * 64 * (KS * 32 * E + 16);
+    if (shared == kSharedFew) {
+        // A block for two workgroups a compute unit, of whole steps of 64 keys.
+        const int64_t wgs_t = (a.tokens + 3) / 4, wanted = ((int64_t)a.n * wgs_t + 2 * cus - 1) / (2 * (int64_t)cus);
+        a.block = (int)min((wanted + 63) / 64 * 64, (int64_t)8192);
+        return launch_scores_shared<F16, FP8, HT, KS, 1>(a, stream);
+    }
     const int wgs_t = (a.tokens + 4 * TW - 1) / (4 * TW);
     int block = 256;
     while (block < 8192 && (int64_t)wgs_t * ((a.n + block - 1) / block) > (int64_t)cus * 16) block *= 2;
     a.block = block;
-    if (lds > 48 * 1024) {
-        static bool raised[16] = {};      // per device: the kernel's LDS limit
-        int device = 0;
-        if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 16) return CRIT_PKV_E_GEOMETRY;
-        if (!raised[device]) {
-            if (hipFuncSetAttribute(reinterpret_cast<const void*>(&index_scores_tokens_kernel<F16, FP8, HT, KS, TW>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-                return CRIT_PKV_E_GEOMETRY;
-            raised[device] = true;
-        }
-    }
-    const dim3 grid((unsigned)((a.n + block - 1) / block), (unsigned)wgs_t);
-    hipLaunchKernelGGL((index_scores_tokens_kernel<F16, FP8, HT, KS, TW>), grid, dim3(256), lds, stream, a);
-    return hip_code(hipGetLastError());
+    return launch_scores_shared<F16, FP8, HT, KS, TW>(a, stream);
 }
 
 template <bool F16, bool FP8>
-int launch_scores_kind(const ScoreArgs& a, int dim, bool many, int cus, hipStream_t stream) {
+int launch_scores_kind(const ScoreArgs& a, int dim, int shared, int cus, hipStream_t stream) {
     const int ht = (a.heads + 15) / 16;
-#define PKV_SHAPE(H, K) if (ht == H && dim == K * 32) return launch_scores_shape<F16, FP8, H, K>(a, many, cus, stream);
+#define PKV_SHAPE(H, K) if (ht == H && dim == K * 32) return launch_scores_shape<F16, FP8, H, K>(a, shared, cus, stream);
     PKV_SHAPE(1, 2) PKV_SHAPE(1, 4) PKV_SHAPE(1, 8)
     PKV_SHAPE(2, 2) PKV_SHAPE(2, 4) PKV_SHAPE(2, 8)
     PKV_SHAPE(4, 2) PKV_SHAPE(4, 4) PKV_SHAPE(4, 8)
@@ -844,13 +860,32 @@ int launch_index_scores(const crit_pkv_index_scores_params* p, hipStream_t strea
     a.scale = p->scale, a.block = 64;
     const int cus = compute_units() > 0 ? compute_units() : 256;
     // many tokens share their keys through LDS, 4 or 8 to a workgroup: where the keys are read in place, a group's
-    // tokens (they share the slots) must fill workgroups, unless one list serves every token (slots_stride 0)
+    // tokens (they share the slots) must fill workgroups, unless one list serves every token
     const int ht = (p->heads + 15) / 16;
     const int wg_tokens = ht * (p->dim / 32) <= 16 && ht <= 4 ? 8 : 4;
-    const bool many = p->tokens >= 16 && (!p->slots || p->slots_stride == 0 || p->group % wg_tokens == 0);
+    auto share = [&](int tokens) { return !p->slots || p->slots_stride == 0 || p->group % tokens == 0; };
+    // Four tokens or more: a workgroup a token would load every key once a token, a request of 16 bytes a lane (its
+    // operand's lanes lie in 16 keys), which bounds such calls (64 heads of 128, 4 tokens over 50,000 keys: 14.8 us, shared
+    // 11.8; 15 over 65,536, with the selection, 56.9 and 43.8; 16 sequences of 4 over 50,000 each 124.3 and 85.8). Not
+    // where many wavefronts would have no token (2 over 65,536 E4M3 keys 23.0 and 24.9; 5 over 10,000 6.9 and 7.9, 6 over
+    // 50,000 16.7 and 17.3), nor where the keys are too few for the steps of 64 (4 tokens: 4,000 keys 5.0 and 5.7, 8,000
+    // 5.65 and 5.71, 12,000 6.3 and 5.8). E4M3 keys are half the requests (24,000 keys: 4 tokens 7.3 and 8.2, 8 tokens 10.3
+    // and 10.9; 32,000: 8 tokens 12.8 and 11.0; 15 over 20,000 11.1 and 12.5), and queries past 16 operands leave one
+    // workgroup a compute unit (128 heads of 128, 8 tokens: 12,000 keys 11.0 and 12.5, 32,000 22.9 and 17.0; E4M3 7 over
+    // 52,000 21.1 and 23.2, 11 over 37,000 28.0 and 23.4).
+    const int64_t products = (int64_t)p->tokens * p->n;
+    const bool wide = ht * (p->dim / 32) > 16, filled = p->tokens == 4 || p->tokens == 7 || p->tokens == 8 || p->tokens >= 10;
+    const int64_t enough = fp8 ? (wide || p->tokens > 8 ? 400000 : 256000) : wide ? 256000 : 48000;
+    const bool fours = filled && products >= enough && (share(4) || (p->tokens < 16 && p->group >= p->tokens));
+    // Calls of 16 tokens and more share eight to a workgroup, in blocks of 256 keys or more, once such workgroups fill the chip,
+    // and fours before that (16 tokens: 2,000 keys 13.9 us, in fours 5.4, 9,000 14.4 and 9.6, 32,000 16.9 and 15.9, 65,536 23.7
+    // both; 48: 9,000 keys 14.5 and 13.3, 65,536 63.0 and 67.1; 128 heads, fours either way: 50 tokens over 2,000 keys 13.9 and
+    // 12.2, 100 14.1 and 15.4).
+    const bool eights = p->tokens >= 16 && share(wg_tokens), few = eights ? products <= (wide ? 128000 : 560000) : fours;
+    const int shared = few ? kSharedFew : eights ? kSharedMany : kSharedNone;
     const bool f16 = p->q_dtype == CRIT_PKV_F16;
-    if (fp8) return f16 ? launch_scores_kind<true, true>(a, p->dim, many, cus, stream) : launch_scores_kind<false, true>(a, p->dim, many, cus, stream);
-    return f16 ? launch_scores_kind<true, false>(a, p->dim, many, cus, stream) : launch_scores_kind<false, false>(a, p->dim, many, cus, stream);
+    if (fp8) return f16 ? launch_scores_kind<true, true>(a, p->dim, shared, cus, stream) : launch_scores_kind<false, true>(a, p->dim, shared, cus, stream);
+    return f16 ? launch_scores_kind<true, false>(a, p->dim, shared, cus, stream) : launch_scores_kind<false, false>(a, p->dim, shared, cus, stream);
 }
 
 int64_t index_topk_work_bytes(int tokens, int n, int k) {

@@ -1,5 +1,5 @@
 """Where the window kernels' pairs of steps, rings, folds and merges, the prompt kernel's loads straight into LDS, the index
-selection's short list and the latent merge's wide stores can go wrong: pieces whose last pair lacks a step, wavefronts
+selection's short list and shared keys and the latent merge's wide stores can go wrong: pieces whose last pair lacks a step, wavefronts
 without a step, units of more pairs than a wavefront holds entries for, three tiles of 8-bit pages, merges of many
 wavefronts and of long rows, and edges of lists. Against float64 attention over the stored values, the oracle's picks, or
 the fused launch bit for bit."""
@@ -118,6 +118,27 @@ def test_picks_where_the_kth_score_has_many_near_it(n, k, equal):
         want = torch.from_numpy(oracle_indexer.sparse_index(rows.double().cpu().numpy(), ends.cpu().numpy(), k))
         import crit_amd.sparse_indexer as si
         assert torch.equal(si.topk(rows, ends, k).long().cpu(), want)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("tokens,heads,d", [(18, 64, 128), (33, 16, 128), (4, 64, 128), (7, 16, 64), (11, 128, 128), (15, 64, 256)])
+@pytest.mark.parametrize("n", [1, 12000, 12001, 16064, 64001])
+def test_a_few_tokens_score_their_keys_together_as_alone(fp8, tokens, heads, d, n):
+    # four to fifteen tokens share a workgroup's keys: edges of its steps of 64 keys, a last workgroup of one to three tokens
+    import crit_amd.sparse_indexer as si
+    g = torch.Generator().manual_seed(n + tokens)
+    q = torch.randn(tokens, heads, d, generator=g).to(dev, torch.bfloat16)
+    rows = torch.randn(n + 3, d, generator=g).to(dev, torch.bfloat16)
+    keys, scales = (rows.to(torch.float8_e4m3fn), torch.rand(n + 3, generator=g).to(dev) + 0.5) if fp8 else (rows, None)
+    w = torch.randn(tokens, heads, generator=g).to(dev)
+    ends = torch.randint(0, n + 1, (tokens,), generator=g, dtype=torch.int32).to(dev)
+    ends[0] = n
+    slots = torch.randperm(n + 3, generator=g)[:n].int().to(dev)
+    for kw in ({"slots": slots}, {"slots": slots[None]}, {}):
+        got = si.scores(q, keys, w, ends, key_scales=scales, **kw)
+        for t in (0, 1, 3, tokens - 1):
+            alone = si.scores(q[t:t + 1], keys, w[t:t + 1], ends[t:t + 1], key_scales=scales, **kw)
+            assert torch.equal(got[t], alone[0]), t
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
