@@ -45,14 +45,15 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 1 : 8 / WAVES) void prefill_
     // K blocks alternate between two buffers. V blocks too with four wavefronts; with eight, half of the wavefronts
     // multiply by a block's values one iteration after the other half (below), so V blocks go round three buffers.
     constexpr int VBUFS = WAVES == 8 ? 3 : 2;
-    // 16-bit rows of 128- and 256-wide heads reach LDS without passing through registers (DMA): K and V blocks alike as [64
-    // keys][D], the 16-byte chunks of a row permuted, chunk c of key n at place c ^ dma_turn(n) (its low four bits, which
-    // spreads the operands' reads over all banks), and the second product's operand is transposed by the LDS on the way out.
-    // Chunks of 256-wide heads, one wavefront a SIMD, spent 2,600 of a block's 4,900 clocks on 1,000 clocks of score
-    // products and the staging among them: 777 tokens after 1,024, 24 / 2 heads, 92.0 -> 80.9 us, 2,048 tokens 165.8 -> 149.8;
-    // 128-wide ones gain up to 3 % (600 tokens after 2,048 72.8 -> 71.0) or nothing (8 chunks of 512). The others pass
-    // through registers, K rows padded and V transposed there.
-    constexpr bool DMA = KIND == 0 && D >= 128;
+    // 16-bit rows of 256-wide heads, and of 128-wide ones with four wavefronts, reach LDS without passing through registers
+    // (DMA): K and V blocks alike as [64 keys][D], the 16-byte chunks of a row permuted, chunk c of key n at place c ^
+    // dma_turn(n) (its low four bits, which spreads the operands' reads over all banks), and the second product's operand is
+    // transposed by the LDS on the way out. Chunks of 256-wide heads, one wavefront a SIMD, spent 2,600 of a block's 4,900
+    // clocks on 1,000 clocks of score products and the staging among them: 777 tokens after 1,024, 24 / 2 heads, 92.0 -> 80.9
+    // us, 2,048 tokens 165.8 -> 149.8; 128-wide ones gain up to 3 % (600 tokens after 2,048 72.8 -> 71.0). With eight
+    // wavefronts, two a SIMD, one hides the other's staging, and the wait for the rows shows instead (8 chunks of 512: 289.1
+    // us, 290.9 so). Those, 64-wide heads and 8-bit pages pass through registers, K rows padded and V transposed there.
+    constexpr bool DMA = KIND == 0 && D >= 128 && WAVES == 4;
     constexpr int ROWB = 2 * D;                          // DMA: bytes of a row
     constexpr int DROWS = 1024 / ROWB, DCH = ROWB / 16;   // ... rows a load of a wavefront takes, chunks of a row
     constexpr int NI = 64 / DROWS / WAVES;               // ... loads of a block's keys (values) a wavefront issues
