@@ -6,17 +6,17 @@
 // pipe cannot keep up with 8-bit pages at HBM rate (one v_dot2 per two multiply-adds, plus the conversions, was two
 // thirds of its cycles): a step is 16 positions of one KV head, and steps are taken in pairs,
 //   S^T[16 positions][16 query rows] = K[16][128] . Q^T      4 x v_mfma_f32_16x16x32 a step (bf16 / f16 operands)
-//   O^T[128 dims][16 query rows]    += V^T[128][32] . P^T    8 x v_mfma_f32_16x16x32 a pair
+//   O^T[128 dims][16 query rows]    += V^T[128][16] . P^T    8 x v_mfma_f32_16x16x16 a step, or
+//                                   += V^T[128][32] . P^T    8 x v_mfma_f32_16x16x32 a pair (pages of scaled rows)
 // with operands laid out so that nothing is shuffled between the two products:
 //   keys    lane (p = lane % 16, u = lane / 16) holds 16-byte pieces of the row of position p; piece c holds dims
 //           32 c + 8 u .. + 7, the eight contraction elements the first product's A operand wants from that lane
 //           (8-bit pages: two pieces of 16 codes, converted to 16-bit pairs, exactly);
-//   scores  come out with lane (c = lane % 16, u) holding query row c at positions 4 u .. 4 u + 3, which is half of
-//           the B operand of the second product, the pair's other step the other half: the probabilities go from the
-//           softmax to the matrix pipe as four packed registers, no LDS, no shuffle;
-//   values  lane (i, u) holds a dim of the rows of positions 4 u .. 4 u + 3 of both steps, as four 16-bit pairs.
-// A pair has one maximum, one factor and one sum a query row where two steps had two, and half the products for the
-// values.
+//   scores  come out with lane (c = lane % 16, u) holding query row c at positions 4 u .. 4 u + 3, which is the B operand
+//           of a step's second product, or half of a pair's: the probabilities go from the softmax to the matrix pipe as
+//           packed registers, no LDS, no shuffle;
+//   values  lane (i, u) holds a dim of the rows of positions 4 u .. 4 u + 3 of a step, as two 16-bit pairs.
+// Which of the two: G, below.
 // The 16 query rows of a tile are rows of the flattened (column, group head) list, so the GQA group's heads share
 // every K/V byte read once. A wavefront serves HW adjacent KV heads (2 where the head count is even) in ONE matrix tile:
 // a step is then 8 positions of both heads (rows 0 .. 7 of the tile the first head's positions, rows 8 .. 15 the
@@ -24,7 +24,7 @@
 // other head's queries are masked), so a load instruction fetches both heads' rows of a position, 512 contiguous bytes
 // of 16-bit pages: what the HBM system streams best from randomly placed pages.
 // Softmax state: the running maximum of a query row is kept equal in the four lanes that hold the row (two
-// v_permlane swaps a pair), the sums per lane until the unit's end.
+// v_permlane swaps a maximum), the sums per lane until the unit's end.
 //
 // How a step's rows reach their operands. With one or two query tiles over 16-bit pages a wavefront loads them straight
 // into the operands' registers, a pair in flight beside the one in use, two workgroups a compute unit. A key operand's lanes
@@ -34,7 +34,7 @@
 // own ring in LDS (global_load_lds: no register holds them, a request takes 64 adjacent bytes) and read the operands from
 // there, values transposed by the LDS itself (ds_read_b64_tr_b16). Nothing is shared between wavefronts, so no barrier
 // orders the ring: the waits count loads. Against the same kernels with all rows in registers: 64 rows ~U[1024, 8192], 32
-// / 8 heads x 128, 5 columns BF16 331 -> 298 us; 8 rows of 16,000, 24 / 4 x 256, fp8:row 74 -> 67; one row of 50,000, 56 /
+// / 8 heads x 128, 5 columns BF16 331 -> 303 us; 8 rows of 16,000, 24 / 4 x 256, fp8:row 74 -> 67; one row of 50,000, 56 /
 // 8, 8 columns, INT8 116 -> 98.
 //
 // Row-exactness: position n is always read in the same step of the same pair of the same wavefront of its unit (pairs do
@@ -56,6 +56,25 @@ PKV_DEV f32x4 mfma_k32(u32x4 a, u32x4 b, f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
     }
 }
+template <bool F16>
+PKV_DEV f32x4 mfma_k16(u32x2 a, u32x2 b, f32x4 c) {
+    typedef __attribute__((ext_vector_type(4))) short s16x4;
+    typedef __attribute__((ext_vector_type(4))) _Float16 f16x4;
+    if constexpr (F16) {
+        return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4, a), __builtin_bit_cast(f16x4, b), c, 0, 0, 0);
+    } else {
+        return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), c, 0, 0, 0);
+    }
+}
+
+// The values of one step, or of a pair's two, as the second product's operand: two 16-bit pairs a step.
+template <bool F16>
+PKV_DEV f32x4 mfma_steps(const uint32_t (&a)[2], const uint32_t (&b)[2], f32x4 c) { return mfma_k16<F16>(u32x2{a[0], a[1]}, u32x2{b[0], b[1]}, c); }
+template <bool F16>
+PKV_DEV f32x4 mfma_steps(const uint32_t (&a)[4], const uint32_t (&b)[4], f32x4 c) {
+    return mfma_k32<F16>(u32x4{a[0], a[1], a[2], a[3]}, u32x4{b[0], b[1], b[2], b[3]}, c);
+}
+
 template <bool F16>
 PKV_DEV uint32_t pair16(float a, float b) {      // two FP32 values as one 16-bit pair, round to nearest even
     if constexpr (F16) return pack_f16(a, b);
@@ -177,6 +196,13 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
     constexpr int EB = KIND == 0 ? 2 : 1;
     constexpr int CPH = kTileRows / HW;      // tile columns a KV head holds
     constexpr int SPW = kTileRows / HW;      // positions a wavefront's step covers (tile rows a KV head holds)
+    // Steps that share one maximum, factor and sum, and one product for their values. Both of a pair where a row's scale is
+    // multiplied into the probability before it is rounded to 16 bits. Elsewhere a step has its own: its largest
+    // probability, where it moves the maximum, is then 1, which 16 bits hold, and one maximum for both leaves the first
+    // step's below 1 (16 rows ~U[1024, 8192], FP32 results, from 64 bits: BF16 1.237e-3 in place of 1.253e-3, 256-wide heads
+    // 1.171e-3 in place of 1.215e-3, FP8 1.364e-3 in place of 1.372e-3; row-scaled FP8 and INT8 1.609e-3 and 1.589e-3
+    // either way). One maximum is the cheaper: 5 columns of 64 such rows BF16 289 us, each its own 303; FP8 174 and 207.
+    constexpr int G = KIND >= 2 ? 2 : 1;
     constexpr int FW = RING ? 64 : D;        // output dims folded at a time
     constexpr int FG = FW / 64;              // groups of four of them a thread folds: dims 64 i + 4 (tid % 16) .. + 3 of column tid / 16
     constexpr int ROWB = D * EB;             // bytes of a key or value row
@@ -615,35 +641,192 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
 
                 const int odd_cur = odd_of(cur);
                 // A pair of steps, in places 2 i and 2 i + 1: positions base .. + SPW - 1 and second .. + SPW - 1 (second < 0: no such
-                // step). keys_here and values_here wait until the pair's have landed.
+                // step). keys_here and values_here wait until the pair's have landed, refill_k and refill_v send for what comes to a
+                // step's place next. Both steps' scores come first, then their probabilities, then the values; two query tiles
+                // in registers go step by step (both steps' scores and probabilities at once are 76 bytes of scratch a lane
+                // more: 64 rows ~U[1024, 8192], 32 / 8 heads, a tree of 4, 279 us, 266 so; one tile 215.7 and 217.8).
+                constexpr bool APART = !RING && QT > 1;
                 auto step = [&](int base, int second, int i, auto&& keys_here, auto&& values_here, auto&& refill_k, auto&& refill_v) __attribute__((always_inline)) {
                     const int base_b = second >= 0 ? second : 0x3fffff00;      // (past every column's last position)
-                    keys_here();
-                    // -- scores: the two steps' are two chains of products
-                    f32x4 s0[QT], s1[QT];
-#pragma unroll
-                    for (int q = 0; q < QT; ++q) s0[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f}, s1[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-                    const uint8_t* const place_a = &s_ring[RING ? wave : 0][RING ? 2 * i : 0][0];
-                    const uint8_t* const place_b = &s_ring[RING ? wave : 0][RING ? 2 * i + 1 : 0][0];
+                    // Both steps wholly seen by every column of the tiles (a draft tree's: before the window's first
+                    // position): nothing is asked of a position.
+                    const bool whole = MASK != kMaskSliding && win <= 0 &&
+                                       base_b + SPW <= min(MASK == kMaskTree ? cur.first : cur.first + cur.c_lo + 1, cur.n_keys);
+                    const uint8_t* const places[2] = {&s_ring[RING ? wave : 0][RING ? 2 * i : 0][0], &s_ring[RING ? wave : 0][RING ? 2 * i + 1 : 0][0]};
+                    // -- scores of steps lo .. hi - 1. A step of its own maximum sums the keys' even pieces and the odd ones apart.
+                    f32x4 s0[2][QT], s1[2][QT];
                     u32x4 held[2][RING ? CPR / 4 : 1];
+                    auto scores = [&](int lo, int hi) __attribute__((always_inline)) {
+#pragma unroll
+                        for (int r = lo; r < hi; ++r)
+#pragma unroll
+                            for (int q = 0; q < QT; ++q) s0[r][q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f}, s1[r][q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                        for (int c = 0; c < 4 * DH; ++c) {
+                            u32x4 k[2];
+#pragma unroll
+                            for (int r = lo; r < hi; ++r) k[r] = key_operand<KIND>(RING ? held[r] : t[RING ? 0 : 2 * i + r].k, c);
+#pragma unroll
+                            for (int q = 0; q < QT; ++q) {
+#pragma unroll
+                                for (int r = lo; r < hi; ++r) {
+                                    f32x4& sum = G == 1 && c % 2 ? s1[r][q] : s0[r][q];
+                                    sum = mfma_k32<F16>(k[r], qb[q][c], sum);
+                                }
+                            }
+                        }
+                    };
+                    float ks8[8], vs8[8];
+                    // -- the lane's probabilities: its column at positions base + r_pos + i, second + r_pos + i of head r_head. Another
+                    // head's column (a lane that is not `mine`) sees nothing: its scores stay out of the maximum, its
+                    // probabilities become zeros (chosen, not multiplied: the other head's values may be anything).
+                    uint32_t pb[2][QT][2 * G];
+                    float alpha[2][QT];
+                    bool rescale[2];
+                    auto soften = [&](int r) __attribute__((always_inline)) {      // step r, or with G 2 both
+                        rescale[r] = false;
+#pragma unroll
+                        for (int q = 0; q < QT; ++q) {
+                            float x[4 * G];
+#pragma unroll
+                            for (int i = 0; i < 4 * G; ++i) {
+                                const int st = G == 1 ? r : i / 4;
+                                const float raw = G == 1 ? s0[st][q][i & 3] + s1[st][q][i & 3] : s0[st][q][i & 3];
+                                x[i] = raw * (KIND >= 2 ? sscale * ks8[4 * st + (i & 3)] : sscale);
+                            }
+                            if (!whole) {
+                                const int room = lim[q] - r_pos;      // position n (of the step's first) is visible while n + i <= room
+#pragma unroll
+                                for (int i = 0; i < 4 * G; ++i) {
+                                    const int at = ((G == 1 ? r : i / 4) == 0 ? base : base_b) + (i & 3);
+                                    bool vis = at <= room;
+                                    if constexpr (MASK != kMaskNone) {
+                                        const int n = at + r_pos;
+                                        if (tree) vis = vis && (n < cur.first || ((anc[q] >> ((n - cur.first) & 63)) & 1ull) != 0);
+                                        if (win > 0) vis = vis && n > cur.first + col[q] - win;
+                                    }
+                                    x[i] = vis ? x[i] : -INFINITY;
+                                }
+                            }
+                            float y = __builtin_fmaxf(__builtin_fmaxf(x[0], x[1]), __builtin_fmaxf(x[2], x[3]));
+                            if constexpr (G == 2) y = __builtin_fmaxf(y, __builtin_fmaxf(__builtin_fmaxf(x[4], x[5]), __builtin_fmaxf(x[6], x[7])));
+                            if constexpr (HW > 1) y = mine ? y : -INFINITY;
+                            const float m_new = __builtin_fmaxf(m[q], max_across_quarters(y));
+                            const float sub = m_new == -INFINITY ? 0.0f : m_new;
+                            alpha[r][q] = m[q] == -INFINITY ? 1.0f : exp2_fast(m[q] - sub);      // (nothing summed yet: nothing to rescale)
+                            rescale[r] = rescale[r] || alpha[r][q] != 1.0f;
+                            m[q] = m_new;
+                            float p[4 * G];
+#pragma unroll
+                            for (int i = 0; i < 4 * G; ++i) p[i] = exp2_fast(x[i] - sub);
+                            float sum = (p[0] + p[1]) + (p[2] + p[3]);
+                            if constexpr (G == 2) sum += (p[4] + p[5]) + (p[6] + p[7]);
+                            sum = HW == 1 || mine ? sum : 0.0f;
+                            l[q] = G == 1 ? __builtin_fmaf(l[q], alpha[r][q], sum) : l[q] * alpha[r][q] + sum;
+#pragma unroll
+                            for (int i = 0; i < 2 * G; ++i) {
+                                const uint32_t w = KIND >= 2 ? pair16<F16>(p[2 * i] * vs8[2 * i], p[2 * i + 1] * vs8[2 * i + 1]) : pair16<F16>(p[2 * i], p[2 * i + 1]);
+                                pb[r][q][i] = HW == 1 || mine ? w : 0u;
+                            }
+                        }
+                    };
+                    auto move = [&](int r) __attribute__((always_inline)) {
+                        if (__builtin_amdgcn_ballot_w64(rescale[r]) != 0) {      // some column's maximum moved
+#pragma unroll
+                            for (int q = 0; q < QT; ++q)
+#pragma unroll
+                                for (int j = 0; j < 8 * DH; ++j) acc[q][j] *= alpha[r][q];
+                        }
+                    };
+                    // The row's last steps: what lies past its keys may be anything, and a probability of zero times a NaN is a
+                    // NaN. Such values become zeros.
+                    auto clean = [&](int r) __attribute__((always_inline)) {
+                        const int at = r == 0 ? base : base_b;
+                        if (at + SPW > cur.n_keys) {
+                            if constexpr (RING) {
+                                uint8_t* values = &s_ring[wave][2 * i + r][HALF];
+                                for (int row = 0; row < 16; ++row) {
+                                    if (at + row % SPW < cur.n_keys) continue;
+                                    uint8_t* to = values + (KIND == 0 ? row : 4 * (row & 3) + (row >> 2)) * ROWB;
+                                    for (int b = lane * 4; b < ROWB; b += 256) *reinterpret_cast<uint32_t*>(to + b) = 0u;
+                                }
+                            } else {
+#pragma unroll
+                                for (int p = 0; p < 4; ++p)
+                                    if (at + r_pos + p >= cur.n_keys) t[RING ? 0 : 2 * i + r].v[p] = u32x4{0, 0, 0, 0};
+                            }
+                        }
+                    };
+                    // -- values: the lane's dims of a step's four rows as two 16-bit pairs, then O^T += V^T P^T
+                    auto values = [&](int r) __attribute__((always_inline)) {      // step r, or with G 2 both
+                        if constexpr (!RING) {      // dims {8 i + j}: a v_perm a pair
+                            const Tile& tl = t[RING ? 0 : 2 * i + r];
+#pragma unroll
+                            for (int w = 0; w < 4; ++w) {
+                                const uint32_t lo[2] = {__builtin_amdgcn_perm(tl.v[1][w], tl.v[0][w], 0x05040100), __builtin_amdgcn_perm(tl.v[3][w], tl.v[2][w], 0x05040100)};
+                                const uint32_t hi[2] = {__builtin_amdgcn_perm(tl.v[1][w], tl.v[0][w], 0x07060302), __builtin_amdgcn_perm(tl.v[3][w], tl.v[2][w], 0x07060302)};
+#pragma unroll
+                                for (int q = 0; q < QT; ++q) {
+                                    acc[q][2 * w] = mfma_steps<F16>(lo, pb[r][q], acc[q][2 * w]);
+                                    acc[q][2 * w + 1] = mfma_steps<F16>(hi, pb[r][q], acc[q][2 * w + 1]);
+                                }
+                            }
+                        } else if constexpr (KIND == 0) {      // dims 16 b + (0 .. 15): transposed by the LDS
+#pragma unroll
+                            for (int b = 0; b < 8 * DH; ++b) {
+                                const u32x2 v = read_transposed(places[r] + (uint32_t)HALF + t_read + (t_turn ^ (uint32_t)(32 * (b & 7))) + (uint32_t)(256 * (b >> 3)));
+                                const uint32_t va[2] = {v.x, v.y};
+#pragma unroll
+                                for (int q = 0; q < QT; ++q) acc[q][b] = mfma_steps<F16>(va, pb[r][q], acc[q][b]);
+                            }
+                        } else {      // dims {8 i + j}: codes of adjacent rows side by side, then as 16-bit pairs
+#pragma unroll
+                            for (int h = 0; h < DH; ++h) {
+                                u32x2 v[G][4];
+#pragma unroll
+                                for (int p = 0; p < 4; ++p) {
+                                    const uint32_t at = (uint32_t)(HALF + (4 * p + u4) * ROWB + 128 * h + 8 * c16);
+#pragma unroll
+                                    for (int g = 0; g < G; ++g) v[g][p] = *reinterpret_cast<const u32x2*>(places[r + g] + at);
+                                }
+#pragma unroll
+                                for (int w = 0; w < 2; ++w) {
+                                    uint32_t va[4][2 * G];
+#pragma unroll
+                                    for (int g = 0; g < G; ++g) {
+                                        // bytes (a0 b0 a1 b1) and (a2 b2 a3 b3): two rows' codes of one dim side by side
+                                        const uint32_t lo01 = __builtin_amdgcn_perm(v[g][1][w], v[g][0][w], 0x05010400), hi01 = __builtin_amdgcn_perm(v[g][1][w], v[g][0][w], 0x07030602);
+                                        const uint32_t lo23 = __builtin_amdgcn_perm(v[g][3][w], v[g][2][w], 0x05010400), hi23 = __builtin_amdgcn_perm(v[g][3][w], v[g][2][w], 0x07030602);
+                                        // (dims 4 w + 0, 1 from the low halves, 2, 3 from the high ones; .x: rows 0, 1; .y: rows 2, 3)
+                                        const u32x2 a01 = codes4_to_pairs<KIND>(lo01), a23 = codes4_to_pairs<KIND>(lo23);
+                                        const u32x2 b01 = codes4_to_pairs<KIND>(hi01), b23 = codes4_to_pairs<KIND>(hi23);
+                                        va[0][2 * g] = a01.x, va[0][2 * g + 1] = a23.x, va[1][2 * g] = a01.y, va[1][2 * g + 1] = a23.y;
+                                        va[2][2 * g] = b01.x, va[2][2 * g + 1] = b23.x, va[3][2 * g] = b01.y, va[3][2 * g + 1] = b23.y;
+                                    }
+#pragma unroll
+                                    for (int q = 0; q < QT; ++q) {
+#pragma unroll
+                                        for (int j = 0; j < 4; ++j) acc[q][8 * h + 4 * w + j] = mfma_steps<F16>(va[j], pb[r][q], acc[q][8 * h + 4 * w + j]);
+                                    }
+                                }
+                            }
+                        }
+                    };
+                    if constexpr (APART) {
+#pragma unroll
+                        for (int r = 0; r < 2; ++r) scores(r, r + 1), refill_k(r), clean(r), soften(r), move(r), values(r), refill_v(r);
+                        return;
+                    }
+                    keys_here();
                     if constexpr (RING) {
 #pragma unroll
                         for (int l = 0; l < CPR / 4; ++l) {
                             const uint32_t at = (k_read ^ (uint32_t)(64 * (l & 3))) + (uint32_t)(256 * (l >> 2));
-                            held[0][l] = *reinterpret_cast<const u32x4*>(place_a + at);
-                            held[1][l] = *reinterpret_cast<const u32x4*>(place_b + at);
+                            held[0][l] = *reinterpret_cast<const u32x4*>(places[0] + at);
+                            held[1][l] = *reinterpret_cast<const u32x4*>(places[1] + at);
                         }
                     }
-#pragma unroll
-                    for (int c = 0; c < 4 * DH; ++c) {
-                        const u32x4 ka = key_operand<KIND>(RING ? held[0] : t[RING ? 0 : 2 * i].k, c), kb = key_operand<KIND>(RING ? held[1] : t[RING ? 0 : 2 * i + 1].k, c);
-#pragma unroll
-                        for (int q = 0; q < QT; ++q) {
-                            s0[q] = mfma_k32<F16>(ka, qb[q][c], s0[q]);
-                            s1[q] = mfma_k32<F16>(kb, qb[q][c], s1[q]);
-                        }
-                    }
-                    float ks8[8], vs8[8];
+                    scores(0, 2);
                     if constexpr (KIND >= 2) {
                         const int first = NARROW ? 16 * odd_cur : 0;
 #pragma unroll
@@ -659,150 +842,16 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
                         }
                     }
                     if constexpr (RING) wait_lds();
-                    refill_k();      // (the keys' registers are free: the loads of NP pairs ahead go out)
-                    // Both steps wholly seen by every column of the tiles (a draft tree's: before the window's first
-                    // position): nothing is asked of a position.
-                    const bool whole = MASK != kMaskSliding && win <= 0 &&
-                                       base_b + SPW <= min(MASK == kMaskTree ? cur.first : cur.first + cur.c_lo + 1, cur.n_keys);
-                    // The lane's scores: its column at positions base + r_pos + i, second + r_pos + i of head r_head. Another
-                    // head's column (a lane that is not `mine`) sees nothing: its scores stay out of the maximum, its
-                    // probabilities become zeros (chosen, not multiplied: the other head's values may be anything).
-                    float x[QT][8], top[QT];
-#pragma unroll
-                    for (int q = 0; q < QT; ++q) {
-#pragma unroll
-                        for (int i = 0; i < 8; ++i) {
-                            const float raw = i < 4 ? s0[q][i & 3] : s1[q][i & 3];
-                            x[q][i] = KIND >= 2 ? raw * (sscale * ks8[i]) : raw;
-                        }
-                        if (!whole) {
-                            const int room = lim[q] - r_pos;      // position n (of the step's first) is visible while n + i <= room
-#pragma unroll
-                            for (int i = 0; i < 8; ++i) {
-                                const int at = (i < 4 ? base : base_b) + (i & 3);
-                                bool vis = at <= room;
-                                if constexpr (MASK != kMaskNone) {
-                                    const int n = at + r_pos;
-                                    if (tree) vis = vis && (n < cur.first || ((anc[q] >> ((n - cur.first) & 63)) & 1ull) != 0);
-                                    if (win > 0) vis = vis && n > cur.first + col[q] - win;
-                                }
-                                x[q][i] = vis ? x[q][i] : -INFINITY;
-                            }
-                        }
-                        float y = __builtin_fmaxf(__builtin_fmaxf(__builtin_fmaxf(x[q][0], x[q][1]), __builtin_fmaxf(x[q][2], x[q][3])),
-                                                  __builtin_fmaxf(__builtin_fmaxf(x[q][4], x[q][5]), __builtin_fmaxf(x[q][6], x[q][7])));
-                        if constexpr (KIND < 2) y *= sscale;      // (positive: -inf stays -inf)
-                        if constexpr (HW > 1) y = mine ? y : -INFINITY;
-                        top[q] = max_across_quarters(y);
-                    }
-                    bool moved[QT], any = false;
-#pragma unroll
-                    for (int q = 0; q < QT; ++q) moved[q] = top[q] > m[q], any = any || moved[q];
-                    if (__builtin_amdgcn_ballot_w64(any) != 0) {
-#pragma unroll
-                        for (int q = 0; q < QT; ++q) {
-                            const float alpha = moved[q] ? exp2_fast(m[q] - top[q]) : 1.0f;
-                            m[q] = moved[q] ? top[q] : m[q];
-                            l[q] *= alpha;
-#pragma unroll
-                            for (int j = 0; j < 8 * DH; ++j) acc[q][j] *= alpha;
-                        }
-                    }
-                    u32x4 pb[QT];
-#pragma unroll
-                    for (int q = 0; q < QT; ++q) {
-                        const float sub = m[q] == -INFINITY ? 0.0f : m[q];
-                        float p[8];
-#pragma unroll
-                        for (int i = 0; i < 8; ++i) p[i] = exp2_fast(KIND >= 2 ? x[q][i] - sub : __builtin_fmaf(x[q][i], sscale, -sub));
-                        const float sum = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
-                        l[q] += HW == 1 || mine ? sum : 0.0f;
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const uint32_t w = KIND >= 2 ? pair16<F16>(p[2 * i] * vs8[2 * i], p[2 * i + 1] * vs8[2 * i + 1]) : pair16<F16>(p[2 * i], p[2 * i + 1]);
-                            pb[q][i] = HW == 1 || mine ? w : 0u;
-                        }
-                    }
+                    refill_k(0), refill_k(1);      // (the keys' places are free: the loads of NP pairs ahead go out)
+                    soften(0);
+                    if constexpr (G == 1) soften(1);
+                    move(0);
                     values_here();
-                    // The row's last steps: what lies past its keys may be anything, and a probability of zero times a NaN is a
-                    // NaN. Such values become zeros.
-                    auto clean = [&](int at, int place) __attribute__((always_inline)) {
-                        if (at + SPW > cur.n_keys) {
-                            if constexpr (RING) {
-                                uint8_t* values = &s_ring[wave][place][HALF];
-                                for (int row = 0; row < 16; ++row) {
-                                    if (at + row % SPW < cur.n_keys) continue;
-                                    uint8_t* to = values + (KIND == 0 ? row : 4 * (row & 3) + (row >> 2)) * ROWB;
-                                    for (int b = lane * 4; b < ROWB; b += 256) *reinterpret_cast<uint32_t*>(to + b) = 0u;
-                                }
-                            } else {
-#pragma unroll
-                                for (int p = 0; p < 4; ++p)
-                                    if (at + r_pos + p >= cur.n_keys) t[RING ? 0 : place].v[p] = u32x4{0, 0, 0, 0};
-                            }
-                        }
-                    };
-                    clean(base, 2 * i), clean(base_b, 2 * i + 1);
-                    // -- values: the lane's dims of the eight rows as four 16-bit pairs, then O^T += V^T P^T
-                    if constexpr (!RING) {      // dims {8 i + j}: a v_perm a pair
-                        const Tile&ta = t[RING ? 0 : 2 * i], &tb = t[RING ? 0 : 2 * i + 1];
-#pragma unroll
-                        for (int w = 0; w < 4; ++w) {
-                            u32x4 lo, hi;
-#pragma unroll
-                            for (int r = 0; r < 2; ++r) {
-                                const Tile& tl = r == 0 ? ta : tb;
-                                lo[2 * r] = __builtin_amdgcn_perm(tl.v[1][w], tl.v[0][w], 0x05040100), lo[2 * r + 1] = __builtin_amdgcn_perm(tl.v[3][w], tl.v[2][w], 0x05040100);
-                                hi[2 * r] = __builtin_amdgcn_perm(tl.v[1][w], tl.v[0][w], 0x07060302), hi[2 * r + 1] = __builtin_amdgcn_perm(tl.v[3][w], tl.v[2][w], 0x07060302);
-                            }
-#pragma unroll
-                            for (int q = 0; q < QT; ++q) {
-                                acc[q][2 * w] = mfma_k32<F16>(lo, pb[q], acc[q][2 * w]);
-                                acc[q][2 * w + 1] = mfma_k32<F16>(hi, pb[q], acc[q][2 * w + 1]);
-                            }
-                        }
-                    } else if constexpr (KIND == 0) {      // dims 16 b + (0 .. 15): transposed by the LDS
-#pragma unroll
-                        for (int b = 0; b < 8 * DH; ++b) {
-                            const uint32_t at = (uint32_t)HALF + t_read + (t_turn ^ (uint32_t)(32 * (b & 7))) + (uint32_t)(256 * (b >> 3));
-                            const u32x2 x = read_transposed(place_a + at), y = read_transposed(place_b + at);
-                            const u32x4 va = {x.x, x.y, y.x, y.y};
-#pragma unroll
-                            for (int q = 0; q < QT; ++q) acc[q][b] = mfma_k32<F16>(va, pb[q], acc[q][b]);
-                        }
-                    } else {      // dims {8 i + j}: codes of adjacent rows side by side, then as 16-bit pairs
-#pragma unroll
-                        for (int h = 0; h < DH; ++h) {
-                            u32x2 v[2][4];
-#pragma unroll
-                            for (int p = 0; p < 4; ++p) {
-                                const uint32_t at = (uint32_t)(HALF + (4 * p + u4) * ROWB + 128 * h + 8 * c16);
-                                v[0][p] = *reinterpret_cast<const u32x2*>(place_a + at), v[1][p] = *reinterpret_cast<const u32x2*>(place_b + at);
-                            }
-#pragma unroll
-                            for (int w = 0; w < 2; ++w) {
-                                u32x4 va[4];
-#pragma unroll
-                                for (int r = 0; r < 2; ++r) {
-                                    // bytes (a0 b0 a1 b1) and (a2 b2 a3 b3): two rows' codes of one dim side by side
-                                    const uint32_t lo01 = __builtin_amdgcn_perm(v[r][1][w], v[r][0][w], 0x05010400), hi01 = __builtin_amdgcn_perm(v[r][1][w], v[r][0][w], 0x07030602);
-                                    const uint32_t lo23 = __builtin_amdgcn_perm(v[r][3][w], v[r][2][w], 0x05010400), hi23 = __builtin_amdgcn_perm(v[r][3][w], v[r][2][w], 0x07030602);
-                                    // (dims 4 w + 0, 1 from the low halves, 2, 3 from the high ones; .x: rows 0, 1; .y: rows 2, 3)
-                                    const u32x2 a01 = codes4_to_pairs<KIND>(lo01), a23 = codes4_to_pairs<KIND>(lo23);
-                                    const u32x2 b01 = codes4_to_pairs<KIND>(hi01), b23 = codes4_to_pairs<KIND>(hi23);
-                                    va[0][2 * r] = a01.x, va[0][2 * r + 1] = a23.x, va[1][2 * r] = a01.y, va[1][2 * r + 1] = a23.y;
-                                    va[2][2 * r] = b01.x, va[2][2 * r + 1] = b23.x, va[3][2 * r] = b01.y, va[3][2 * r + 1] = b23.y;
-                                }
-#pragma unroll
-                                for (int q = 0; q < QT; ++q) {
-#pragma unroll
-                                    for (int j = 0; j < 4; ++j) acc[q][8 * h + 4 * w + j] = mfma_k32<F16>(va[j], pb[q], acc[q][8 * h + 4 * w + j]);
-                                }
-                            }
-                        }
-                    }
+                    clean(0), clean(1);
+                    values(0);
+                    if constexpr (G == 1) move(1), values(1);
                     if constexpr (RING) wait_lds();
-                    refill_v();
+                    refill_v(0), refill_v(1);
                 };
 
                 if (part != part_lo) {
@@ -837,20 +886,20 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
                                      if constexpr (NP == 2) { if (more) wait_dma<NK + NV + NK>(); else if (follows) wait_dma<NK + NV>(); else wait_dma<0>(); }
                                      else { if (more) wait_dma<NK>(); else wait_dma<0>(); }
                                  },
-                                 [&]() __attribute__((always_inline)) { if (more) fetch_k(cur, ahead.s0, 2 * i), fetch_k(cur, ahead.s1, 2 * i + 1); },
-                                 [&]() __attribute__((always_inline)) { if (more) fetch_v(cur, ahead.s0, 2 * i), fetch_v(cur, ahead.s1, 2 * i + 1); });
+                                 [&](int r) __attribute__((always_inline)) { if (more) fetch_k(cur, r == 0 ? ahead.s0 : ahead.s1, 2 * i + r); },
+                                 [&](int r) __attribute__((always_inline)) { if (more) fetch_v(cur, r == 0 ? ahead.s0 : ahead.s1, 2 * i + r); });
                             at[i] = ahead, ++n;
                         }
                     }
                 } else if (at[0].base >= 0) {
                     // In registers the compiler counts the loads: the loop's are unconditional (exact waits), the last pair is peeled.
                     static_assert(RING || NP == 1, "one pair in registers");
-                    const auto none = []() {};
+                    const auto none = [](auto...) {};
                     Pair ahead = pair_no(cur, steps, n);
                     while (ahead.base >= 0) {
                         step(at[0].base, at[0].second, 0, none, none,
-                             [&]() __attribute__((always_inline)) { fetch_k(cur, ahead.s0, 0), fetch_k(cur, ahead.s1, 1); },
-                             [&]() __attribute__((always_inline)) { fetch_v(cur, ahead.s0, 0), fetch_v(cur, ahead.s1, 1); });
+                             [&](int r) __attribute__((always_inline)) { fetch_k(cur, r == 0 ? ahead.s0 : ahead.s1, r); },
+                             [&](int r) __attribute__((always_inline)) { fetch_v(cur, r == 0 ? ahead.s0 : ahead.s1, r); });
                         at[0] = ahead;
                         ahead = pair_no(cur, steps, ++n);
                     }
