@@ -34,7 +34,7 @@
 // own ring in LDS (global_load_lds: no register holds them, a request takes 64 adjacent bytes) and read the operands from
 // there, values transposed by the LDS itself (ds_read_b64_tr_b16). Nothing is shared between wavefronts, so no barrier
 // orders the ring: the waits count loads. Against the same kernels with all rows in registers: 64 rows ~U[1024, 8192], 32
-// / 8 heads x 128, 5 columns BF16 331 -> 303 us; 8 rows of 16,000, 24 / 4 x 256, fp8:row 74 -> 67; one row of 50,000, 56 /
+// / 8 heads x 128, 5 columns BF16 331 -> 284 us; 8 rows of 16,000, 24 / 4 x 256, fp8:row 74 -> 67; one row of 50,000, 56 /
 // 8, 8 columns, INT8 116 -> 98.
 //
 // Row-exactness: position n is always read in the same step of the same pair of the same wavefront of its unit (pairs do
@@ -201,7 +201,8 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
     // probability, where it moves the maximum, is then 1, which 16 bits hold, and one maximum for both leaves the first
     // step's below 1 (16 rows ~U[1024, 8192], FP32 results, from 64 bits: BF16 1.237e-3 in place of 1.253e-3, 256-wide heads
     // 1.171e-3 in place of 1.215e-3, FP8 1.364e-3 in place of 1.372e-3; row-scaled FP8 and INT8 1.609e-3 and 1.589e-3
-    // either way). One maximum is the cheaper: 5 columns of 64 such rows BF16 289 us, each its own 303; FP8 174 and 207.
+    // either way). One maximum is the cheaper (5 columns of 64 such rows, the queries' signs then still set here, see lane_values: BF16 289
+    // us, each its own 303; FP8 174 and 207).
     constexpr int G = KIND >= 2 ? 2 : 1;
     constexpr int FW = RING ? 64 : D;        // output dims folded at a time
     constexpr int FG = FW / 64;              // groups of four of them a thread folds: dims 64 i + 4 (tid % 16) .. + 3 of column tid / 16
@@ -544,17 +545,12 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
             for (int h = 0; h < HW; ++h) vm_nxt[h] = a.hm ? a.hm[a.hkv + un.kvh0 + h] : a.v_mult;
         }
     };
+    // (Nothing is done to the queries here: they are the youngest loads, and a wait on them waits for all rows requested
+    // before. A negative scale's sign set in them: 64 rows ~U[1024, 8192], 5 columns BF16 303 us, 284 so; 16 rows of 4
+    // columns, 24 / 4 x 256, 113 and 101; 64 rows of 24 / 2 x 256, one column, 156 and 147.)
     auto lane_values = [&](const Unit& un) __attribute__((always_inline)) {
         const int odd = odd_of(un);
         if constexpr (KIND == 1) sscale = a.sscale * (a.hm ? a.hm[NARROW ? 2 * (un.kvh0 + hsel) + odd : un.kvh0 + hsel] : a.k_mult);
-        // (16-bit and FP8 pages: the scale rides on the exponent's multiply-add and on the maximum, so it is kept positive,
-        // its sign in the queries, and above zero: a hidden position's score of -inf times it stays -inf)
-        uint32_t flip = 0u;
-        if constexpr (KIND < 2) {
-            const float given = KIND == 1 ? sscale : a.sscale;
-            flip = given < 0.0f ? 0x80008000u : 0u;
-            sscale = __builtin_fmaxf(__builtin_fabsf(given), 0x1p-126f);
-        }
 #pragma unroll
         for (int q = 0; q < QT; ++q) {
             const int jr = un.j0 + q * CPH + c16 % CPH;
@@ -574,7 +570,6 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
                 } else {
                     if (live) qb[q][c] = *reinterpret_cast<const u32x4*>(row + dim * 2);
                 }
-                if constexpr (KIND < 2) qb[q][c] ^= u32x4{flip, flip, flip, flip};
             }
         }
     };

@@ -46,6 +46,22 @@ def test_scales_of_any_sign(kind, scale):
     close(out, cache.want(q, 0, 698, 2, scale=scale)[0])
 
 
+@pytest.mark.parametrize("kind,hkv,d", [("bf16", 2, 128), ("bf16", 3, 128), ("fp16", 2, 256), ("fp8", 2, 128), ("fp8", 4, 64), ("fp8:row", 2, 128), ("int8", 2, 128)])
+@pytest.mark.parametrize("fused", [False, True])
+def test_a_scale_that_is_no_number_shows(kind, hkv, d, fused):
+    cache = Cache(kind, hkv, d, d, 16, [700])
+    q = rand_q(2, 4 * hkv, d, 69)
+    assert bool(cache.attend(q, [0], [0], [698], 2, scale=float("nan"), fused=fused).isnan().all())
+    if kind == "fp8":      # a head's multiplier: its own query heads, and no others
+        want = cache.attend(q, [0], [0], [698], 2, fused=fused)
+        per_head = torch.tensor([[0.02] * hkv, [0.03] * hkv])
+        per_head[0, 1] = float("nan")
+        cache.multipliers = per_head
+        out = cache.attend(q, [0], [0], [698], 2, fused=fused)
+        assert bool(out[:, 4:8].isnan().all())
+        assert torch.equal(out[:, :4], want[:, :4]) and torch.equal(out[:, 8:], want[:, 8:])
+
+
 @pytest.mark.parametrize("kind", ["fp8", "fp8:row", "int8"])
 @pytest.mark.parametrize("tree", [False, True])
 def test_three_tiles_of_8_bit_pages_in_a_launch_that_fills_the_card(kind, tree):
