@@ -449,7 +449,7 @@ static int launch_attend_checked(const crit_pkv_attend_params* p, hipStream_t st
         const int64_t apart = (int64_t)p->n_rows * (p->kv_heads / a.heads_per_wave) * a.tiles * p->partitions;
         if (a.tiles >= 3 || apart > (int64_t)compute_units() * 2) {
             const bool full = !p->counts || p->window_tokens == (int64_t)p->n_rows * p->columns;
-            a.query_tiles = window_tiles_8bit(a.tiles, full, (int64_t)p->n_rows * (p->kv_heads / a.heads_per_wave) * gy, compute_units());
+            a.query_tiles = window_tiles_8bit(p->kind >= 2, a.tiles, full, (int64_t)p->n_rows * (p->kv_heads / a.heads_per_wave) * gy, compute_units());
             a.tiles = (a.tiles + a.query_tiles - 1) / a.query_tiles;
         }
     }

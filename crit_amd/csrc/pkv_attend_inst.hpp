@@ -141,11 +141,14 @@ static int launch_mfma_masked(const AttendArgs& u, bool fused, dim3 grid, hipStr
             else if (pair) PKV_MFMA(2, false, MASK, 1, 2);
             else PKV_MFMA(1, false, MASK, 1, 2);
             return hip_code(hipGetLastError());
-        case 3:      // split launches of 128-wide heads, one workgroup a compute unit
-            if (u.dk == 256) return CRIT_PKV_E_GEOMETRY;
-            if (pair) PKV_MFMA(2, false, MASK, 1, 3);
-            else PKV_MFMA(1, false, MASK, 1, 3);
-            return hip_code(hipGetLastError());
+        case 3:      // split launches of 128-wide heads, one workgroup a compute unit, over 16-bit pages and scaled rows
+            if constexpr (KIND != 1) {
+                if (u.dk == 256) return CRIT_PKV_E_GEOMETRY;
+                if (pair) PKV_MFMA(2, false, MASK, 1, 3);
+                else PKV_MFMA(1, false, MASK, 1, 3);
+                return hip_code(hipGetLastError());
+            }
+            break;
         case 4:      // ... over 16-bit pages
             if constexpr (KIND == 0) {
                 if (u.dk == 256) return CRIT_PKV_E_GEOMETRY;

@@ -174,9 +174,9 @@ struct MfmaShape {
 // the registers, are multiplied with each tile's queries and probabilities in turn, every tile with its own softmax
 // state and accumulators, so a tile's bits are what they are alone and the rows are read once for QT tiles instead of
 // once a tile. More than one tile takes the registers of a second workgroup on the compute unit (one stays). Built for
-// four or three tiles (or a window's two) of 128-wide heads over 16-bit pages and two or three over 8-bit pages (pairs still fit two
-// workgroups a compute unit) or of 256-wide heads, where it measured faster (64 rows ~U[1024, 8192] of 32 / 8 heads, 8
-// columns: 676 -> 480 us, FP8 376 -> 224); four tiles of 8-bit pages measured slower.
+// four or three tiles (or a window's two) of 128-wide heads over 16-bit pages, two over 8-bit pages and three over scaled
+// rows (pairs still fit two workgroups a compute unit) or of 256-wide heads, where it measured faster (64 rows ~U[1024,
+// 8192] of 32 / 8 heads, 8 columns: 676 -> 480 us, FP8 376 -> 224); four tiles of 8-bit pages measured slower.
 // NARROW: 64-wide heads, read as 128-wide ones. Two adjacent KV heads' rows of a position are 128 contiguous values,
 // which is what a 128-wide head's row is: the launcher hands the kernel half the KV heads at twice the width and GQA
 // groups twice as large (a group's first half the query heads of the even KV head, its second half the odd one's: the

@@ -77,13 +77,17 @@ PKV_SPLIT_FN int window_tiles_16bit(int64_t tiles, bool full, int64_t places, in
     return threes == 1 || full || (threes - 1) * threes * places <= 2 * units ? 3 : 4;
 }
 
-// The same over 8-bit pages, for windows of three tiles or more: two tiles a workgroup, two workgroups a compute unit; three
-// in one workgroup (one a compute unit) where that holds a row whole and the launch has more of them than two a compute
-// unit: a row is then read and converted once instead of twice. 64 rows ~U[1024, 8192], 32 / 8 heads x 128, 5 columns: FP8
-// 209 -> 172 us, INT8 222 -> 195. Small launches miss the second workgroup (3 rows of up to 4,000: 38 us in twos, 49 in
-// threes), and four tiles in one wavefront are too long a step (8 columns of one row of 50,000, 56 / 8 heads, 99 and 126).
-PKV_SPLIT_FN int window_tiles_8bit(int64_t tiles, bool full, int64_t places, int64_t units) {
-    return tiles == 3 && full && places > 2 * units ? 3 : 2;
+// The same over 8-bit pages, for windows of three tiles or more: two tiles a workgroup, two workgroups a compute unit. Pages of
+// scaled rows (a step pair has one maximum there, half the softmax and value products): three in one workgroup, one a
+// compute unit, where that holds a row whole and the tables have room for more of them than two a compute unit: a row is
+// then read and converted once instead of twice. 64 rows ~U[1024, 8192], 32 / 8 heads x 128, 5 columns: INT8 217 -> 189 us,
+// fp8:row 216 -> 177; 16 rows of 4,600 in tables of 8,192 pages 74 -> 62. Small launches miss the second workgroup (3 rows
+// of up to 4,000 in tables of their own length: 38 us in twos, 49 in threes; in tables of 8,192 pages, which the rule cannot
+// tell from long rows, 53 and 57), and four tiles in one wavefront are too long a step (8 columns of one row of 50,000, 56
+// / 8 heads, 99 and 126). FP8 with its multipliers gains nothing by threes (64 rows 203 and 200, 32 rows 116 and 118, 3
+// rows in tables of 8,192 pages 51 and 60, 32 rows of 700 there 37 and 43).
+PKV_SPLIT_FN int window_tiles_8bit(bool scaled_rows, int64_t tiles, bool full, int64_t places, int64_t units) {
+    return scaled_rows && tiles == 3 && full && places > 2 * units ? 3 : 2;
 }
 
 }   // namespace pkv

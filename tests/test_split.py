@@ -20,6 +20,7 @@ def split(tmp_path_factory):
 extern "C" int xcds_log2(int64_t pairs, int64_t tiles, int64_t units, int64_t held) { return pkv::xcds_of_pair_log2(pairs, tiles, units, held); }
 extern "C" int64_t workgroups(int64_t pairs, int64_t tiles, int l) { return pkv::dealt_workgroups(pairs, tiles, l); }
 extern "C" int window_tiles(int64_t tiles, int full, int64_t places, int64_t units) { return pkv::window_tiles_16bit(tiles, full != 0, places, units); }
+extern "C" int window_tiles_8bit(int scaled, int64_t tiles, int full, int64_t places, int64_t units) { return pkv::window_tiles_8bit(scaled != 0, tiles, full != 0, places, units); }
 extern "C" void deal(int64_t pairs, int64_t tiles, int l, int* pair, int* tile) {
     const int64_t n = pkv::dealt_workgroups(pairs, tiles, l);
     for (int64_t w = 0; w < n; ++w) {
@@ -34,6 +35,7 @@ extern "C" void deal(int64_t pairs, int64_t tiles, int l, int* pair, int* tile) 
     lib = ctypes.CDLL(out)
     lib.xcds_log2.argtypes, lib.workgroups.argtypes = [ctypes.c_int64] * 4, [ctypes.c_int64, ctypes.c_int64, ctypes.c_int]
     lib.window_tiles.argtypes = [ctypes.c_int64, ctypes.c_int, ctypes.c_int64, ctypes.c_int64]
+    lib.window_tiles_8bit.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int64, ctypes.c_int64]
     lib.workgroups.restype = ctypes.c_int64
     lib.deal.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
     return lib
@@ -104,3 +106,13 @@ def test_a_row_of_four_tiles_is_not_read_twice_in_a_large_launch(split):
     assert [split.window_tiles(t, 0, 4096, 256) for t in (3, 4, 5, 6, 7, 8, 9, 10)] == [3, 4, 4, 4, 4, 4, 4, 4]
     # one row of 4 head pairs and 64 partitions: its second workgroups run beside its first
     assert [split.window_tiles(t, 0, 256, 256) for t in (5, 6, 9)] == [3, 3, 4] and split.window_tiles(9, 0, 42, 256) == 3
+
+
+def test_8_bit_windows_of_three_tiles(split):
+    # three in one workgroup only where they are a whole full row of scaled rows in a launch past two workgroups a compute unit;
+    # FP8 with its multipliers goes in twos whatever the tables have room for (3 rows in tables of 8,192 pages: 1,536 places)
+    for tiles in range(2, 10):
+        for full in (0, 1):
+            for places in (1, 511, 512, 513, 1536, 1 << 20):
+                assert split.window_tiles_8bit(0, tiles, full, places, 256) == 2
+                assert split.window_tiles_8bit(1, tiles, full, places, 256) == (3 if tiles == 3 and full and places > 512 else 2)
