@@ -14,20 +14,19 @@ int launch_attend_fp8(const AttendArgs& a, int lpr, int qr, bool fused, bool pag
 int launch_attend_fp8row(const AttendArgs& a, int lpr, int qr, bool fused, bool page16, dim3 grid, hipStream_t stream);
 int launch_attend_int8(const AttendArgs& a, int lpr, int qr, bool fused, bool page16, dim3 grid, hipStream_t stream);
 
-// One wavefront per (column, head, row): folds the partitions that hold the column's positions, in order.
 // Lane `at`'s value of x (at: the same in every lane).
 PKV_DEV float lane_value(float x, int at) { return u2f((uint32_t)__builtin_amdgcn_readlane((int)f2u(x), at)); }
 
-// MANY: launches of as many wavefronts as the card holds at once of the other form, or more, whose batches of 32 partitions take 160
-// registers: batches of 8, three times the wavefronts (10,240 of up to 17 partitions: 18.7 -> 13.3 us).
-template <int DV, bool MANY>
-__global__ __launch_bounds__(64) void merge_kernel(AttendArgs a) {
-    constexpr int EPL = DV < 64 ? 1 : DV / 64;      // (value rows narrower than a wavefront: the lanes past them idle)
-    const int c = blockIdx.x, head = blockIdx.y, r = blockIdx.z;
-    const int lane = DV < 64 ? min((int)threadIdx.x, DV - 1) : (int)threadIdx.x;
+// A (column, head, row) triple's merge: how many partitions hold the column's positions (-1: no such column), and the place of
+// their first state.
+struct Merge {
+    int nb;
+    int64_t at;
+};
+PKV_DEV Merge merge_of(const AttendArgs& a, int c, int head, int r) {
     int count = a.columns;
     if (a.counts) count = min(a.counts[r], a.columns);
-    if (c >= count) return;
+    if (c >= count) return Merge{-1, 0};
     int64_t first = a.firsts[r];
     first = first < 0 ? 0 : (first > (int64_t)0x3fffffff ? (int64_t)0x3fffffff : first);
     const int64_t seen = min(first + c + 1, (int64_t)a.max_keys);
@@ -35,7 +34,16 @@ __global__ __launch_bounds__(64) void merge_kernel(AttendArgs a) {
     const uint32_t run = a.blocks ? (uint32_t)a.listed_keys : (uint32_t)seen;
     const int nb = (int)min((uint32_t)a.parts, (run + (uint32_t)a.piece - 1u) / (uint32_t)a.piece);
     const int64_t prow = a.offsets ? (int64_t)(a.offsets[r] - a.offsets[0]) : (int64_t)r * a.columns;
-    const int64_t at = ((prow + c) * a.hq + head) * a.parts;
+    return Merge{nb, ((prow + c) * a.hq + head) * a.parts};
+}
+
+// One wavefront's fold of a triple's partitions, in order, and its result. MANY: batches of 8 in place of 32.
+template <int DV, bool MANY>
+PKV_DEV void merge_by_wavefront(const AttendArgs& a, int c, int head, int r, const Merge& m) {
+    constexpr int EPL = DV < 64 ? 1 : DV / 64;      // (value rows narrower than a wavefront: the lanes past them idle)
+    const int lane = DV < 64 ? min((int)threadIdx.x, DV - 1) : (int)threadIdx.x;
+    const int nb = m.nb;
+    const int64_t at = m.at;
     float M = -INFINITY, L = 0.0f, A[EPL];
 #pragma unroll
     for (int e = 0; e < EPL; ++e) A[e] = 0.0f;
@@ -138,11 +146,24 @@ __global__ __launch_bounds__(64) void merge_kernel(AttendArgs a) {
     if (a.lse && threadIdx.x == 0) a.lse[token * a.hq + head] = L != 0.0f ? __builtin_fmaf(M, kLn2, __logf(L)) : -INFINITY;
 }
 
-// The same fold for few (column, head, row) triples of many partitions (long rows): a workgroup each. One wavefront would
-// fetch its partials a batch after another, at a round trip to memory a batch (200,000 positions in splits of 1,024, 40
-// heads: 15.3 us in 40 wavefronts, 10.7 here). Here 256 threads bring up to a hundred kilobytes of them into LDS at once,
+// One wavefront per (column, head, row).
+// MANY: launches of as many wavefronts as the card holds at once of the other form, or more, whose batches of 32 partitions take 160
+// registers: batches of 8, three times the wavefronts (10,240 of up to 17 partitions: 18.7 -> 13.3 us).
+template <int DV, bool MANY>
+__global__ __launch_bounds__(64) void merge_kernel(AttendArgs a) {
+    const int c = blockIdx.x, head = blockIdx.y, r = blockIdx.z;
+    const Merge m = merge_of(a, c, head, r);
+    if (m.nb >= 0) merge_by_wavefront<DV, MANY>(a, c, head, r, m);
+}
+
+// The same for few triples in tables with room for many partitions: a workgroup a triple. Which way is the row's own: what the
+// tables have room for says nothing of its length. Up to kFewPartitions, one wavefront all the same (3 rows of up to 4,000
+// in tables of 8,192 pages, 32 / 8 heads: 29.7 us a call by the workgroup, 28.3 so; one of 16,000 23.9 and 23.1). More, and
+// one wavefront would fetch its partials a batch after another, at a round trip to memory a batch (200,000 positions in
+// splits of 1,024, 40 heads: 15.3 us in 40 wavefronts, 10.7 here): 256 threads bring up to 128 KB of them into LDS at once,
 // make every partition's factors (a prefix maximum over the threads, exact in any order), and a thread a value dim folds
-// them in order: the operations of merge_kernel on the same values.
+// them in order: the operations of merge_by_wavefront on the same values.
+constexpr int kFewPartitions = 32;      // what a wavefront loads at once (256-wide values: in two batches)
 template <int DV>
 __global__ __launch_bounds__(256) void merge_long_kernel(AttendArgs a) {
     typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));      // (four floats of a workspace that is any floats)
@@ -152,16 +173,13 @@ __global__ __launch_bounds__(256) void merge_long_kernel(AttendArgs a) {
     __shared__ float s_top[4];
     const int c = blockIdx.x, head = blockIdx.y, r = blockIdx.z;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    int count = a.columns;
-    if (a.counts) count = min(a.counts[r], a.columns);
-    if (c >= count) return;
-    int64_t first = a.firsts[r];
-    first = first < 0 ? 0 : (first > (int64_t)0x3fffffff ? (int64_t)0x3fffffff : first);
-    const int64_t seen = min(first + c + 1, (int64_t)a.max_keys);
-    const uint32_t run = a.blocks ? (uint32_t)a.listed_keys : (uint32_t)seen;
-    const int nb = (int)min((uint32_t)a.parts, (run + (uint32_t)a.piece - 1u) / (uint32_t)a.piece);
-    const int64_t prow = a.offsets ? (int64_t)(a.offsets[r] - a.offsets[0]) : (int64_t)r * a.columns;
-    const int64_t at = ((prow + c) * a.hq + head) * a.parts;
+    const Merge m = merge_of(a, c, head, r);
+    const int nb = m.nb;
+    const int64_t at = m.at;
+    if (nb <= kFewPartitions) {
+        if (nb >= 0 && __builtin_amdgcn_readfirstlane(wave) == 0) merge_by_wavefront<DV, false>(a, c, head, r, m);
+        return;
+    }
     float M = -INFINITY, L = 0.0f, A = 0.0f;
     for (int b0 = 0; b0 < nb; b0 += CH) {
         const int n = min(CH, nb - b0);
@@ -486,10 +504,10 @@ static int launch_attend_checked(const crit_pkv_attend_params* p, hipStream_t st
     if (rc || p->phases == 1) return rc;
     const dim3 mgrid((unsigned)p->columns, (unsigned)p->heads, (unsigned)p->n_rows);
     // Which merge: by the wavefronts of the launch and the partitions a row may have (the bits are the same). Up to a
-    // triple a compute unit of more than 32 partitions, a workgroup each; 8 wavefronts a compute unit (what the card holds of
-    // the form with batches of 32) or more, batches of 8.
+    // triple a compute unit in tables with room for more than kFewPartitions, a workgroup each, which looks at its row; 8
+    // wavefronts a compute unit (what the card holds of the form with batches of 32) or more, batches of 8.
     const int64_t triples = (int64_t)p->columns * p->heads * p->n_rows, units = compute_units();
-    const bool long_rows = triples <= units && gy > 32, many = triples >= 8 * units;
+    const bool long_rows = triples <= units && gy > kFewPartitions, many = triples >= 8 * units;
 #define PKV_MERGE(W)                                                                                                        \
     case W:                                                                                                                 \
         if (many) hipLaunchKernelGGL((merge_kernel<W, true>), mgrid, dim3(64), 0, stream, a);                               \

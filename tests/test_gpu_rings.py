@@ -94,6 +94,30 @@ def test_merges_of_long_rows_and_of_many_wavefronts(kind, hkv, g, d, n, parts, r
     close(run()[:1], cache.want(q[:1], 0, n - 1, 1)[0]) if with_sinks is None else None
 
 
+@pytest.mark.parametrize("hkv,g,d", [(2, 4, 128), (1, 4, 256), (2, 4, 64)])
+def test_merges_of_short_rows_in_wide_tables(hkv, g, d):
+    # tables with room for 100 partitions: rows of up to 32 go by one wavefront, others by the workgroup, both beside each other
+    lengths = [1, 16 * 8, 16 * 8 + 1, 16 * 32, 16 * 32 + 1, 16 * 60 - 5]
+    cache = Cache("bf16", hkv, d, d, 16, lengths)
+    q = rand_q(2 * len(lengths), hkv * g, d, 71)
+    sinks = torch.linspace(-2, 2, hkv * g, device=dev)
+    rows, starts, firsts = list(range(6)), [2 * r for r in range(6)], [max(n - 2, 0) for n in lengths]
+    counts = torch.tensor([min(n, 2) for n in lengths], dtype=torch.int32, device=dev)
+    narrow = cache.tables
+    for with_sinks in (None, sinks):
+        lse, same = torch.empty(12, hkv * g, device=dev), torch.empty(12, hkv * g, device=dev)
+        cache.tables = torch.cat([narrow, narrow[:, :1].expand(-1, 100 - narrow.shape[1])], 1).contiguous()
+        out = cache.attend(q, rows, starts, firsts, 2, counts=counts, partitions=100, piece=16, sinks=with_sinks, lse=lse)
+        fused = cache.attend(q, rows, starts, firsts, 2, counts=counts, partitions=100, piece=16, sinks=with_sinks, lse=same, fused=True)
+        for r, n in enumerate(lengths):
+            at = slice(2 * r, 2 * r + min(n, 2))
+            assert torch.equal(out[at], fused[at]) and torch.equal(lse[at], same[at]), r
+            if with_sinks is None:
+                want, want_lse = cache.want(q[at], r, firsts[r], min(n, 2))
+                close(out[at], want, msg=str(r))
+                torch.testing.assert_close(lse[at].double().cpu(), want_lse, atol=1e-3, rtol=1e-4, msg=str(r))
+
+
 def test_a_workspace_that_starts_on_any_float():
     pk = kernels()
     cache = Cache("int8", 2, 128, 128, 16, [900, 3000])
