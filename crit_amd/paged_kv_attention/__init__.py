@@ -359,9 +359,10 @@ def workspace_floats(tokens, heads, partitions, value_dim):
 
 
 def _workspace(device, tokens, heads, parts, dv, given=None):
-    """The addresses of a split launch's partial outputs, maxima and sums, one behind another in the caller's FP32
-    workspace, or in the one the current owner holds on the device. (Addresses: three views of the workspace were a fifth
-    of a small launch's time on the host.)"""
+    """The memory of a split launch's partials, and the addresses of its outputs, maxima and sums, one behind another in the
+    caller's FP32 workspace or in the one the current owner holds on the device. The caller keeps the first until its
+    launch is queued: release() on another thread may drop the owner's own hold before. (Addresses: three views of the
+    workspace were a fifth of a small launch's time on the host.)"""
     states = tokens * heads * parts
     floats = states * (dv + 2)
     if given is None:
@@ -371,7 +372,7 @@ def _workspace(device, tokens, heads, parts, dv, given=None):
         raise ValueError(f"workspace: {floats} contiguous FP32 floats for this launch (workspace_floats()), "
                          f"{given.numel()} given")
     base = given.data_ptr()
-    return base, base + 4 * states * dv, base + 4 * states * (dv + 1)
+    return given, base, base + 4 * states * dv, base + 4 * states * (dv + 1)
 
 
 # -- writes ----------------------------------------------------------------------------------------------------------------
@@ -647,7 +648,7 @@ def attend(q, key_pages, value_pages, kind, tables, rows, starts, firsts, column
     if fused or static:
         po = pm = pl = None
     else:
-        po, pm, pl = _workspace(device, partial_rows, hq, parts, dv, workspace)
+        held, po, pm, pl = _workspace(device, partial_rows, hq, parts, dv, workspace)      # (`held` until the launch is queued)
     if out is None:
         out = torch.empty(T, hq, dv, dtype=q.dtype, device=device)
     out_dtype, out_step = _DTYPE.get(out.dtype), out.stride()

@@ -48,3 +48,18 @@ def test_the_split_launchs_order_knobs_follow_the_rule_or_the_engines_tuning():
         assert pk.partitions("cpu", 4, "bf16", 128, 128) == 16
     finally:
         pk._crit_tuning = None
+
+
+def test_a_launchs_partials_outlive_their_owners_release(monkeypatch):
+    # another thread's release() between a call's look at its workspace and its launch: the memory stays the call's
+    import gc
+    import weakref
+    import torch
+    import crit_amd.paged_kv_attention as pk
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    with pk.owner("gone"):
+        parts = pk._workspace(torch.device("cpu", 0), 2, 4, 3, 16)
+    memory = weakref.ref(pk._holdings[(0, "gone")].partials)
+    pk.release("gone")
+    gc.collect()
+    assert memory() is not None and parts[1:] == (memory().data_ptr(), memory().data_ptr() + 4 * 24 * 16, memory().data_ptr() + 4 * 24 * 17)
