@@ -89,9 +89,16 @@ def test_merges_of_long_rows_and_of_many_wavefronts(kind, hkv, g, d, n, parts, r
     for with_sinks in (None, sinks):
         lse, fused_lse = torch.empty(rows, hkv * g, device=dev), torch.empty(rows, hkv * g, device=dev)
         run = lambda **kw: cache.attend(q, [0] * rows, list(range(rows)), [n - 1] * rows, 1, partitions=parts, piece=16, sinks=with_sinks, **kw)
-        assert torch.equal(run(lse=lse), run(lse=fused_lse, fused=True))
+        out = run(lse=lse)
+        assert torch.equal(out, run(lse=fused_lse, fused=True))
         assert torch.equal(lse, fused_lse)
-    close(run()[:1], cache.want(q[:1], 0, n - 1, 1)[0]) if with_sinks is None else None
+        for r in {0, rows - 1}:
+            want, want_lse = cache.want(q[r:r + 1], 0, n - 1, 1)
+            if with_sinks is not None:      # a logit more in the sum, with no value
+                with_sink = torch.logaddexp(want_lse, sinks.double().cpu())
+                want, want_lse = want * torch.exp(want_lse - with_sink)[..., None], with_sink
+            close(out[r:r + 1], want, msg=str(r))
+            torch.testing.assert_close(lse[r:r + 1].double().cpu(), want_lse, atol=1e-3, rtol=1e-4, msg=str(r))
 
 
 @pytest.mark.parametrize("hkv,g,d", [(2, 4, 128), (1, 4, 256), (2, 4, 64)])
