@@ -64,17 +64,25 @@ def test_a_scale_that_is_no_number_shows(kind, hkv, d, fused):
 
 @pytest.mark.parametrize("kind", ["fp8", "fp8:row", "int8"])
 @pytest.mark.parametrize("tree", [False, True])
-def test_three_tiles_of_8_bit_pages_in_a_launch_that_fills_the_card(kind, tree):
-    rows, columns = 130, 5      # 130 rows of 4 pairs of heads: more than two a compute unit
+@pytest.mark.parametrize("sliding", [0, 33])
+@pytest.mark.parametrize("hkv,columns", [(8, 5), (8, 6), (3, 11), (3, 12)])
+def test_three_tiles_of_8_bit_pages_in_a_launch_that_fills_the_card(kind, tree, sliding, hkv, columns):
+    # 180 rows of 4 pairs of heads (tiles of 8 rows) or of 3 heads (of 16): more than two a compute unit. The rows' columns as
+    # the caller leaves them unsaid, and as a verify round says them: counts, and partial rows packed by their offsets
+    rows, g = 180, 4
     lengths = [columns + 1 + (11 * r) % 90 for r in range(rows)]
-    cache = Cache(kind, 8, 128, 128, 16, lengths)
-    q = rand_q(rows * columns, 32, 128, 63)
+    cache = Cache(kind, hkv, 128, 128, 16, lengths)
+    q = rand_q(rows * columns, hkv * g, 128, 63)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)
     starts, firsts = [columns * r for r in range(rows)], [n - columns for n in lengths]
-    parents = torch.tensor([-1, 0, 0, 1, 3] * rows, dtype=torch.int32, device=dev) if tree else None
-    out = cache.attend(q, list(range(rows)), starts, firsts, columns, parents=parents)
-    assert torch.equal(out, cache.attend(q, list(range(rows)), starts, firsts, columns, parents=parents, fused=True))
-    for r in (0, 7, 129):
-        want, _ = cache.want(q[starts[r]:starts[r] + columns], r, firsts[r], columns, parents=[-1, 0, 0, 1, 3] if tree else None)
+    links = [-1, 0, 0, 1, 3, 2, 5, 4, 4, 8, 9, 6][:columns] if tree else None
+    parents = i32(links * rows) if tree else None
+    run = lambda **kw: cache.attend(q, list(range(rows)), starts, firsts, columns, parents=parents, sliding=sliding, **kw)
+    out = run()
+    assert torch.equal(out, run(fused=True))
+    assert torch.equal(out, run(counts=i32([columns] * rows), offsets=i32(starts), tokens=rows * columns))
+    for r in (0, 7, 179):
+        want, _ = cache.want(q[starts[r]:starts[r] + columns], r, firsts[r], columns, sliding=sliding, parents=links)
         close(out[starts[r]:starts[r] + columns], want, msg=str(r))
 
 
