@@ -467,7 +467,9 @@ PKV_DEV uint32_t wave_max(uint32_t x) {
     return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
-constexpr int kShortList = 512;      // keys of one bin that are ranked against each other
+// Keys of one bin that are ranked against each other, one a lane (the wavefronts share the comparisons; one wavefront's own loop
+// over 64 keys was 1.6 us where a pass over a digit is 0.7).
+constexpr int kShortList = 64;
 
 template <int LEVEL, int EPT>
 __global__ __launch_bounds__(1024) void index_topk_runs_kernel(TopkArgs a) {
@@ -475,12 +477,22 @@ __global__ __launch_bounds__(1024) void index_topk_runs_kernel(TopkArgs a) {
     // different bins meet in different banks, and the scan reads a thread's bins as one word or two, no two lanes in a
     // bank), the copies 16 words out of step, so that a bin's four copies are four banks too.
     constexpr int COPIES = 4, COPY_WORDS = 2048 + 16;
+    // Whose range the digits divide. The whole keys' from the top (11, 11 and 10 bits): an instruction an element, and two digits
+    // for most rows, after which a handful of keys are left. Or the row's own, 2,048 bins over the bits below the highest that
+    // differs between its smallest and largest key: two barriers and a few instructions an element more, and one digit where
+    // the scores have one sign (such a row lies in a few dozen bins of the whole key, where its atomics meet). The latter in
+    // the slices of long rows and their candidates, of up to 16 elements a thread, where its registers leave two workgroups
+    // a compute unit. k = 2,048, us by three digits always / by the row's own range always and up to 512 keys ranked by
+    // comparison / so; scores around zero: a row of 8,192 8.1 / 13.7 / 7.9, of 50,000 20.6 / 26.2 / 20.1, 1,024 rows of 30,000
+    // 58 / 91 / 57, 64 of 50,000 22.3 / 31.9 / 22.5; of one sign 8.7 / 7.4 / 8.4, 22.3 / 18.7 / 18.2, 64.5 / 71.3 / 62.2, 23.8 /
+    // 20.6 / 19.8.
+    constexpr bool RANGE = LEVEL == 1 ? EPT <= 16 : LEVEL == 2 && EPT <= 12;
     __shared__ __align__(16) unsigned s_hist[COPIES * COPY_WORDS];
     __shared__ __align__(16) unsigned s_wave[16];
     __shared__ unsigned s_pick[3];
     __shared__ unsigned s_range[2][16];
-    __shared__ unsigned s_count;
-    __shared__ __align__(16) uint32_t s_list[kShortList];
+    __shared__ unsigned s_count, s_rank[kShortList];
+    __shared__ uint32_t s_list[kShortList];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int t = blockIdx.x, part = LEVEL == 1 ? blockIdx.y : 0;
     const int end = min(max(a.ends[t], 0), a.n);
@@ -553,10 +565,9 @@ __global__ __launch_bounds__(1024) void index_topk_runs_kernel(TopkArgs a) {
     unsigned want = 0u;               // of the keys equal to the k-th, the `want` first are taken
     if (!all) {
         want = (unsigned)k;
-        // A pass: the keys by their digit `of(key)`, below `bins`, where `in(key)` says; s_pick: the bin that holds the
+        // A pass: the keys by their digit `of(key)`, below 2,048, where `in(key)` says; s_pick: the bin that holds the
         // want-th of them from the top, the want that is left for that bin, the bin's keys.
-        auto pass = [&](auto bins_c, auto&& in, auto&& of) __attribute__((always_inline)) {
-            constexpr int bins = decltype(bins_c)::value;
+        auto pass = [&](auto&& in, auto&& of) __attribute__((always_inline)) {
             for (int i = tid; i < COPIES * COPY_WORDS / 4; i += 1024) reinterpret_cast<u32x4*>(s_hist)[i] = u32x4{0u, 0u, 0u, 0u};
             lds_barrier();
             if (mine) {
@@ -567,24 +578,15 @@ __global__ __launch_bounds__(1024) void index_topk_runs_kernel(TopkArgs a) {
                 }
             }
             lds_barrier();
-            // thread tid: the bins per * tid upwards (per of them); a scan of the counts from bin 0 up, and what lies
-            // above a bin is the total less the scan up to it
-            constexpr int per = bins / 1024;
-            unsigned h[per], sum = 0u;
-#pragma unroll
-            for (int i = 0; i < per; ++i) h[i] = 0u;
+            // thread tid: bins 2 tid and 2 tid + 1; a scan of the counts from bin 0 up, and what lies above a bin is the
+            // total less the scan up to it
+            unsigned h[2] = {0u, 0u};
 #pragma unroll
             for (int c = 0; c < COPIES; ++c) {
-                const unsigned* mine_of = s_hist + c * COPY_WORDS + per * tid;
-                if constexpr (per == 2) {
-                    const u32x2 v = *reinterpret_cast<const u32x2*>(mine_of);
-                    h[0] += v.x, h[1] += v.y;
-                } else {
-                    h[0] += mine_of[0];
-                }
+                const u32x2 v = *reinterpret_cast<const u32x2*>(s_hist + c * COPY_WORDS + 2 * tid);
+                h[0] += v.x, h[1] += v.y;
             }
-#pragma unroll
-            for (int i = 0; i < per; ++i) sum += h[i];
+            const unsigned sum = h[0] + h[1];
             unsigned incl = wave_inclusive_sum(sum);
             if (lane == 63) s_wave[wave] = incl;
             lds_barrier();
@@ -592,59 +594,78 @@ __global__ __launch_bounds__(1024) void index_topk_runs_kernel(TopkArgs a) {
             incl += waves_before(s_wave, wave, lane, total);
             unsigned before = total - incl;      // the keys in the bins above this thread's
 #pragma unroll
-            for (int i = per - 1; i >= 0; --i) {
+            for (int i = 1; i >= 0; --i) {
                 const unsigned upto = before + h[i];
-                if (upto >= want && before < want) s_pick[0] = (unsigned)(tid * per + i), s_pick[1] = want - before, s_pick[2] = h[i];
+                if (upto >= want && before < want) s_pick[0] = (unsigned)(2 * tid + i), s_pick[1] = want - before, s_pick[2] = h[i];
                 before = upto;
             }
             lds_barrier();
         };
-        // The first digit is taken from the keys' own range: the bits below the highest that differs between the candidates'
-        // smallest and largest key, 2,048 bins over what lies between them, where the top bits of the keys as they are put a
-        // row of scores into a few dozen bins (which its atomics then meet in) and leave thousands of keys to two more
-        // digits. A bin then holds a few dozen keys around the k-th, which are ranked against each other at once.
-        uint32_t hi = 0u, lo_not = 0u;      // (elements that are no candidates count as keys of 0: below the range, in bin 0)
-#pragma unroll
-        for (int j = 0; j < EPT; ++j) {
-            hi = max(hi, key[j]);
-            lo_not = max(lo_not, ((ok >> j) & 1u) ? ~key[j] : 0u);
-        }
-        hi = wave_max(hi), lo_not = wave_max(lo_not);
-        if (lane == 0) s_range[0][wave] = hi, s_range[1][wave] = lo_not;
+        // Digits of 11 bits until a bin holds few enough keys to rank them against each other, or a digit holds the last bit.
+        if (tid < kShortList) s_rank[tid] = 0u;
         if (tid == 0) s_count = 0u;
-        lds_barrier();
-        hi = wave_max(s_range[0][lane & 15]), lo_not = wave_max(s_range[1][lane & 15]);
-        const uint32_t low = ~lo_not, span = hi - low;
-        const int shift0 = span < 2048u ? 0 : 21 - __builtin_clz(span);      // (span >> shift0 is below 2,048)
-        auto digit = [&](uint32_t x) __attribute__((always_inline)) -> uint32_t { return x < low ? 0u : (x - low) >> shift0; };
-        pass(std::integral_constant<int, 2048>{}, [](uint32_t) { return true; }, digit);
-        const unsigned bin = s_pick[0], left = s_pick[1], held = s_pick[2];
-        if (held <= (unsigned)kShortList) {
+        int rest;      // the bits below the digits already chosen
+        unsigned held;
+        auto chosen = [&](int below) __attribute__((always_inline)) {
+            prefix += (uint32_t)__builtin_amdgcn_readfirstlane((int)s_pick[0]) << below, rest = below;      // the bin's first key
+            want = s_pick[1], held = (unsigned)__builtin_amdgcn_readfirstlane((int)s_pick[2]);
+        };
+        auto in_bin = [&](uint32_t x) __attribute__((always_inline)) -> bool {
+            if constexpr (RANGE) return x >= prefix && ((x - prefix) >> rest) == 0u;
+            return (x >> rest) == (prefix >> rest);
+        };
+        if constexpr (RANGE) {
+            uint32_t hi = 0u, lo_not = 0u;      // (elements that are no candidates count as keys of 0: below the range, in bin 0)
+#pragma unroll
+            for (int j = 0; j < EPT; ++j) {
+                hi = max(hi, key[j]);
+                lo_not = max(lo_not, ((ok >> j) & 1u) ? ~key[j] : 0u);
+            }
+            hi = wave_max(hi), lo_not = wave_max(lo_not);
+            if (lane == 0) s_range[0][wave] = hi, s_range[1][wave] = lo_not;
+            lds_barrier();
+            hi = wave_max(s_range[0][lane & 15]), lo_not = wave_max(s_range[1][lane & 15]);
+            const uint32_t low = ~lo_not, span = hi - low;
+            const int first_rest = span < 2048u ? 0 : 21 - __builtin_clz(span);      // (span >> first_rest is below 2,048)
+            pass([](uint32_t) { return true; }, [&](uint32_t x) -> uint32_t { return (max(x, low) - low) >> first_rest; });
+            prefix = low;
+            chosen(first_rest);
+            while (rest > 0 && held > (unsigned)kShortList) {
+                const int next = max(rest - 11, 0);
+                pass(in_bin, [&](uint32_t x) -> uint32_t { return (x - prefix) >> next; });
+                chosen(next);
+            }
+        } else {
+            static_for<3>([&](auto step) __attribute__((always_inline)) {
+                constexpr int p = step, shift = p == 0 ? 21 : p == 1 ? 10 : 0, above = p == 0 ? 32 : p == 1 ? 21 : 10;
+                if (p == 0 || held > (unsigned)kShortList) {
+                    pass([&](uint32_t x) { return p == 0 || (x >> (above & 31)) == (prefix >> (above & 31)); },
+                         [](uint32_t x) -> uint32_t { return (x >> shift) & (uint32_t)((1ull << (above - shift)) - 1ull); });
+                    chosen(shift);
+                }
+            });
+        }
+        if (rest > 0) {      // the key with fewer than `want` above it and, with its equals, at least `want`
             if (mine) {
 #pragma unroll
                 for (int j = 0; j < EPT; ++j)
-                    if (digit(key[j]) == bin) s_list[atomicAdd(&s_count, 1u)] = key[j];
+                    if (in_bin(key[j])) s_list[atomicAdd(&s_count, 1u)] = key[j];
             }
             lds_barrier();
-            if (tid < (int)held) {      // the key with fewer than `left` above it and, with its equals, at least `left`
-                const uint32_t x = s_list[tid];
-                unsigned above = 0u, equal = 0u;
-                for (unsigned i = 0; i < held; ++i) above += s_list[i] > x ? 1u : 0u, equal += s_list[i] == x ? 1u : 0u;
-                if (above < left && above + equal >= left) s_pick[0] = x, s_pick[1] = left - above;
+            const int n = __builtin_amdgcn_readfirstlane((int)s_count);
+            const uint32_t x = s_list[lane];
+            unsigned rank = 0u;      // above | equal << 16, of the list's keys wave, wave + 16, ..
+            for (int i = wave; i < n; i += 16) {
+                const uint32_t other = (uint32_t)__builtin_amdgcn_readlane((int)x, i);
+                rank += other > x ? 1u : other == x ? 0x10000u : 0u;
             }
+            if (lane < n) atomicAdd(&s_rank[lane], rank);
             lds_barrier();
-            prefix = s_pick[0], want = s_pick[1];
-        } else {      // (many equal or nearly equal keys: digits of 11, 11 and 10 bits from the top)
-            static_for<3>([&](auto step) {
-                constexpr int p = step;
-                constexpr int kShift[3] = {21, 10, 0}, kDigit[3] = {11, 11, 10};
-                constexpr int shift = kShift[p], bins = 1 << kDigit[p], done = shift + kDigit[p];      // `done`: the bits below the digits already chosen
-                pass(std::integral_constant<int, bins>{},
-                     [&](uint32_t x) { return p == 0 || (x >> (done & 31)) == (prefix >> (done & 31)); },
-                     [&](uint32_t x) { return (x >> shift) & (unsigned)(bins - 1); });
-                prefix |= s_pick[0] << shift;
-                want = s_pick[1];
-            });
+            rank = s_rank[lane];
+            const unsigned before = rank & 0xffffu, upto = before + (rank >> 16);
+            const unsigned long long kth = __builtin_amdgcn_ballot_w64(lane < n && before < want && upto >= want);
+            const int at = __builtin_ctzll(kth | 1ull << 63);
+            prefix = (uint32_t)__builtin_amdgcn_readlane((int)x, at), want -= (unsigned)__builtin_amdgcn_readlane((int)before, at);
         }
     }
     // What each thread writes (above the k-th key | equal to it << 16), then the places before each thread's. A key of

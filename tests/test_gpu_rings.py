@@ -156,9 +156,9 @@ def test_prompt_chunks_at_the_edges_of_a_block_of_keys(d, hkv, g, page, position
 
 
 @pytest.mark.parametrize("n,k", [(9000, 700), (3000, 512), (50000, 2048)])
-@pytest.mark.parametrize("equal", [1, 511, 512, 513, 600])
+@pytest.mark.parametrize("equal", [1, 62, 63, 64, 65, 511, 512, 513, 600])
 def test_picks_where_the_kth_score_has_many_near_it(n, k, equal):
-    # `equal` scores tie at the k-th place (a list of up to 512 is ranked at once, longer ones go by digits), among neighbours
+    # `equal` scores tie at the k-th place (a list of up to 64 is ranked at once, longer ones go by digits), among neighbours
     # one bit apart, over a range of all signs or of fewer bits than the digit has
     g = torch.Generator().manual_seed(n + equal)
     wide = torch.randn(n, generator=g) * 10 ** torch.empty(n).uniform_(-3, 3, generator=g)
