@@ -295,6 +295,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 1 : 8 / WAVES) void prefill_
         });
         });
     };
+    auto dma_turn = [](int n) __attribute__((always_inline)) -> int { return 4 * (n & 3) + ((n >> 2) & 3); };      // DMA: what permutes key n's chunks
     // Operand reads, two operands a step. K, step i: k-step i of both 32-key halves. V, step i: keys
     // 16 (i / (NB / 2)) .. + 15 of the 32-dim blocks 2 (i % (NB / 2)) and the next one.
     auto read_k = [&](const uint16_t* kl, auto ic, u32x4 (&dst)[2]) __attribute__((always_inline)) {
@@ -304,7 +305,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 1 : 8 / WAVES) void prefill_
             if constexpr (IQK) {
                 dst[kb] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint8_t*>(kl) + (32 * kb + n32) * KSTR8 + 32 * i + 16 * h);
             } else if constexpr (DMA) {
-                const uint32_t row = (uint32_t)(n32 * ROWB + 16 * (h ^ (4 * (n32 & 3) + ((n32 >> 2) & 3))));
+                const uint32_t row = (uint32_t)(n32 * ROWB + 16 * (h ^ dma_turn(n32)));
                 dst[kb] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint8_t*>(kl) + (row ^ (32u * (i & 7))) + 256 * (i >> 3) + 32 * kb * ROWB);
             } else {
                 dst[kb] = *reinterpret_cast<const u32x4*>(&kl[(32 * kb + n32) * KSTR + 16 * i + 8 * h]);
@@ -323,7 +324,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 1 : 8 / WAVES) void prefill_
             const int nb = 2 * (i % (NB / 2)) + j;
             if constexpr (DMA) {      // groups 4 g + h and 4 g + 2 + h of four keys: two transposing reads
                 const int key = 4 * h + ((lane & 15) >> 2);
-                const uint32_t at = ((uint32_t)(key * ROWB + 8 * (lane & 1) + 16 * ((2 * ((lane >> 4) & 1) + ((lane >> 1) & 1)) ^ (4 * (key & 3) + ((key >> 2) & 3)))) ^ (64u * (nb & 3))) + 256u * (nb >> 2);
+                const uint32_t at = ((uint32_t)(key * ROWB + 8 * (lane & 1) + 16 * ((2 * ((lane >> 4) & 1) + ((lane >> 1) & 1)) ^ dma_turn(key))) ^ (64u * (nb & 3))) + 256u * (nb >> 2);
                 const u32x2 x = read_transposed(vb + at + 16 * g * ROWB), y = read_transposed(vb + (at ^ 32u) + (16 * g + 8) * ROWB);
                 dst[j] = u32x4{x.x, x.y, y.x, y.y};
                 continue;
@@ -334,8 +335,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 1 : 8 / WAVES) void prefill_
     };
 
     // DMA. Load j of a wavefront takes rows DROWS (NI wave + j) .. of a block; lane i's 16 bytes go to byte 16 i of the
-    // kilobyte, so a lane fetches the chunk that belongs there. row_of: its row of the block.
-    auto dma_turn = [](int n) __attribute__((always_inline)) -> int { return 4 * (n & 3) + ((n >> 2) & 3); };
+    // kilobyte, so a lane fetches the chunk that belongs there.
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     uint32_t send_slot[DMA ? NI : 1];      // the slots of the lane's rows of the block that is sent for next
     auto dma_slots = [&]() __attribute__((always_inline)) {      // ... from the entries, lane i holding position i's
@@ -396,7 +396,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 1 : 8 / WAVES) void prefill_
     if (DMA && any_block) {
         load_entries(kt_lo);
         dma_slots();
-        static_for<2 * NI>([&](auto ic) __attribute__((always_inline)) { send(ic, kt_lo & 1, WAVES == 8 ? 0 : kt_lo & 1); });
+        static_for<2 * NI>([&](auto ic) __attribute__((always_inline)) { send(ic, kt_lo & 1, kt_lo & 1); });
         load_entries(upto(kt_lo + 1));
     }
     if (!DMA && any_block) {
@@ -639,34 +639,41 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 1 : 8 / WAVES) void prefill_
             int vcur = 0, kt = kt_lo;
             if constexpr (RESUME) {
                 for (; kt < kt_lead; ++kt) {
-                    begin(kt), scores(kt, after(vcur)), weigh(kt, vcur, c1), values(kt, vcur), end(kt);
+                    scores(kt, after(vcur)), weigh(kt, vcur, c1), values(kt, vcur);
+                    __syncthreads();
                     vcur = after(vcur);
                 }
             }
             for (; kt < kt_full; ++kt) {
-                begin(kt), scores(kt, after(vcur)), weigh(kt, vcur, c0), values(kt, vcur), end(kt);
+                scores(kt, after(vcur)), weigh(kt, vcur, c0), values(kt, vcur);
+                __syncthreads();
                 vcur = after(vcur);
             }
             for (; kt <= kt_hi; ++kt) {
-                begin(kt), scores(kt, after(vcur)), weigh(kt, vcur, c1), values(kt, vcur), end(kt);
+                scores(kt, after(vcur)), weigh(kt, vcur, c1), values(kt, vcur);
+                __syncthreads();
                 vcur = after(vcur);
             }
         } else {
             // iteration kt weighs block kt - 1: masked while that block is below kt_lead or from kt_full on
-            begin(kt_lo), scores(kt_lo, 1), end(kt_lo);
+            scores(kt_lo, 1);
+            __syncthreads();
             int vprev = 0, vcur = 1, kt = kt_lo + 1;
             if constexpr (RESUME) {
                 for (; kt <= min(kt_lead, kt_hi); ++kt) {
-                    begin(kt), weigh(kt - 1, vprev, c1), values(kt - 1, vprev), scores(kt, after(vcur)), end(kt);
+                    weigh(kt - 1, vprev, c1), values(kt - 1, vprev), scores(kt, after(vcur));
+                    __syncthreads();
                     vprev = vcur, vcur = after(vcur);
                 }
             }
             for (; kt <= min(kt_full, kt_hi); ++kt) {
-                begin(kt), weigh(kt - 1, vprev, c0), values(kt - 1, vprev), scores(kt, after(vcur)), end(kt);
+                weigh(kt - 1, vprev, c0), values(kt - 1, vprev), scores(kt, after(vcur));
+                __syncthreads();
                 vprev = vcur, vcur = after(vcur);
             }
             for (; kt <= kt_hi; ++kt) {
-                begin(kt), weigh(kt - 1, vprev, c1), values(kt - 1, vprev), scores(kt, after(vcur)), end(kt);
+                weigh(kt - 1, vprev, c1), values(kt - 1, vprev), scores(kt, after(vcur));
+                __syncthreads();
                 vprev = vcur, vcur = after(vcur);
             }
             weigh(kt_hi, vprev, c1), values(kt_hi, vprev);      // (a mask over a wholly visible block changes nothing)
