@@ -386,15 +386,9 @@ PKV_DEV f32x16 mfma_32(u32x4 a, u32x4 b, f32x16 c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
     }
 }
-// (The loads are spelled in assembly so that the compiler neither counts them nor waits for them: the waits are the
-// kernel's own, and those and the barrier are "memory" clobbers, which keeps a tile's LDS reads behind them.)
-// 64 lanes x 16 bytes from base + offset (a lane's own) to LDS bytes lds .. lds + 1023.
-PKV_DEV void dma_row(uint32_t offset, const uint8_t* base, unsigned lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds));
-}
-// The score products and their operand reads are spelled out too, with the accumulators in ordinary registers (the
-// compiler would put them where the value accumulators are and move 16 of those out and back every step) and the waits
-// counted by hand: `ahead` reads are in flight behind the one a product needs.
+// The score products and their operand reads are spelled out, as the loads to LDS are (pkv_dma.hpp), with the accumulators in
+// ordinary registers (the compiler would put them where the value accumulators are and move 16 of those out and back every
+// step) and the waits counted by hand: `ahead` reads are in flight behind the one a product needs.
 template <bool F16>
 PKV_DEV void score_product(f32x16& c, const u32x4& a, const u32x4& b) {
     if constexpr (F16) asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
@@ -559,7 +553,7 @@ __global__ __launch_bounds__(256, 1) void latent_heads_kernel(LatentArgs a) {
             }
         } else if constexpr (k < 8) {
             const uint32_t place = (uint32_t)(ln ^ ((2 * wave + k / 4) & 3)) * 16u;
-            dma_row(place ^ (uint32_t)(64 * (k & 3)), plan_row0 + min(k, plan_room) * (W * 2), plan_to + (unsigned)((8 * wave + k) * (R * 2)));
+            dma_rows<false>(place ^ (uint32_t)(64 * (k & 3)), plan_row0 + min(k, plan_room) * (W * 2), plan_to + (unsigned)((8 * wave + k) * (R * 2)));
         } else {
             const int tail_row = ln >> 3;
             const uint32_t tail_at = (uint32_t)(R * 2 + 16 * ((ln & 7) ^ (((8 * wave + tail_row) >> 1) & 7)));
