@@ -163,9 +163,9 @@ struct MfmaShape {
 // for the next launch that uses them. Without counters the units are dealt in turn.
 // MASK: what hides positions of a column beside its own end: nothing, a draft tree, or a sliding window (with or
 // without a tree). Trees and windows are kernels of their own: a tree's short mask (in the step) is of no use to a
-// window, whose kernels it cost registers (20 bytes of scratch a lane in the fused 16-bit ones, 40 more in pairs of
-// tiles) and time: 64 rows ~U[1024, 8192], 32 / 8 heads, a window of 1,024, 3 columns: BF16 174 us in one kernel, 154
-// apart; INT8 194 and 184; and a tree's kernels keep fewer registers without a window: INT8, 5 columns 305 -> 283 us.
+// window, whose kernels it cost registers and time (when all rows went through registers: 64 rows ~U[1024, 8192], 32 / 8
+// heads, a window of 1,024, 3 columns: BF16 174 us in one kernel, 154 apart, INT8 194 and 184; a tree's kernels without a
+// window, INT8, 5 columns, 305 -> 283).
 // DH: 128-wide halves of a head (1: heads of 128; 2: heads of 256, whose rows
 // are 512 bytes of 16-bit pages by themselves, so a wavefront serves one KV head: HW 1): twice the key pieces, query
 // pieces, score products and output tiles, the same layouts otherwise; twice the registers too, so one workgroup a
@@ -176,7 +176,8 @@ struct MfmaShape {
 // once a tile. More than one tile takes the registers of a second workgroup on the compute unit (one stays). Built for
 // four or three tiles (or a window's two) of 128-wide heads over 16-bit pages, two over 8-bit pages and three over scaled
 // rows (pairs still fit two workgroups a compute unit) or of 256-wide heads, where it measured faster (64 rows ~U[1024,
-// 8192] of 32 / 8 heads, 8 columns: 676 -> 480 us, FP8 376 -> 224); four tiles of 8-bit pages measured slower.
+// 8192] of 32 / 8 heads, 8 columns, a tile at a time and so: 663 and 333 us, FP8 342 and 222); four tiles of 8-bit pages
+// measured slower.
 // NARROW: 64-wide heads, read as 128-wide ones. Two adjacent KV heads' rows of a position are 128 contiguous values,
 // which is what a 128-wide head's row is: the launcher hands the kernel half the KV heads at twice the width and GQA
 // groups twice as large (a group's first half the query heads of the even KV head, its second half the odd one's: the
@@ -239,9 +240,7 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
     const unsigned per_row = (unsigned)(hgroups * a.tiles);
     const int slot_bytes = a.hkv * D * EB;
     const bool tree = MASK == kMaskTree || (MASK == kMaskSliding && (a.parents != nullptr || a.parents64 != nullptr));
-    // (A tree's launch has no window. The kernel of four tiles asks for one all the same: left out, the compiler schedules
-    // its steps so that 98 registers a lane go to scratch instead of 39, 64 rows of 8 columns 600 us instead of 520.)
-    const int win = MASK == kMaskSliding || (MASK == kMaskTree && QT > 3) ? a.sliding : 0;
+    const int win = MASK == kMaskSliding ? a.sliding : 0;      // (a tree's launch has no window)
 
     // Quotients by the launch's own numbers (none of them a power of two in general: a division is forty instructions).
     auto by_group = [&](int x) __attribute__((always_inline)) -> int { return (int)div32(a.group_div, (uint32_t)x); };
