@@ -24,7 +24,8 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=o
 # The window and prompt kernels' accumulators are rescaled by the vector pipe between products, which cannot reach the
 # registers that the compiler keeps products in for kernels of one wavefront a SIMD (160 moves a pair of steps with three
 # query tiles; prompt chunks of 256-wide heads 104 bytes of scratch a lane, and 97.4 -> 91.3 us without, 254 -> 222 over
-# fp8:row pages): their products take ordinary registers. The bits are the same.
+# fp8:row pages): their products take ordinary registers. The bits are the same. (An internal option of this image's
+# compiler: one that does not know it stops with "Unknown command line argument", and is to be run without.)
 OWN_FLAGS = {start: ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for start in ("pkv_attend_", "pkv_prefill")}
 
 

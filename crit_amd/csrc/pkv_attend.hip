@@ -444,25 +444,24 @@ static int launch_attend_checked(const crit_pkv_attend_params* p, hipStream_t st
     a.max_keys = (int)(table_keys < 0x3fffffff ? table_keys : 0x3fffffff);
     const int64_t live_parts = ((p->blocks ? (int64_t)a.listed_keys : (int64_t)a.max_keys) + (int64_t)p->piece - 1) / p->piece;
     const unsigned gy = (unsigned)(live_parts < p->partitions ? live_parts : p->partitions);
-    // Windows of several tiles of 128-wide heads over 16-bit pages, split launch: a workgroup holds four tiles (one
-    // workgroup a compute unit), or the two of a window of two (two workgroups still, with two dozen registers in
-    // scratch, all but four of a tree's accesses outside the steps), and reads the rows once for all of them. A tile's
-    // bits are the same however many share a workgroup, so this may follow the launch. Measured on MI355X (32 / 8 heads,
-    // 64 rows ~U[1024, 8192]): 4 columns 383 -> 288 us, 5 columns 519 -> 424, 8 columns 676 -> 480; one row of 32,768:
-    // 55 -> 45, 72 -> 56 and 91 -> 62. Not taken where it measured slower: four tiles of 8-bit pages (8 columns 376 ->
-    // 334 us but 5 columns 279 -> 302, one row 55 -> 92: the converted rows' steps are too long a chain for one
-    // wavefront a SIMD). Three tiles, which leave nothing in scratch, in place of four where window_tiles_16bit() says
-    // so. (Three in a second workgroup's registers would spill 336 bytes a lane.)
+    // Windows of several tiles of 128-wide heads over 16-bit pages, split launch: a workgroup holds three or four tiles
+    // (one workgroup a compute unit, the rows in LDS, nothing in scratch; window_tiles_16bit() says which), or the two of a
+    // window of two (two workgroups, 20 to 48 bytes of scratch a lane), and reads the rows once for all of them. A tile's
+    // bits are the same however many share a workgroup, so this may follow the launch. Measured on MI355X, a tile a
+    // workgroup and so (32 / 8 heads, 64 rows ~U[1024, 8192]): 4 columns 371 and 255 us, 5 columns 507 and 281, 8 columns
+    // 663 and 333; one row of 32,768: 53 and 36, 71 and 42, 93 and 48. In twos throughout 5 columns are 389, 8 columns 409.
+    // (Three in a second workgroup's registers would spill 336 bytes a lane.)
     a.query_tiles = 1;
     if (a.fast128 && !p->blocks && !p->fused && wide128 && p->kind == 0 && a.tiles >= 2) {
         const bool full = !p->counts || p->window_tokens == (int64_t)p->n_rows * p->columns;
         a.query_tiles = window_tiles_16bit(a.tiles, full, (int64_t)p->n_rows * (p->kv_heads / a.heads_per_wave) * gy, compute_units());
         a.tiles = (a.tiles + a.query_tiles - 1) / a.query_tiles;
     }
-    // 8-bit pages: two tiles a workgroup, two workgroups a compute unit still (FP8 in 242-252 registers; the row-scaled
-    // kinds with two dozen in scratch, one or two accesses of them inside the steps). 64 rows, 4 / 5 / 8 columns: FP8 207 -> 147, 279 -> 214, 376 ->
-    // 230 us, INT8 224 -> 167, 307 -> 264, 428 -> 287 us; one row of 32,768 (FP8): 54 -> 52 and 64 -> 52 us, but a pair
-    // alone (4 columns) 40 -> 51 us, so a window of two tiles pairs them only in launches that fill the card.
+    // 8-bit pages: two tiles a workgroup, two workgroups a compute unit still (nothing in scratch), three of scaled rows where
+    // window_tiles_8bit() says so. 64 rows, 4 / 5 / 8 columns, a tile a workgroup and so: FP8 201 and 146, 266 and 208, 342
+    // and 222 us, INT8 214 and 155, 276 and 197, 352 and 234. One row of 32,768 (FP8): 8 columns 60 and 49 us, but 5 columns
+    // 44.5 and 49, and a pair alone (4 columns) 38 and 49, so a window of two tiles pairs them only in launches that fill
+    // the card.
     if (a.fast128 && !p->blocks && !p->fused && wide128 && p->kind >= 1 && a.tiles >= 2) {
         const int64_t apart = (int64_t)p->n_rows * (p->kv_heads / a.heads_per_wave) * a.tiles * p->partitions;
         if (a.tiles >= 3 || apart > (int64_t)compute_units() * 2) {
@@ -471,9 +470,9 @@ static int launch_attend_checked(const crit_pkv_attend_params* p, hipStream_t st
             a.tiles = (a.tiles + a.query_tiles - 1) / a.query_tiles;
         }
     }
-    // 256-wide heads: pairs of tiles with one step in flight a wavefront instead of two (with two, 56-85 registers went
-    // to scratch and 64 rows x 4 columns took 554 us against 443 apart; with one, 24 / 2 heads x 256 bf16, 64 rows, 2 / 4
-    // / 5 / 8 columns: 287 -> 232, 445 -> 410, 569 -> 452, 856 -> 676 us; one row of 200,000: 255 -> 146 and 344 -> 237).
+    // 256-wide heads: pairs of tiles, with a pair of steps (8-bit pages: two pairs) in flight in LDS as one tile has. 24 / 2
+    // heads x 256 bf16, 64 rows ~U[1024, 8192], 2 / 4 / 5 / 8 columns, a tile a workgroup and so: 230 and 176, 332 and 300,
+    // 416 and 323, 607 and 472 us; one row of 200,000, 5 / 8 columns: 256 and 141, 332 and 215.
     if (a.fast128 && !p->blocks && !p->fused && wide256 && a.tiles >= 2) {
         a.query_tiles = 2;
         a.tiles = (a.tiles + a.query_tiles - 1) / a.query_tiles;

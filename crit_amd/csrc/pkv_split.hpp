@@ -63,13 +63,13 @@ PKV_SPLIT_FN DealtTile dealt_tile(uint32_t workgroup, uint32_t share_tiles, int 
 // of a wavefront, partition) triples of the launch; `units`: the card's compute units.
 //   - Three tiles instead of four wherever they take no more workgroups (3, 5, 6 and 9 tiles): a step is bound by its
 //     matrix and softmax work, which tiles that no row fills cost as well. 64 rows ~U[1024, 8192], 32 / 8 heads x 128,
-//     BF16, three against four: 5 columns (3 tiles) 373 us against 430, 9 columns (5) 653 / 809, 12 columns (6) 718 / 868;
-//     64 / 8 heads, 9 columns (9) 1,031 / 1,270.
+//     BF16, three against four: 5 columns (3 tiles) 280 us against 314, 9 columns (5) 476 / 557, 12 columns (6) 494 / 582;
+//     64 / 8 heads, 9 columns (9) 714 / 853.
 //   - But a row of four tiles in a launch sized for five, six or nine has one workgroup of four, and two of three, each
-//     of which reads the row: 56 / 8 heads, a launch of 5 columns, rows of 4: 602 us in threes, 475 in fours. So those
+//     of which reads the row: 56 / 8 heads, a launch of 5 columns, rows of 4: 459 us in threes, 329 in fours. So those
 //     launches take threes only where every row is full, or where the launch is small enough that the second workgroup
-//     runs beside the first: up to two workgroups a compute unit where a row has two of them (one row of 32,768: 83 us
-//     against 105 whatever its columns; 3 rows of 32,768, three times as many: 215 against 161), one where it has three.
+//     runs beside the first: up to two workgroups a compute unit where a row has two of them (one row of 32,768: 66 us
+//     against 77; 3 rows of 32,768, three times as many: 159 against 120), one where it has three.
 PKV_SPLIT_FN int window_tiles_16bit(int64_t tiles, bool full, int64_t places, int64_t units) {
     if (tiles <= 2) return (int)tiles;
     const int64_t threes = (tiles + 2) / 3;
