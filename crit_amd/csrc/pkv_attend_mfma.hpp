@@ -223,7 +223,7 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
     __shared__ int s_wave_sum[4];
     __shared__ uint16_t s_order[kLdsRows];   // the dense list: the rows by the size of their last partition
     int* const s_key = reinterpret_cast<int*>(&s_acc[0][0][0]);      // ... (while the list is made)
-    static_assert(sizeof(s_acc) >= kLdsRows * sizeof(int), "the list's keys lie in the fold's array");
+    static_assert(sizeof(s_acc) >= (kLdsRows + 256) * sizeof(int), "the list's keys lie in the fold's array");
     __shared__ unsigned s_unit;
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -284,36 +284,43 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT>::kGroups)) void atten
         if (r1 <= a.n_rows) s_before[r1] = upto + c0;
         if (tid == 255 && kLdsRows <= a.n_rows) s_before[kLdsRows] = upto + c0 + c1;
         // The rows' last partitions are taken largest first (a launch's tail is as long as its last units): positions
-        // the last partition holds (more than a piece where partitions hold several pieces), ties by row.
-        for (int r = tid; r < a.n_rows; r += 256) {
-            const int count = s_rows[r][0];
-            int key = -1;
+        // the last partition holds (more than a piece where partitions hold several pieces), ties by row. A row's place is the
+        // number of rows before it. Up to 256 rows, in launches of more units than workgroups; more rows cost more to rank
+        // than it returns.
+        const bool ranked = a.n_rows <= 256 && (unsigned)a.units_x * (unsigned)a.units_y > grid;
+        int* const s_rank = s_key + kLdsRows;
+        for (int r = tid; r < (ranked ? 256 : a.n_rows); r += 256) {
+            const int count = r < a.n_rows ? s_rows[r][0] : 0;
+            unsigned key = 0;      // a size of 23 bits, then the row: no two alike, and none above those past the last row
             if (count > 0) {
                 const int n_keys = min(s_rows[r][1] + count, a.max_keys);
                 const int n_pieces = pieces_of(n_keys);
-                key = FUSED ? n_keys : (n_pieces > a.parts ? a.piece + 1 : n_keys - (n_pieces - 1) * a.piece);
+                const int size = FUSED ? n_keys : (n_pieces > a.parts ? a.piece + 1 : n_keys - (n_pieces - 1) * a.piece);
+                key = (unsigned)min(size, 0x7ffffe) + 1u;
             }
-            s_key[r] = key;
+            if (ranked) s_key[r] = (int)(r < a.n_rows ? (key << 8) + (unsigned)(255 - r) : 0u), s_rank[r] = 0;
+            else s_order[r] = (uint16_t)r;
         }
         lds_barrier();
-        if (a.n_rows <= 256 && (unsigned)a.units_x * (unsigned)a.units_y > grid) {
-            // A row's place is the number of rows before it. A wavefront holds 64 rows' keys, a lane each, and goes through them by
-            // v_readlane: no round trip to LDS a row (64 rows: 4,800 of a workgroup's 22,000 clocks before its first step as a
-            // loop over LDS; with the quotients and the search by multiplications and ballots, 64 rows ~U[1024, 8192], 5 columns
-            // 298 -> 294 us, of 24 / 2 heads x 256 BF16, one column, 159 -> 154).
-            if (64 * wave < a.n_rows) {
-                const int key = tid < a.n_rows ? s_key[tid] : 0;
+        if (ranked) {
+            // 64 rows a wavefront, a lane each, four others a read; the wavefronts that 64 or 128 rows leave over share the
+            // others. (One other at a time, by v_readlane, and ties by a comparison of rows were 5 us of a launch of 128 rows: of
+            // 40 to 300 positions, 24 / 3 heads x 128, BF16 27.8 us, 22.6 so; 64 rows ~U[1024, 8192], 32 / 8 heads, one column
+            // BF16 215.7 and 211.6, FP8 119.0 and 115.3.)
+            const int shares = a.n_rows <= 64 ? 4 : a.n_rows <= 128 ? 2 : 1, row = 64 * (wave / shares) + lane;
+            if (64 * (wave / shares) < a.n_rows) {
+                const unsigned key = (unsigned)s_key[row];
                 int rank = 0;
-                for (int r0 = 0; r0 < a.n_rows; r0 += 64) {
-                    const int keys = r0 + lane < a.n_rows ? s_key[r0 + lane] : 0;
-                    const int upto = min(64, a.n_rows - r0);
 #pragma unroll 4
-                    for (int o = 0; o < upto; ++o) rank += __builtin_amdgcn_readlane(keys, o) + (r0 + o < tid ? 1 : 0) > key ? 1 : 0;
+                for (int o = 4 * (wave % shares); o < a.n_rows; o += 4 * shares) {
+                    const u32x4 others = *reinterpret_cast<const u32x4*>(s_key + o);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) rank += others[i] > key ? 1 : 0;
                 }
-                if (tid < a.n_rows) s_order[rank] = (uint16_t)tid;
+                atomicAdd(&s_rank[row], rank);
             }
-        } else {      // (more rows: ranking them costs more than it returns; a unit a workgroup: all start at once)
-            for (int r = tid; r < a.n_rows; r += 256) s_order[r] = (uint16_t)r;
+            lds_barrier();
+            if (tid < a.n_rows) s_order[s_rank[tid]] = (uint16_t)tid;
         }
         lds_barrier();
     }

@@ -133,6 +133,28 @@ def test_merges_of_short_rows_in_wide_tables(hkv, g, d):
                 torch.testing.assert_close(lse[at].double().cpu(), want_lse, atol=1e-3, rtol=1e-4, msg=str(r))
 
 
+@pytest.mark.parametrize("kind", ["bf16", "fp8"])
+@pytest.mark.parametrize("rows", [43, 63, 64, 65, 127, 128, 129, 191, 255, 256, 257])
+@pytest.mark.parametrize("alike", [False, True])
+def test_every_row_has_its_place_in_the_list(kind, rows, alike):
+    # more units than workgroups: rows are ranked by their last partitions, 64 a wavefront, up to 256; rows of one length
+    # (ties), of none and of several partitions among them. Every row as in launches too small to be ranked
+    lengths = [90 if alike else 1 + (37 * r) % 150 for r in range(6)]
+    cache = Cache(kind, 3, 128, 128, 16, lengths, seed=rows)
+    q = rand_q(rows, 12, 128, 72)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)
+    of = [(5 * r + r // 6) % 6 for r in range(rows)]
+    counts = [0 if r % 19 == 7 and not alike else 1 for r in range(rows)]
+    def run(at, **kw):
+        out = torch.zeros(rows, 12, 128, dtype=torch.bfloat16, device=dev)
+        return cache.attend(q, [of[r] for r in at], list(at), [lengths[of[r]] - 1 for r in at], 1, counts=i32([counts[r] for r in at]),
+                            out=out, partitions=3, piece=64, **kw)
+    want = sum(run(range(r, min(r + 16, rows))).float() for r in range(0, rows, 16)).bfloat16()
+    for fused in (False, True):
+        assert torch.equal(run(range(rows), fused=fused), want)
+    close(want[:1], cache.want(q[:1], of[0], lengths[of[0]] - 1, 1)[0])
+
+
 def test_a_workspace_that_starts_on_any_float():
     pk = kernels()
     cache = Cache("int8", 2, 128, 128, 16, [900, 3000])
