@@ -890,20 +890,24 @@ int launch_index_scores(const crit_pkv_index_scores_params* p, hipStream_t strea
     // operand's lanes lie in 16 keys), which bounds such calls (64 heads of 128, 4 tokens over 50,000 keys: 14.8 us, shared
     // 11.8; 15 over 65,536, with the selection, 56.9 and 43.8; 16 sequences of 4 over 50,000 each 124.3 and 85.8). Not
     // where many wavefronts would have no token (2 over 65,536 E4M3 keys 23.0 and 24.9; 5 over 10,000 6.9 and 7.9, 6 over
-    // 50,000 16.7 and 17.3), nor where the keys are too few for the steps of 64 (4 tokens: 4,000 keys 5.0 and 5.7, 8,000
-    // 5.65 and 5.71, 12,000 6.3 and 5.8). E4M3 keys are half the requests (24,000 keys: 4 tokens 7.3 and 8.2, 8 tokens 10.3
-    // and 10.9; 32,000: 8 tokens 12.8 and 11.0; 15 over 20,000 11.1 and 12.5), and queries past 16 operands leave one
-    // workgroup a compute unit (128 heads of 128, 8 tokens: 12,000 keys 11.0 and 12.5, 32,000 22.9 and 17.0; E4M3 7 over
-    // 52,000 21.1 and 23.2, 11 over 37,000 28.0 and 23.4).
+    // 50,000 16.7 and 17.3; 7 and 10 over 50,000 E4M3 keys 12.4 and 14.2, 14.9 and 16.7, 7 over as many 16-bit ones of 128
+    // heads 17.9 and 21.3), nor where the keys are too few for the steps of 64 (4 tokens: 4,000 keys 5.0 and 5.7, 8,000
+    // 5.65 and 5.71, 12,000 6.3 and 5.8; 8 over 12,000 6.9 and 7.4, over 20,000 9.9 and 9.3; 10 over 12,000 8.1 and 9.1, over
+    // 20,000 12.7 and 9.4). E4M3 keys are half the requests (24,000 keys: 4 tokens 7.3 and 8.2, 8 tokens 10.3 and 10.9;
+    // 32,000: 8 tokens 12.8 and 11.0; 15 over 20,000 11.1 and 12.5, over 32,000 15.3 and 16.3; 12 over 50,000 19.0 and 16.9), and
+    // queries past 16 operands leave one workgroup a compute unit (128 heads of 128: 8 tokens over 12,000 keys 11.0 and 12.5,
+    // over 32,000 22.9 and 17.0; 15 over 20,000 16.7 and 18.1; E4M3 11 over 37,000 28.0 and 23.4).
     const int64_t products = (int64_t)p->tokens * p->n;
-    const bool wide = ht * (p->dim / 32) > 16, filled = p->tokens == 4 || p->tokens == 7 || p->tokens == 8 || p->tokens >= 10;
-    const int64_t enough = fp8 ? (wide || p->tokens > 8 ? 400000 : 256000) : wide ? 256000 : 48000;
+    const bool wide = ht * (p->dim / 32) > 16, idle = p->tokens == 7 || p->tokens == 10;      // (a wavefront in four, two in six)
+    const bool filled = p->tokens == 4 || p->tokens == 8 || p->tokens >= 11 || (idle && !fp8 && !wide);
+    const int64_t enough = fp8 ? (p->tokens > 8 ? 500000 : wide ? 400000 : 256000) : wide ? (p->tokens > 8 ? 400000 : 256000) : p->tokens == 4 ? 48000 : (int64_t)p->tokens * 16000;
     const bool fours = filled && products >= enough && (share(4) || (p->tokens < 16 && p->group >= p->tokens));
     // Calls of 16 tokens and more share eight to a workgroup, in blocks of 256 keys or more, once such workgroups fill the chip,
     // and fours before that (16 tokens: 2,000 keys 13.9 us, in fours 5.4, 9,000 14.4 and 9.6, 32,000 16.9 and 15.9, 65,536 23.7
     // both; 48: 9,000 keys 14.5 and 13.3, 65,536 63.0 and 67.1; 128 heads, fours either way: 50 tokens over 2,000 keys 13.9 and
-    // 12.2, 100 14.1 and 15.4).
-    const bool eights = p->tokens >= 16 && share(wg_tokens), few = eights ? products <= (wide ? 128000 : 560000) : fours;
+    // 12.2, 100 14.1 and 15.4; E4M3 keys of 256, 32 heads, 24 tokens over 20,000 17.4 and 19.5).
+    const bool eights = p->tokens >= 16 && share(wg_tokens);
+    const bool few = eights ? products <= (wide ? 128000 : fp8 && p->dim == 256 ? 320000 : 560000) : fours;
     const int shared = few ? kSharedFew : eights ? kSharedMany : kSharedNone;
     const bool f16 = p->q_dtype == CRIT_PKV_F16;
     if (fp8) return f16 ? launch_scores_kind<true, true>(a, p->dim, shared, cus, stream) : launch_scores_kind<false, true>(a, p->dim, shared, cus, stream);
