@@ -119,8 +119,10 @@ PyObject* attend(PyObject*, PyObject* const* x, Py_ssize_t n) {
     const int64_t wider = d > dv ? d : dv, width = wider == 64 ? 128 : wider, fits = (kind == 0 ? 65536 : 196608) / width / 16 * 16;
     const int64_t block = 4 * (64 / (wider / 8));
     const int64_t piece = ((fits < 256 ? 256 : fits > 2048 ? 2048 : fits) + block - 1) / block * block;
-    const int64_t states = (offsets ? tokens : n_rows * columns) * hq * parts;
-    NEED(work->scalar_type() == at::kFloat && work->is_contiguous() && work->numel() >= states * (dv + 2));
+    int64_t states, floats;      // (a mistaken count of tokens or partitions may name more than 64 bits hold)
+    NEED(!__builtin_mul_overflow(offsets ? tokens : n_rows * columns, hq, &states) && !__builtin_mul_overflow(states, parts, &states) &&
+         !__builtin_mul_overflow(states, dv + 2, &floats));
+    NEED(work->scalar_type() == at::kFloat && work->is_contiguous() && work->numel() >= floats);
     float* const base = work->data_ptr<float>();
 
     crit_pkv_attend_params p = {};

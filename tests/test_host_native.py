@@ -86,6 +86,11 @@ def test_other_forms_of_a_window_and_every_mistake_are_left_alone():
         scaled = window(kind)
         assert attend_native({**scaled, "key_scales": None}) is None and attend_native({**scaled, "value_scales": None}) is None
     assert attend_native({**window("bf16", columns=65, rows=1), "parents": None}) is None
+    # more partials than 64 bits count: no workspace holds them (a count that wraps would be below any)
+    for heads, tokens, partitions in ((128, 1 << 40, 1 << 15), (128, (1 << 40) - 1, 65535), (8, 1 << 40, (1 << 31) - 1)):
+        case_of = window("bf16", hq=heads, hkv=2)
+        assert attend_native(case_of) is not None
+        assert attend_native({**case_of, "tokens": tokens, "partitions": partitions}) is None, (heads, tokens, partitions)
     # a batch of calls under a transform is not one call
     from torch._C._functorch import _add_batch_dim, _vmap_decrement_nesting, _vmap_increment_nesting
     level = _vmap_increment_nesting(2, "error")
