@@ -2,6 +2,10 @@
 
     python -m crit_amd.build            # compile everything, link crit_amd/lib/libcrit_pkv.so
 
+With it goes _pkv_host.so, the native share of the package's host code, which takes g++ and the headers of Python and torch
+and is optional: where it does not compile the build says so and the package's Python code does it all. With $CRIT_PKV_OUT the
+library alone is linked, there, and the two in crit_amd/lib stay as they are.
+
 hipcc cross-compiles for gfx950 without a GPU. No fast-math; FP contraction is off so that every fused multiply-add in
 the kernels is one the source spells out (a column's bits must not depend on which template instance computed it).
 """
@@ -33,17 +37,22 @@ HOST_LIB = os.path.join(LIB_DIR, "_pkv_host.so")
 
 
 def _compile_host():
-    """The native share of the package's host code: a Python extension module against this interpreter and this torch."""
+    """The native share of the package's host code: a Python extension module against this interpreter and this torch. The old
+    one goes first (a module that does not match the library is worse than none); the new one is there whole or not at all."""
+    if os.path.exists(HOST_LIB):
+        os.remove(HOST_LIB)
     import sysconfig
     import torch
     from torch.utils.cpp_extension import include_paths, library_paths
+    part = f"{HOST_LIB}.{os.getpid()}"
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", f'-DCRIT_TORCH_VERSION="{torch.__version__}"',
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I" + sysconfig.get_paths()["include"],
-           *["-isystem" + path for path in include_paths()], os.path.join(CSRC, "pkv_host.cpp"), "-o", HOST_LIB,
+           *["-isystem" + path for path in include_paths()], os.path.join(CSRC, "pkv_host.cpp"), "-o", part,
            *["-L" + path for path in library_paths()], "-ltorch_python", "-ltorch_cpu", "-lc10"]
     done = subprocess.run(cmd, capture_output=True, text=True)
     if done.returncode:
         raise RuntimeError(f"g++ failed on pkv_host.cpp:\n{done.stderr}")
+    os.replace(part, HOST_LIB)
 
 
 def sources():
@@ -65,19 +74,20 @@ def _compile(src):
 def build(verbose=True, jobs=None):
     """Compile every .hip under csrc/ for gfx950 and link the shared library; returns its path."""
     os.makedirs(OBJ_DIR, exist_ok=True)
+    out = os.environ.get("CRIT_PKV_OUT", LIB)
     jobs = jobs or min(8, os.cpu_count() or 1)
     with ThreadPoolExecutor(jobs) as pool:
-        host = pool.submit(_compile_host)
+        host = pool.submit(_compile_host) if os.path.abspath(out) == LIB else None
         found = list(pool.map(_compile, sources()))
-        host.result()
     for _, err in found:
         if err.strip() and verbose:
             print(err, file=sys.stderr)
-    out = os.environ.get("CRIT_PKV_OUT", LIB)
     link = ["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-o", out, *[obj for obj, _ in found]]
     done = subprocess.run(link, capture_output=True, text=True)
     if done.returncode:
         raise RuntimeError(f"link failed:\n{done.stderr}")
+    if host is not None and host.exception() is not None:
+        print(f"without the native host code, which is optional: {host.exception()}", file=sys.stderr)
     if verbose:
         print(f"built {out}")
     return out
