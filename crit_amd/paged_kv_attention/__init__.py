@@ -202,21 +202,20 @@ def _ptr(t):
 
 
 def _native_host():
-    """The native share of attend()'s and write()'s host code (crit_amd/csrc/pkv_host.cpp), where it is beside the library and
-    was built against this torch and this ABI; None: the calls below do it all, the same launches."""
-    here = os.path.dirname(os.path.abspath(__file__))
-    for path in (os.path.join(here, "_pkv_host.so"), os.path.join(os.path.dirname(here), "lib", "_pkv_host.so")):
-        if os.path.exists(path):
-            try:
-                loader = importlib.machinery.ExtensionFileLoader("_pkv_host", path)
-                found = importlib.util.module_from_spec(importlib.util.spec_from_loader("_pkv_host", loader))
-                loader.exec_module(found)
-            except ImportError:      # (another torch, another Python)
-                return None
-            same = (found.torch_version == torch.__version__ and found.abi_version == _abi.ABI_VERSION and
-                    found.attend_size == ctypes.sizeof(_abi.AttendParams) and found.write_size == ctypes.sizeof(_abi.WriteParams))
-            return found if same else None
-    return None
+    """The native share of attend()'s and write()'s host code (crit_amd/csrc/pkv_host.cpp), where the in-tree build made it
+    against this torch and this ABI; None (a staged copy of this package has none): the calls below do it all, the same launches."""
+    path = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "lib", "_pkv_host.so")
+    if not os.path.exists(path):
+        return None
+    try:
+        loader = importlib.machinery.ExtensionFileLoader("_pkv_host", path)
+        found = importlib.util.module_from_spec(importlib.util.spec_from_loader("_pkv_host", loader))
+        loader.exec_module(found)
+    except ImportError:      # (another torch, another Python)
+        return None
+    same = (found.torch_version == torch.__version__ and found.abi_version == _abi.ABI_VERSION and
+            found.attend_size == ctypes.sizeof(_abi.AttendParams) and found.write_size == ctypes.sizeof(_abi.WriteParams))
+    return found if same else None
 
 
 _host = _native_host()

@@ -3,14 +3,23 @@ fills, over the forms it takes; what it does not take (every mistake among it) i
 no entry point to call it hands back the parameters."""
 import ctypes
 import itertools
+import os
 
 import pytest
 import torch
 
 import crit_amd.paged_kv_attention as pk
+from crit_amd import build as builder
 
 STORE = {"bf16": torch.bfloat16, "fp16": torch.float16, "fp8": torch.float8_e4m3fn, "fp8:row": torch.float8_e4m3fn, "int8": torch.int8}
 native = pytest.mark.skipif(pk._host is None, reason="the extension is not built")
+
+
+def test_an_extension_that_is_built_is_in_use():
+    # (one that does not load, or was built against something else, would leave the calls to the Python code without a word)
+    if not os.path.exists(builder.HOST_LIB):
+        pytest.skip("the extension is not built")
+    assert pk._host is not None and os.path.samefile(pk._host.__file__, builder.HOST_LIB)
 
 
 @pytest.fixture
