@@ -204,15 +204,16 @@ static int launch_mfma(const AttendArgs& a, bool fused, dim3 grid, hipStream_t s
     const int mask = a.sliding > 0 ? kMaskSliding : (a.parents != nullptr || a.parents64 != nullptr ? kMaskTree : kMaskNone);
     // A workgroup a place of the tables ((row, heads, tiles) times partitions), no list of units. Up to a compute unit a place:
     // one workgroup a compute unit, more of its steps in flight (tables longer than their rows have places without work, and
-    // more places than compute units may be any launch). One or two rows of more places: the ordinary kernels' steps, as many
-    // workgroups a compute unit as their registers allow (three, without the list), the hardware's own order. A row's places
-    // are alike but its last: 2 rows of 30,000 to 50,000, 32 / 8 heads x 128, BF16 71.7 -> 60.4 us, of 100,000 158.6 -> 144.5;
-    // one of 200,000 in splits of 1,024 163.8 -> 157.5, FP8 78.9 -> 76.9, INT8 88.6 -> 87.2; a tree of 5 of 60,000, 56 / 8 heads,
-    // FP8 73.6 -> 69.2; 64-wide heads in pairs, one of 200,000 in splits 75.1 -> 72.8 and 45.2 -> 42.4. More rows are uneven, and the list's longest-first order and prefetch are the better (BF16 / FP8: 4
-    // rows of 30,000 to 60,000 143.8 / 65.9 us, 137.7 / 78.4 without it; 24 of 1,000 to 12,000 111.6 / 60.9 and 122.7 / 71.8; 64 of
-    // 1,024 to 8,192 209.9 / 113.6 and 239.3 / 120.7).
+    // more places than compute units may be any launch). One row or two of more places: the ordinary kernels' steps, three
+    // workgroups a compute unit of one tile (160 registers and fewer without the list) and two of two tiles, two rows' units
+    // by row_place(). One of 200,000, 40 / 8 heads x 128, in splits of 1,024, BF16 166 -> 160 us, FP8 96 -> 89, INT8 101 -> 95; one
+    // of 50,000, 56 / 8 heads, a tree of 5, FP8 69 -> 65; 2 rows of 100,000 160 -> 147, of 30,000 and 50,000 67.5 -> 63.8, of
+    // 2,000 in tables of 8,192 pages 30.0 -> 17.5, FP8 40.1 -> 28.3. More rows keep the list: by the tables' places, rows that are
+    // alike gain and uneven ones lose (3 of 50,000, BF16 / FP8, 116 / 68.5 us, 101 / 63 without it; 4 of 30,000 to 60,000 144 / 74
+    // and 145 / 87; 64 of 1,024 to 8,192 209.9 / 113.6 and 239.3 / 120.7). An odd number of KV heads, a wavefront a head, and
+    // sliding windows have no such kernels and were not measured.
     const bool places = !fused && (a.dk == 256 || a.heads_per_wave == 2) && (KIND == 0 || a.query_tiles <= 2) && mask != kMaskSliding && grid.y <= 65535;
-    u.places = kPlacesNone;
+    u.places = kPlacesNone, u.cus = compute_units();
     if (places && (int64_t)grid.x * grid.y <= compute_units()) u.places = kPlacesDeep;
     else if (places && a.n_rows <= 2 && a.dk == 128 && a.query_tiles <= 2) u.places = kPlacesPlain;
     if (u.places != kPlacesNone) pgrid = grid;

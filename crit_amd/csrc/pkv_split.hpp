@@ -90,4 +90,54 @@ PKV_SPLIT_FN int window_tiles_8bit(bool scaled_rows, int64_t tiles, bool full, i
     return scaled_rows && tiles == 3 && full && places > 2 * units ? 3 : 2;
 }
 
+// -- windows of two rows without a list of units: the place a workgroup takes ------------------------------------------------
+// Rows of `p0` and `p1` pieces in up to `parts` partitions each (piece i in partition i % parts), `per_row` places (heads, tiles) a
+// partition, by_row(x) = x / per_row, `units` compute units. Workgroups from per_row * (both rows' partitions) on have none. With
+// those between the others (a row's places by the tables' partitions, the rows beside each other) the hardware, which deals
+// workgroups out round by round and counts them too, left some compute units with twice the work of others. For the same
+// reason workgroups `units` apart share a unit, and so:
+//   - Both rows' partitions beside each other while both have them, then the longer one's others, the rows' last ones, which
+//     are parts of pieces, at the end. Which row comes first changes every eight workgroups: they go to the XCDs by number, and
+//     a row would be on half of the XCDs.
+//   - Partitions of more pieces in one row than in the other: a row after the other. In a launch of two rounds at most the
+//     shorter one first: the longest places are then the first round's last, which share with none or with the second's last
+//     (where the first row takes a round by itself, the other's p % parts partitions of a piece more come last, or they would
+//     share with that row's). In a longer launch the longer one first.
+// 32 / 8 heads x 128, BF16 / FP8 / fp8:row / INT8, from a list of units, by the tables' partitions, and so: 2 rows of 30,000 and
+// 50,000 67.5 / 41.0 / 41.0 / 43.5 us, 72 / 44.0 / 47.3 / 46.8, 63.8 / 37.5 / 38.7 / 41.0; of 10,000 and 90,000 87 / 54.2 / 56 / 56,
+// 96 / 55.8 / 61 / 62, 83.5 / 51.3 / 53.8 / 53.6; of 60,000 and 100,000 131 / 72.6 / 74 / 79, 125 / 82.5 / 87 / 89, 108 / 67.5 / 70 /
+// 74.5; in splits of 1,024, 30,000 and 90,000, 84 / 56 / 57.5 / 58, 95 / 60.7 / 65 / 66, 79.5 / 50.5 / 53 / 53.8; alike, 100,000 160 /
+// 98.5 / 101 / 103.7, 146 / 93 / 95.5 / 98.5, 147 / 94.5 / 96 / 99.
+struct RowPlace {
+    int row;
+    uint32_t partition, place;
+};
+template <typename DIV>
+PKV_SPLIT_FN RowPlace row_place(uint32_t workgroup, uint32_t p0, uint32_t p1, uint32_t parts, uint32_t per_row, uint32_t units, DIV by_row) {
+    const uint32_t n0 = p0 < parts ? p0 : parts, n1 = p1 < parts ? p1 : parts;
+    if ((p0 > parts || p1 > parts) && p0 / parts != p1 / parts) {
+        const bool two_rounds = per_row * (n0 + n1) <= 2 * units;
+        const uint32_t head = (p0 < p1) == two_rounds ? 0 : 1, taken = per_row * (head ? n1 : n0);
+        if (workgroup < taken) {
+            const uint32_t b = by_row(workgroup);
+            return RowPlace{(int)head, b, workgroup - b * per_row};
+        }
+        const uint32_t p = head ? p0 : p1, n = head ? n0 : n1, rest = workgroup - taken, q = by_row(rest);
+        const uint32_t b = two_rounds && taken >= units && p > parts ? q + p % parts : q;
+        return RowPlace{(int)(head ^ 1), b < n ? b : b - n, rest - q * per_row};
+    }
+    const uint32_t whole0 = n0 ? n0 - 1 : 0, whole1 = n1 ? n1 - 1 : 0, both = whole0 < whole1 ? whole0 : whole1;
+    if (workgroup < 2 * per_row * both) {
+        const uint32_t b = by_row(workgroup / 2), x = workgroup - 2 * per_row * b;
+        return RowPlace{(int)((x >= per_row ? 1u : 0u) ^ ((b * per_row / 4) & 1u)), b, x >= per_row ? x - per_row : x};
+    }
+    if (workgroup < per_row * (whole0 + whole1)) {
+        const uint32_t rest = workgroup - 2 * per_row * both, q = by_row(rest);
+        return RowPlace{whole1 > whole0 ? 1 : 0, both + q, rest - q * per_row};
+    }
+    const uint32_t rest = workgroup - per_row * (whole0 + whole1);
+    const bool second = !n0 || rest >= per_row;
+    return RowPlace{second ? 1 : 0, second ? whole1 : whole0, rest < per_row ? rest : rest - per_row};
+}
+
 }   // namespace pkv

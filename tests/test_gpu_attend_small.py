@@ -81,3 +81,28 @@ def test_one_or_two_rows_of_more_places_than_compute_units(kind, lengths, column
         at = slice(starts[i], starts[i] + columns)
         want, _ = cache.want(q[at], i, first, columns, parents=torch.tensor([-1, 0, 0, 1], dtype=torch.int32) if tree else None)
         torch.testing.assert_close(out[at].double().cpu(), want, atol=ATOL, rtol=RTOL)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "fp8", "int8"])
+@pytest.mark.parametrize("partitions", [30, 50, 120])
+@pytest.mark.parametrize("lengths,counts", [([6000, 900], [3, 3]), ([900, 6000], [3, 3]), ([6000, 6000], [3, 2]), ([3300, 6000], [3, 3]), ([4000, 70], [0, 3]),
+                                            ([5000, 5000], [3, 0])])
+def test_two_uneven_rows_in_partitions_of_one_piece_and_of_several(kind, partitions, lengths, counts):
+    # pieces of 64: up to 94 of a row; more places than compute units in one partition a piece and in several pieces a partition
+    hq, hkv, d, columns = 32, 8, 128, 3
+    cache = Cache(kind, hkv, d, d, 16, lengths, seed=partitions)
+    cache.tables = torch.cat([cache.tables, cache.tables[:, :1].expand(2, 500)], 1).contiguous()      # (tables wider than their rows)
+    q = rand_q(2 * columns, hq, d, 13)
+    firsts, starts = [x - columns for x in lengths], [0, columns]
+    given = dict(partitions=partitions, piece=64, counts=torch.tensor(counts, dtype=torch.int32, device=dev))
+    results = []
+    for fused in (False, True):
+        out, lse = torch.zeros(2 * columns, hq, d, device=dev), torch.zeros(2 * columns, hq, device=dev)
+        cache.attend(q, [0, 1], starts, firsts, columns, out=out, lse=lse, fused=fused, **given)
+        results += [out, lse]
+    assert torch.equal(results[0], results[2]) and torch.equal(results[1], results[3])
+    for i, (first, count) in enumerate(zip(firsts, counts)):
+        at = slice(starts[i], starts[i] + count)
+        if count:
+            want, _ = cache.want(q[at], i, first, count)
+            torch.testing.assert_close(results[0][at].double().cpu(), want, atol=ATOL, rtol=RTOL)

@@ -21,6 +21,12 @@ extern "C" int xcds_log2(int64_t pairs, int64_t tiles, int64_t units, int64_t he
 extern "C" int64_t workgroups(int64_t pairs, int64_t tiles, int l) { return pkv::dealt_workgroups(pairs, tiles, l); }
 extern "C" int window_tiles(int64_t tiles, int full, int64_t places, int64_t units) { return pkv::window_tiles_16bit(tiles, full != 0, places, units); }
 extern "C" int window_tiles_8bit(int scaled, int64_t tiles, int full, int64_t places, int64_t units) { return pkv::window_tiles_8bit(scaled != 0, tiles, full != 0, places, units); }
+extern "C" void rows(uint32_t workgroups, uint32_t p0, uint32_t p1, uint32_t parts, uint32_t per_row, int* row, uint32_t* partition, uint32_t* place) {
+    for (uint32_t w = 0; w < workgroups; ++w) {
+        const pkv::RowPlace at = pkv::row_place(w, p0, p1, parts, per_row, 256, [=](uint32_t x) { return x / per_row; });
+        row[w] = at.row, partition[w] = at.partition, place[w] = at.place;
+    }
+}
 extern "C" void deal(int64_t pairs, int64_t tiles, int l, int* pair, int* tile) {
     const int64_t n = pkv::dealt_workgroups(pairs, tiles, l);
     for (int64_t w = 0; w < n; ++w) {
@@ -37,6 +43,7 @@ extern "C" void deal(int64_t pairs, int64_t tiles, int l, int* pair, int* tile) 
     lib.window_tiles.argtypes = [ctypes.c_int64, ctypes.c_int, ctypes.c_int64, ctypes.c_int64]
     lib.window_tiles_8bit.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int64, ctypes.c_int64]
     lib.workgroups.restype = ctypes.c_int64
+    lib.rows.argtypes = [ctypes.c_uint32] * 5 + [ctypes.c_void_p] * 3
     lib.deal.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
     return lib
 
@@ -116,3 +123,28 @@ def test_8_bit_windows_of_three_tiles(split):
             for places in (1, 511, 512, 513, 1536, 1 << 20):
                 assert split.window_tiles_8bit(0, tiles, full, places, 256) == 2
                 assert split.window_tiles_8bit(1, tiles, full, places, 256) == (3 if tiles == 3 and full and places > 512 else 2)
+
+
+@pytest.mark.parametrize("per_row", [1, 2, 3, 4, 5, 8, 14, 16, 28])
+@pytest.mark.parametrize("parts", [1, 64, 1000])
+def test_two_rows_without_a_list(split, per_row, parts):
+    for p0, p1 in ((0, 0), (1, 0), (0, 1), (40, 0), (0, 17), (1, 1), (59, 64), (64, 59), (20, 33), (7, 59), (64, 64), (30, 88), (88, 30), (196, 196), (1, 200),
+                   (118, 196), (196, 40), (40, 66), (128, 64), (64, 128), (0, 70), (70, 0)):
+        n0, n1 = min(p0, parts), min(p1, parts)
+        live = per_row * (n0 + n1)
+        row, partition, place = (ctypes.c_int * live)(), (ctypes.c_uint32 * live)(), (ctypes.c_uint32 * live)()
+        split.rows(live, p0, p1, parts, per_row, row, partition, place)
+        units = list(zip(row, partition, place))
+        # every unit of both rows once, on the first workgroups, none without work between them
+        assert sorted(units) == [(r, b, x) for r, n in ((0, n0), (1, n1)) for b in range(n) for x in range(per_row)], (p0, p1)
+        for r in (0, 1):      # a row is on every XCD alike
+            load = [0] * 8
+            for w in range(live):
+                load[w % 8] += row[w] == r
+            assert max(load) - min(load) <= 12, (p0, p1, load)
+        pieces = [(p0, p1)[r] // parts + (b < (p0, p1)[r] % parts) for r, b, _ in units]
+        if max(p0, p1) <= parts:      # the rows' last partitions end the launch
+            assert all(b == (n0, n1)[r] - 1 for r, b, _ in units[live - per_row * (bool(n0) + bool(n1)):])
+        elif live <= 512 and p0 // parts != p1 // parts:      # two of the longest share a compute unit only where no shorter one is alone
+            worst = max((a + b for a, b in zip(pieces, pieces[256:])), default=0)
+            assert worst < 2 * max(pieces) or min(pieces[:256]) == max(pieces), (p0, p1)
