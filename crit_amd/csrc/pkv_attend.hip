@@ -37,17 +37,18 @@ PKV_DEV Merge merge_of(const AttendArgs& a, int c, int head, int r) {
     return Merge{nb, ((prow + c) * a.hq + head) * a.parts};
 }
 
-// One wavefront's fold of a triple's partitions, in order, and its result. MANY: batches of 8 in place of 32.
-template <int DV, bool MANY>
+// One wavefront's fold of a triple's partitions, in order, and its result. MANY: batches of 8 in place of 32. APART: a lane's value
+// dims 64 apart, or side by side.
+template <int DV, bool MANY, bool APART>
 PKV_DEV void merge_by_wavefront(const AttendArgs& a, int c, int head, int r, const Merge& m) {
-    // A lane's value dims lie side by side (128-wide values: two, a load of 8 bytes a partition in place of two of 4, and one
-    // store: 192 triples of up to 22 partitions, 256 wide, 4.7 -> 4.4 us; 448 of 33 5.65 -> 5.35; 1,024 of 40 6.1 -> 6.7), or with
-    // MANY 64 apart (64 rows of 5 columns, 10,240 triples of up to 17, behind their split launch: 276.2 us side by side, 274.5 so). Value rows narrower than a wavefront: the lanes past them idle.
+    // A lane's value dims lie side by side (a load of 8 or 16 bytes a partition and one store), or APART 64 apart: of how many
+    // wavefronts a launch may have either way, see merge_dims_apart(). Value rows narrower than a wavefront: the lanes past
+    // them idle.
     constexpr int EPL = DV < 64 ? 1 : DV / 64;
     typedef float dims_t __attribute__((ext_vector_type(EPL), aligned(4)));      // (of a workspace that is any floats)
     const int lane = DV < 64 ? min((int)threadIdx.x, DV - 1) : (int)threadIdx.x;
     auto load_dims = [&](int64_t state, float (&to)[EPL]) __attribute__((always_inline)) {
-        if constexpr (MANY) {
+        if constexpr (APART) {
 #pragma unroll
             for (int e = 0; e < EPL; ++e) to[e] = a.po[state * DV + 64 * e + lane];
             return;
@@ -154,7 +155,7 @@ PKV_DEV void merge_by_wavefront(const AttendArgs& a, int c, int head, int r, con
 #pragma unroll
     for (int e = 0; e < EPL; ++e) o[e] = L != 0.0f ? A[e] / L : 0.0f;
     bool whole = false;      // 32-bit results, and 16-bit ones on 4 bytes in pairs (results may be a slice of anything)
-    if constexpr (EPL > 1 && !MANY) whole = a.out_dtype == CRIT_PKV_F32 || ((reinterpret_cast<uintptr_t>(a.out) >> 1) + (uint64_t)row) % 2 == 0;
+    if constexpr (EPL > 1 && !APART) whole = a.out_dtype == CRIT_PKV_F32 || ((reinterpret_cast<uintptr_t>(a.out) >> 1) + (uint64_t)row) % 2 == 0;
     if (whole) {
         if (a.out_dtype == CRIT_PKV_F32) {
             dims_t x;
@@ -168,7 +169,7 @@ PKV_DEV void merge_by_wavefront(const AttendArgs& a, int c, int head, int r, con
         }
     } else if (DV >= 64 || (int)threadIdx.x < DV) {
 #pragma unroll
-        for (int e = 0; e < EPL; ++e) store_out(a.out, a.out_dtype, MANY ? row + 64 * e + lane : to + e, o[e]);
+        for (int e = 0; e < EPL; ++e) store_out(a.out, a.out_dtype, APART ? row + 64 * e + lane : to + e, o[e]);
     }
     if (a.lse && threadIdx.x == 0) a.lse[token * a.hq + head] = L != 0.0f ? __builtin_fmaf(M, kLn2, __logf(L)) : -INFINITY;
 }
@@ -176,11 +177,11 @@ PKV_DEV void merge_by_wavefront(const AttendArgs& a, int c, int head, int r, con
 // One wavefront per (column, head, row).
 // MANY: launches of as many wavefronts as the card holds at once of the other form, or more, whose batches of 32 partitions take 160
 // registers: batches of 8, three times the wavefronts (10,240 of up to 17 partitions: 18.7 -> 13.3 us).
-template <int DV, bool MANY>
+template <int DV, bool MANY, bool APART>
 __global__ __launch_bounds__(64) void merge_kernel(AttendArgs a) {
     const int c = blockIdx.x, head = blockIdx.y, r = blockIdx.z;
     const Merge m = merge_of(a, c, head, r);
-    if (m.nb >= 0) merge_by_wavefront<DV, MANY>(a, c, head, r, m);
+    if (m.nb >= 0) merge_by_wavefront<DV, MANY, APART>(a, c, head, r, m);
 }
 
 // The same for few triples in tables with room for many partitions: workgroups of their own. Which way is the row's own: what
@@ -210,7 +211,7 @@ __global__ __launch_bounds__(256) void merge_long_kernel(AttendArgs a) {
     const int nb = m.nb;
     const int64_t at = m.at;
     if (nb <= kFewPartitions) {
-        if (nb >= 0 && wave == 0 && d0 == 0) merge_by_wavefront<DV, false>(a, c, head, r, m);
+        if (nb >= 0 && wave == 0 && d0 == 0) merge_by_wavefront<DV, false, false>(a, c, head, r, m);
         return;
     }
     float M = -INFINITY, L = 0.0f, A = 0.0f;
@@ -559,13 +560,15 @@ static int launch_attend_checked(const crit_pkv_attend_params* p, hipStream_t st
     const dim3 mgrid((unsigned)p->columns, (unsigned)p->heads, (unsigned)p->n_rows);
     // Which merge: by the wavefronts of the launch and the partitions a row may have (the bits are the same). Up to a
     // triple a compute unit in tables with room for more than kFewPartitions, a workgroup each, which looks at its row; 8
-    // wavefronts a compute unit (what the card holds of the form with batches of 32) or more, batches of 8.
+    // wavefronts a compute unit (what the card holds of the form with batches of 32) or more, batches of 8; which lanes take
+    // which value dims: merge_dims_apart().
     const int64_t triples = (int64_t)p->columns * p->heads * p->n_rows, units = compute_units();
-    const bool long_rows = triples <= units && gy > kFewPartitions, many = triples >= 8 * units;
+    const bool long_rows = triples <= units && gy > kFewPartitions, many = triples >= 8 * units, apart = merge_dims_apart(p->value_dim, triples, gy, units);
 #define PKV_MERGE(W)                                                                                                        \
     case W:                                                                                                                 \
-        if (many) hipLaunchKernelGGL((merge_kernel<W, true>), mgrid, dim3(64), 0, stream, a);                               \
-        else hipLaunchKernelGGL((merge_kernel<W, false>), mgrid, dim3(64), 0, stream, a);                                   \
+        if (many) hipLaunchKernelGGL((merge_kernel<W, true, true>), mgrid, dim3(64), 0, stream, a);                         \
+        else if (apart) hipLaunchKernelGGL((merge_kernel<W, false, (W == 128)>), mgrid, dim3(64), 0, stream, a);              \
+        else hipLaunchKernelGGL((merge_kernel<W, false, false>), mgrid, dim3(64), 0, stream, a);                            \
         break;
     if (long_rows && p->value_dim >= 64) {
         const dim3 lgrid((unsigned)(p->columns * (p->value_dim / merge_dims(p->value_dim))), mgrid.y, mgrid.z);

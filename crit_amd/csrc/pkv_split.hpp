@@ -140,4 +140,16 @@ PKV_SPLIT_FN RowPlace row_place(uint32_t workgroup, uint32_t p0, uint32_t p1, ui
     return RowPlace{second ? 1 : 0, second ? whole1 : whole0, rest < per_row ? rest : rest - per_row};
 }
 
+// -- merges: which value dims a wavefront's lanes take -------------------------------------------------------------------
+// Side by side (a load of 8 or 16 bytes a partition in place of two or four of 4) where a wavefront's own time is the launch's;
+// but 128-wide values of more than two wavefronts a compute unit with batches of 32 partitions in flight (rows of more than 8
+// partitions) come 64 apart. Triples of 128-wide values of 4 / 12 / 32 partitions, side by side and 64 apart: 512 3.0 / 4.27 / 4.65 us
+// and 3.1 / 4.4 / 4.8; 640 3.1 / 4.55 / 5.0 and 3.2 / 4.5 / 4.9; 896 3.2 / 4.95 / 5.45 and 3.3 / 4.6 / 5.05; 1,536 3.6 / 6.2 / 6.7 and 3.7 /
+// 5.6 / 6.2; 2,016 3.85 / 6.9 / 8.0 and 3.9 / 5.95 / 7.0. 256-wide values (batches of 16) gain side by side at every size (1,512 of
+// 4 / 12 / 32 4.1 / 9.4 / 19.0 and 4.3 / 9.9 / 19.7). 8 wavefronts a compute unit and more (batches of 8): 64 apart (10,240 triples of
+// up to 17, behind their split launch: 276.2 us side by side, 274.5 so).
+PKV_SPLIT_FN bool merge_dims_apart(int value_dim, int64_t triples, int64_t partitions, int64_t units) {
+    return triples >= 8 * units || (value_dim == 128 && 2 * triples >= 5 * units && partitions > 8);
+}
+
 }   // namespace pkv

@@ -21,6 +21,7 @@ extern "C" int xcds_log2(int64_t pairs, int64_t tiles, int64_t units, int64_t he
 extern "C" int64_t workgroups(int64_t pairs, int64_t tiles, int l) { return pkv::dealt_workgroups(pairs, tiles, l); }
 extern "C" int window_tiles(int64_t tiles, int full, int64_t places, int64_t units) { return pkv::window_tiles_16bit(tiles, full != 0, places, units); }
 extern "C" int window_tiles_8bit(int scaled, int64_t tiles, int full, int64_t places, int64_t units) { return pkv::window_tiles_8bit(scaled != 0, tiles, full != 0, places, units); }
+extern "C" int apart(int value_dim, int64_t triples, int64_t partitions, int64_t units) { return pkv::merge_dims_apart(value_dim, triples, partitions, units); }
 extern "C" void rows(uint32_t workgroups, uint32_t p0, uint32_t p1, uint32_t parts, uint32_t per_row, int* row, uint32_t* partition, uint32_t* place) {
     for (uint32_t w = 0; w < workgroups; ++w) {
         const pkv::RowPlace at = pkv::row_place(w, p0, p1, parts, per_row, 256, [=](uint32_t x) { return x / per_row; });
@@ -43,6 +44,7 @@ extern "C" void deal(int64_t pairs, int64_t tiles, int l, int* pair, int* tile) 
     lib.window_tiles.argtypes = [ctypes.c_int64, ctypes.c_int, ctypes.c_int64, ctypes.c_int64]
     lib.window_tiles_8bit.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int64, ctypes.c_int64]
     lib.workgroups.restype = ctypes.c_int64
+    lib.apart.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64]
     lib.rows.argtypes = [ctypes.c_uint32] * 5 + [ctypes.c_void_p] * 3
     lib.deal.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
     return lib
@@ -148,3 +150,11 @@ def test_two_rows_without_a_list(split, per_row, parts):
         elif live <= 512 and p0 // parts != p1 // parts:      # two of the longest share a compute unit only where no shorter one is alone
             worst = max((a + b for a, b in zip(pieces, pieces[256:])), default=0)
             assert worst < 2 * max(pieces) or min(pieces[:256]) == max(pieces), (p0, p1)
+
+
+def test_merges_of_many_long_rows_take_their_dims_apart(split):
+    # 128-wide values: 20 to 63 rows of 32 heads and more than 8 partitions; small launches, few partitions and 256-wide values do not
+    assert all(split.apart(128, rows * 32, parts, 256) for rows in (20, 32, 63, 64, 128) for parts in (9, 17, 64))
+    assert not any(split.apart(128, rows * 32, parts, 256) for rows in (1, 16, 19) for parts in (4, 17, 64))
+    assert not any(split.apart(128, rows * 32, parts, 256) for rows in (20, 63) for parts in (1, 4, 8))
+    assert not any(split.apart(256, triples, 64, 256) for triples in (24, 640, 2047))
