@@ -608,8 +608,9 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT, PLACES>::kGroups)) vo
     // What a unit needs beside its rows is requested with its page table entries, a unit ahead, and is there when its rows are
     // sent for. A wait on any of it behind the unit's rows would wait for those too, and behind the fold for the partials'
     // stores as well, which the compiler cannot count; a workgroup alone on its compute unit has nothing to do meanwhile
-    // (64 rows ~U[1024, 8192], 32 / 8 heads x 128 BF16, 5 columns: 277.2 -> 274.4 us). A tree's links, walked a load at a time
-    // for every tile, were most of what a lone row gained (one of 50,000, 56 / 8 heads, INT8, a tree of 8: 98.9 -> 96.5).
+    // (64 rows ~U[1024, 8192], 32 / 8 heads x 128 BF16, 5 columns: 277.2 and 274.4 us, which is as much as two runs differ). A
+    // tree's links, walked a load at a time for every tile, were most of what a lone row gained (one of 50,000, 56 / 8 heads,
+    // INT8, a tree of 8: 98.9 -> 96.5).
     auto request = [&](const Unit& un) __attribute__((always_inline)) {
         if constexpr (KIND == 1) {
 #pragma unroll

@@ -371,7 +371,7 @@ __global__ __launch_bounds__(256, NT == 1 ? 3 : 2) void latent_kernel(LatentArgs
 // matrix instructions (scores 1,800, softmax and the probabilities' way through LDS 750, values 1,900, barriers 300),
 // so 16-bit rows now send a step's value products out one step later, with the next step's softmax between them. A
 // unit's start (whose row it is 4,700, the table 1,200, the queries with the first tile 10,700) and end (the last values 1,700,
-// 256 KB of partials 5,600) are another 28,000. With one workgroup a compute unit nothing hides either, so launches of a few rows
+// 256 KB of partials 5,600) are another 24,000. With one workgroup a compute unit nothing hides either, so launches of a few rows
 // are slower than with the small tiles (1 row: 67 us against 40): tile_rows = 16 asks for those. E4M3 rows (see the
 // kernel's constants): 158 us.
 constexpr float kLazyHeads = 8.0f;
@@ -617,7 +617,9 @@ __global__ __launch_bounds__(256, 1) void latent_heads_kernel(LatentArgs a) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(bq[ks]));
     if constexpr (FP8) lds_barrier();      // (another wavefront's queries lay where the first tile's values go)
-    // (the first tile has landed with the queries; the next two tiles go out behind them)
+    // (The first tile has landed with the queries; behind them go the next tile of 16-bit rows, the next two of E4M3. In the ring's
+    // tiles 2 and 3 lie 16-bit caches' queries, which other wavefronts may still read: nothing is sent there before the first
+    // step's lds_barrier().)
     int base1 = issue(1, 1), base2 = FP8 ? issue(2, 2) : 0;
     // E4M3: the wavefront's rows of raw tile `from`, as 16-bit values in tile `to` (a lane: 16 codes a turn).
     // (In five parts, without a branch, so that a part can go between the value products: the last part's upper lanes
