@@ -59,8 +59,8 @@ struct AttendArgs {
     int derive_rot, derive_weighted;
     int narrow;   // 64-wide heads read in pairs as 128-wide ones: hkv, g, dk and dv above are the pairs' (half, twice, 128, 128)
     int iqk;      // INT8 pages: the queries as INT8 codes at each row's own scale (prefill's int8_qk read as windows)
-    int places;   // a workgroup a place of the tables, without a list of units: kPlacesNone, kPlacesDeep, kPlacesPlain
-    int cus;      // the card's compute units
+    int places;   // a workgroup a place of the tables, without a list of units: kPlacesNone, kPlacesDeep, kPlacesPlain, kPlacesTwo
+    int cus;      // kPlacesTwo: the card's compute units
 };
 
 // A workgroup barrier that orders the shared arrays only: a wavefront waits for its own LDS traffic, then for the

@@ -147,6 +147,12 @@ static int launch_mfma_masked(const AttendArgs& u, bool fused, dim3 grid, hipStr
             else PKV_MFMA(2, false, MASK, 1, 2, false, kPlacesPlain);
             return hip_code(hipGetLastError());
         }
+        if (u.places == kPlacesTwo) {
+            if (u.narrow) PKV_MFMA(2, false, MASK, 1, 1, true, kPlacesTwo);
+            else if (u.query_tiles == 1) PKV_MFMA(2, false, MASK, 1, 1, false, kPlacesTwo);
+            else PKV_MFMA(2, false, MASK, 1, 2, false, kPlacesTwo);
+            return hip_code(hipGetLastError());
+        }
     }
     if (u.narrow) {
         if (u.query_tiles != 1) return CRIT_PKV_E_GEOMETRY;
@@ -215,7 +221,7 @@ static int launch_mfma(const AttendArgs& a, bool fused, dim3 grid, hipStream_t s
     const bool places = !fused && (a.dk == 256 || a.heads_per_wave == 2) && (KIND == 0 || a.query_tiles <= 2) && mask != kMaskSliding && grid.y <= 65535;
     u.places = kPlacesNone, u.cus = compute_units();
     if (places && (int64_t)grid.x * grid.y <= compute_units()) u.places = kPlacesDeep;
-    else if (places && a.n_rows <= 2 && a.dk == 128 && a.query_tiles <= 2) u.places = kPlacesPlain;
+    else if (places && a.n_rows <= 2 && a.dk == 128 && a.query_tiles <= 2) u.places = a.n_rows == 1 ? kPlacesPlain : kPlacesTwo;
     if (u.places != kPlacesNone) pgrid = grid;
     switch (mask) {
         case kMaskNone: return launch_mfma_masked<KIND, F16, kMaskNone>(u, fused, pgrid, stream);

@@ -134,8 +134,9 @@ PKV_DEV u32x4 key_operand(const u32x4* k, int c) {
 }
 
 // Launches without a list of units, a workgroup a place of the tables (the launcher's rule): with more of its steps in flight, or as
-// the list's.
-constexpr int kPlacesNone = 0, kPlacesDeep = 1, kPlacesPlain = 2;
+// the list's; of two rows, the place by row_place() (a kernel of its own: with both in one, a lone row's window of two tiles of INT8
+// pages took 97.6 us in place of 96.8).
+constexpr int kPlacesNone = 0, kPlacesDeep = 1, kPlacesPlain = 2, kPlacesTwo = 3;
 constexpr int kMaskNone = 0, kMaskTree = 1, kMaskSliding = 2;
 constexpr int kTileRows = 16;      // query rows (columns of S^T) a tile holds
 constexpr int kLdsRows = 512;      // batch rows whose descriptors a workgroup keeps in LDS (the others are read from memory)
@@ -358,24 +359,19 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT, PLACES>::kGroups)) vo
         int bx, b, r;
         bool last = false;      // dense list: the row's last partition
         int d[5];
-        if constexpr (PLACES == kPlacesPlain) {
-            if (a.n_rows == 1) {
-                r = 0, b = (int)blockIdx.y, bx = (int)blockIdx.x;
-                row_from_memory(0, d);
-            } else {      // (both rows' numbers in one round trip to memory)
-                int d1[5];
-                row_from_memory(0, d), row_from_memory(1, d1);
-                auto pieces_of_row = [&](const int (&n)[5]) __attribute__((always_inline)) -> uint32_t {
-                    return (uint32_t)__builtin_amdgcn_readfirstlane(n[0] > 0 ? pieces_of(min(n[1] + n[0], a.max_keys)) : 0);
-                };
-                const uint32_t p0 = pieces_of_row(d), p1 = pieces_of_row(d1), mine = blockIdx.y * grid + blockIdx.x;
-                if (mine >= per_row * (min(p0, (uint32_t)a.parts) + min(p1, (uint32_t)a.parts))) return un;
-                const RowPlace at = row_place(mine, p0, p1, (uint32_t)a.parts, per_row, (uint32_t)a.cus,
-                                              [&](uint32_t x) __attribute__((always_inline)) -> uint32_t { return div32(a.row_div, x); });
-                r = at.row, b = (int)at.partition, bx = (int)at.place;
+        if constexpr (PLACES == kPlacesTwo) {      // (both rows' numbers in one round trip to memory)
+            int d1[5];
+            row_from_memory(0, d), row_from_memory(1, d1);
+            auto pieces_of_row = [&](const int (&n)[5]) __attribute__((always_inline)) -> uint32_t {
+                return (uint32_t)__builtin_amdgcn_readfirstlane(n[0] > 0 ? pieces_of(min(n[1] + n[0], a.max_keys)) : 0);
+            };
+            const uint32_t p0 = pieces_of_row(d), p1 = pieces_of_row(d1), mine = blockIdx.y * grid + blockIdx.x;
+            if (mine >= per_row * (min(p0, (uint32_t)a.parts) + min(p1, (uint32_t)a.parts))) return un;
+            const RowPlace at = row_place(mine, p0, p1, (uint32_t)a.parts, per_row, (uint32_t)a.cus,
+                                          [&](uint32_t x) __attribute__((always_inline)) -> uint32_t { return div32(a.row_div, x); });
+            r = at.row, b = (int)at.partition, bx = (int)at.place;
 #pragma unroll
-                for (int i = 0; i < 5; ++i) d[i] = r ? d1[i] : d[i];
-            }
+            for (int i = 0; i < 5; ++i) d[i] = r ? d1[i] : d[i];
         } else if constexpr (ALONE) {
             r = (int)div32(a.row_div, blockIdx.x), b = (int)blockIdx.y;
             bx = (int)blockIdx.x - r * (int)per_row;
@@ -400,7 +396,7 @@ __global__ __launch_bounds__(256, (MfmaShape<KIND, DH, QT, PLACES>::kGroups)) vo
         }
         const int tiles_before = (int)div32(a.tiles_div, (uint32_t)bx), tile = bx - tiles_before * a.tiles;
         un.kvh0 = tiles_before * HW;      // the first of the wavefronts' KV heads
-        if constexpr (PLACES != kPlacesPlain) {
+        if constexpr (PLACES != kPlacesTwo) {
             if (!ALONE && r < kLdsRows) {
 #pragma unroll
                 for (int i = 0; i < 5; ++i) d[i] = s_rows[r][i];
